@@ -181,6 +181,10 @@ const std::shared_ptr<DeviceCache> &Context::current_cache() const
 }
 
 // ---------------------------------------------------------------- context
+// v in [0, q] as the double nearest zero of its residue class: products with it
+// are half as large
+static double centred(uint64_t v, uint64_t q) { return v > q / 2 ? -(double)(q - v) : (double)v; }
+
 Context::Context(int logn_, const std::vector<int> &bit_sizes, uint32_t hw, size_t sparse, size_t special)
     : logn(logn_), n(size_t(1) << logn_), alpha(special), hamming_weight(hw), sparse_slots(sparse)
 {
@@ -201,7 +205,7 @@ Context::Context(int logn_, const std::vector<int> &bit_sizes, uint32_t hw, size
 
     const size_t P = moduli.size();
     std::vector<ulonglong2> fwd(P * n), inv(P * n), ninv(P);
-    std::vector<double> fwd_d(P * n), inv_d(P * n), ninv_d(P);  // exact for primes below 2^53
+    std::vector<double> fwd_d(P * n), inv_d(P * n), ninv_d(P);  // centred; exact for primes below 2^53
     std::vector<double2> qd(P);
     fwd_host.resize(P);
     inv_host.resize(P);
@@ -211,12 +215,12 @@ Context::Context(int logn_, const std::vector<int> &bit_sizes, uint32_t hw, size
         for (size_t k = 0; k < n; k++) {
             fwd[i * n + k] = make_ulonglong2(fwd_host[i][k], shoup_quotient(fwd_host[i][k], q));
             inv[i * n + k] = make_ulonglong2(inv_host[i][k], shoup_quotient(inv_host[i][k], q));
-            fwd_d[i * n + k] = (double)fwd_host[i][k];
-            inv_d[i * n + k] = (double)inv_host[i][k];
+            fwd_d[i * n + k] = centred(fwd_host[i][k], q);
+            inv_d[i * n + k] = centred(inv_host[i][k], q);
         }
         uint64_t ni = host_inv_mod(n % q, q);
         ninv[i] = make_ulonglong2(ni, shoup_quotient(ni, q));
-        ninv_d[i] = (double)ni;
+        ninv_d[i] = centred(ni, q);
         qd[i] = make_double2((double)q, 1.0 / (double)q);
     }
     // rescale constants: row `l` (limbs before the rescale), column i < l-1
@@ -288,14 +292,14 @@ Context::Context(int logn_, const std::vector<int> &bit_sizes, uint32_t hw, size
 // Double-precision copy of a ModDown conversion table over A input primes
 // (rows k < A: factors f_ki, row A: the base product mod q_i): rows k < A as
 // doubles, row A as q_i - (row A).  Used for output primes below 2^51 when every
-// input prime is below 2^51.
+// input prime is below 2^51.  Every entry is centred.
 static std::vector<double> moddown_conv_doubles(const uint64_t *conv, size_t A, size_t L,
                                                 const std::vector<uint64_t> &moduli)
 {
     std::vector<double> d((A + 1) * L, 0.0);
     for (size_t i = 0; i < L; i++) {
-        for (size_t k = 0; k < A; k++) d[k * L + i] = (double)conv[k * L + i];
-        d[A * L + i] = (double)(moduli[i] - conv[A * L + i] % moduli[i]);
+        for (size_t k = 0; k < A; k++) d[k * L + i] = centred(conv[k * L + i], moduli[i]);
+        d[A * L + i] = centred(moduli[i] - conv[A * L + i] % moduli[i], moduli[i]);
     }
     return d;
 }
@@ -408,7 +412,8 @@ void Context::build_hybrid_tables()
     NX_HIP(hipMemcpy(d_modup_conv, uc.data(), uc.size() * sizeof(uint64_t), hipMemcpyHostToDevice));
     {
         // the same factors as doubles (exact: every factor is below its prime, < 2^53 where used)
-        std::vector<double> ucd(uc.begin(), uc.end());
+        std::vector<double> ucd(uc.size());
+        for (size_t i = 0; i < uc.size(); i++) ucd[i] = centred(uc[i], moduli[i % K]);
         NX_HIP(hipMalloc(&d_modup_conv_d, ucd.size() * sizeof(double)));
         NX_HIP(hipMemcpy(d_modup_conv_d, ucd.data(), ucd.size() * sizeof(double), hipMemcpyHostToDevice));
     }

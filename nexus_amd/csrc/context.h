@@ -343,6 +343,19 @@ void ks_out_primes(const Context &c, size_t l, uint8_t *outp);
 DevBuf ks_modup(Context &c, const uint64_t *targets, size_t B, size_t l);
 // ModUp of B <= kNttSrcMax targets given by pointer ([l][n] each)
 DevBuf ks_modup_list(Context &c, const uint64_t *const *targets, size_t B, size_t l);
+// Whether key switches run without a stored ModUp (kernels_ks.hip).
+bool ks_rows_fused(const Context &c);
+// Inner products of the digits of B targets ([B][l][n] NTT form, or B <=
+// kNttSrcMax pointers) with keys, the digits in chunks (ks_rows_fused only):
+// acc[B][2][l+alpha][n] with the one key keys[0]; or with perms, target b
+// rotated by perms[b] under keys[b] and summed into acc[2][l+alpha][n] (added
+// to it with accumulate).  aseeds as KSwitchKeys::seeds_of, one per key.
+void ks_inner(Context &c, uint64_t *acc, const uint64_t *targets, const uint64_t *const *target_list, size_t B,
+              size_t l, const uint64_t *const *keys, const uint64_t *const *aseeds, const uint32_t *const *perms,
+              bool accumulate);
+// acc[B][2][l+alpha][n]: the same with one key, on any ring
+void ks_inner_one_key(Context &c, uint64_t *acc, const uint64_t *targets, size_t B, size_t l, const DevBuf &key,
+                      const uint64_t *aseed);
 // ModDown up to the final combination: INTT of the special limbs of acc
 // [B][2][l+alpha][n], conversion, NTT; returns tmp [B][2][l][n] for
 // out = (acc - tmp) P^-1.

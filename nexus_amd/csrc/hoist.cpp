@@ -228,11 +228,13 @@ void op_rotate_sum_many(const std::vector<std::vector<const Ciphertext *>> &grou
         }
     }
     std::vector<char> started(G, 0);
+    const bool fused = ks_rows_fused(c);
     for (size_t base = 0; base < sw.size(); base += kMaxHoist) {
         const size_t cnt = std::min<size_t>(kMaxHoist, sw.size() - base);
         std::vector<const uint64_t *> c1s(cnt);
         for (size_t r = 0; r < cnt; r++) c1s[r] = sw[base + r].c1;
-        DevBuf T = ks_modup_list(c, c1s.data(), cnt, l);
+        DevBuf T;
+        if (!fused) T = ks_modup_list(c, c1s.data(), cnt, l);
         for (size_t r0 = 0; r0 < cnt;) {
             const size_t g = sw[base + r0].g;
             size_t r1 = r0;
@@ -244,10 +246,14 @@ void op_rotate_sum_many(const std::vector<std::vector<const Ciphertext *>> &grou
                 seeds.push_back(sw[base + r].seed);
                 rperms.push_back(sw[base + r].perm);
             }
-            ks_inner_product_rot_sum(c.tables, acc.get() + g * 2 * nout * n, T.get() + r0 * nout * digits * n,
-                                     keys.data(), rperms.data(), (uint32_t)(r1 - r0), (uint32_t)digits,
-                                     (uint32_t)c.key_limbs(), outp, (uint32_t)nout, started[g] != 0, c.stream,
-                                     nout * digits * n, seeds.data());
+            if (fused)
+                ks_inner(c, acc.get() + g * 2 * nout * n, nullptr, c1s.data() + r0, r1 - r0, l, keys.data(),
+                         seeds.data(), rperms.data(), started[g] != 0);
+            else
+                ks_inner_product_rot_sum(c.tables, acc.get() + g * 2 * nout * n, T.get() + r0 * nout * digits * n,
+                                         keys.data(), rperms.data(), (uint32_t)(r1 - r0), (uint32_t)digits,
+                                         (uint32_t)c.key_limbs(), outp, (uint32_t)nout, started[g] != 0, c.stream,
+                                         nout * digits * n, seeds.data());
             started[g] = 1;
             r0 = r1;
         }
@@ -377,6 +383,11 @@ void op_rotate_sum(const std::vector<const Ciphertext *> &in, const std::vector<
         DevBuf acc(&c, 2 * nout * n);
         for (size_t base = 0; base < keys.size(); base += kMaxHoist) {
             const size_t cnt = std::min<size_t>(kMaxHoist, keys.size() - base);
+            if (ks_rows_fused(c)) {
+                ks_inner(c, acc.get(), nullptr, c1s.data() + base, cnt, l, keys.data() + base, seeds.data() + base,
+                         rperms.data() + base, base > 0);
+                continue;
+            }
             DevBuf T = ks_modup_list(c, c1s.data() + base, cnt, l);
             ks_inner_product_rot_sum(c.tables, acc.get(), T.get(), keys.data() + base, rperms.data() + base,
                                      (uint32_t)cnt, (uint32_t)digits, (uint32_t)c.key_limbs(), outp, (uint32_t)nout,

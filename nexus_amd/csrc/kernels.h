@@ -20,8 +20,8 @@ struct DeviceTables {
     const ulonglong2 *fwd;   // [prime][n] {psi power, Shoup quotient}, SEAL bit-reversed order
     const ulonglong2 *inv;   // [prime][n] {inverse psi power, Shoup quotient}, SEAL scrambled order
     const ulonglong2 *ninv;  // [prime] {n^-1 mod q, Shoup quotient}
-    const double *fwd_d;     // [prime][n] the fwd powers as doubles (exact below 2^53)
-    const double *inv_d;     // [prime][n] the inv powers as doubles
+    const double *fwd_d;     // [prime][n] the fwd powers as doubles, centred (exact below 2^53)
+    const double *inv_d;     // [prime][n] the inv powers as doubles, centred
     const double *ninv_d;    // [prime] n^-1 mod q as doubles
     const double *modup_conv_d = nullptr;  // hybrid ModUp factors as doubles (Context::d_modup_conv)
     const ModConst *mod;     // [prime]
@@ -92,6 +92,7 @@ struct NttBatch {
     uint32_t rows_only = 0;
 };
 constexpr int kNttSrcMax = 32;
+constexpr int kMaxHoist = 32;  // rotations of one hoisted inner product
 
 // Forward negacyclic NTT: natural order in, SEAL bit-reversed order out, [0, q).
 void ntt_forward(const DeviceTables &t, const NttBatch &b, hipStream_t s);
@@ -239,15 +240,36 @@ void ks_modup_copy_own(const DeviceTables &t, uint64_t *T, const uint64_t *targe
 // (ks_modup_copy_own).  Needs ks_modup_col_ok: every prime below 2^51,
 // 2 <= alpha <= 8, 2^14 <= n <= 2^17, the double-precision factor table.
 bool ks_modup_col_ok(const DeviceTables &t, uint32_t alpha);
-// per power-of-two bucket of B: -1 = unfused; otherwise fused, with k =
-// mode & 255 outputs per workgroup (0: the default rule), 4-column tiles
-// instead of 8 when mode & 256, 512 threads per workgroup (8-column tiles,
-// half the registers per thread) when mode & 512
+// per power-of-two bucket of B: -1 = unfused; otherwise fused, with `mode`
+// outputs per workgroup (0: the default rule)
 void ks_modup_col_set(uint32_t B, int mode);
 int ks_modup_col_get(uint32_t B);
 void ks_modup_convert_col(const DeviceTables &t, uint64_t *T, const uint64_t *coef, const ulonglong2 *w,
                           uint32_t B, uint32_t l, uint32_t alpha, uint32_t key_limbs, const uint8_t *out_primes_host,
-                          uint32_t nout, hipStream_t s);
+                          uint32_t nout, hipStream_t s, bool raw = false);
+// The digits of a key switch from the column pass to the inner product
+// (kernels_ks.hip): T[b][I - i0][j] for the output primes i0 .. i0 + icount - 1
+// outside digit j holds column-transformed values as ks_row_inner reads them
+// (doubles below 2^51, lazily reduced words above), written by ks_lift_col
+// (one special prime) or ks_modup_convert_col with raw set (i0 = 0, icount =
+// nout).  ks_row_inner runs the row pass and multiplies by the keys.
+bool ks_row_inner_ok(const DeviceTables &t, uint32_t alpha);
+void ks_lift_col(const DeviceTables &t, uint64_t *T, const uint64_t *coef, uint32_t B, uint32_t l, uint32_t i0,
+                 uint32_t icount, const uint8_t *out_primes_host, uint32_t nout, hipStream_t s);
+struct KsRowInner {
+    uint64_t *acc = nullptr;       // [count][2][nout][n], or [2][nout][n] for a sum of rotations
+    const uint64_t *T = nullptr;   // [count][icount][digits][n], t_stride words per input
+    uint64_t t_stride = 0;
+    const uint64_t *own = nullptr;             // the inputs in NTT form, [count][l][n] ...
+    const uint64_t *const *own_list = nullptr; // ... or a pointer each (count <= kMaxHoist)
+    const uint64_t *const *keys = nullptr;     // one key, or one per rotation
+    const uint64_t *const *aseeds = nullptr;   // per key: its uniform half's digit seeds, or null
+    const uint32_t *const *perms = nullptr;    // set: acc (+)= the sum over the inputs of their rotations
+    uint32_t count = 0, l = 0, alpha = 0, digits = 0, nout = 0, i0 = 0, icount = 0, key_limbs = 0;
+    bool accumulate = false;       // sums of rotations: add to acc
+    const uint8_t *out_primes = nullptr;
+};
+void ks_row_inner(const DeviceTables &t, const KsRowInner &p, hipStream_t s);
 // ModDown conversion fused into the forward column pass: the A coefficient-form
 // limbs lo .. lo + A - 1 of each poly of acc (primes in_primes_host, Shoup
 // constants w, double factor table convd with rows k <= A of stride L as in
@@ -315,7 +337,6 @@ void block_mix(const DeviceTables &t, const MixPtrs &p, const uint64_t *table, c
 // (T[I][j][perms[r][c]]) and uses key keys[r].  _rot writes one result per
 // rotation, acc[r][2][nout][n]; _rot_sum writes (or adds to acc) their sum,
 // acc[2][nout][n].
-constexpr int kMaxHoist = 32;
 void ks_inner_product_rot(const DeviceTables &t, uint64_t *acc, const uint64_t *T, const uint64_t *const *keys,
                           const uint32_t *const *perms, uint32_t count, uint32_t l, uint32_t key_limbs,
                           const uint8_t *out_primes_host, uint32_t nout, hipStream_t s,

@@ -33,13 +33,12 @@
 #include <stdexcept>
 
 #include "kernels.h"
+#include "ntt_steps.h"
 #include "prof.h"
 
 namespace nx {
 
 namespace {
-
-enum Role { kWhole = 0, kCol = 1, kRow = 2 };
 
 struct NttKArgs {
     uint64_t *data;
@@ -55,6 +54,7 @@ struct NttKArgs {
     uint32_t poly_period;
     const ulonglong2 *tw;
     const ModConst *mod;
+    const double2 *qd;
     const ulonglong2 *ninv;
     const double *twd;    // the same twiddles as doubles
     const double *ninvd;  // n^-1 mod q as doubles
@@ -92,150 +92,7 @@ __device__ __forceinline__ void epi_store(const NttEpilogue &e, uint32_t p, uint
     e.outs[ct][((uint64_t)k * l + i) * n + gidx] = r;
 }
 
-constexpr int kThreads = 256;
 constexpr int kTuneLogNMin = 14, kTuneLogN = 4, kTuneBuckets = 9;
-
-// CW: sub-transforms per workgroup -- columns of the column pass (8 by
-// default: a 16 KB tile keeps twice the workgroups of a 16-wide one resident,
-// and once a batch outgrows the last-level cache the strided column reads of
-// 8-wide tiles stream faster), and an upper bound on the rows of the row pass.
-template <int LOGS, int ROLE, int CW>
-struct Geometry {
-    static constexpr int S = 1 << LOGS;
-    static constexpr int ROWS = S >= 2048 ? 1 : 2048 / S;
-    static constexpr int C = ROLE == kCol ? CW : (ROLE == kRow ? (ROWS < CW ? ROWS : CW) : 1);
-    static constexpr int TILE = S * C;
-};
-
-// LDS address of local position `pos` of sub-transform `cc`.
-template <int ROLE, int S, int C>
-__device__ __forceinline__ int lds_addr(int cc, int pos)
-{
-    return ROLE == kCol ? pos * C + cc : cc * S + pos;
-}
-
-// Forward radix-2^K step over local stages s .. s+K-1.
-template <int LOGS, int ROLE, int K, int CW>
-__device__ __forceinline__ void fwd_step(uint64_t *lds, int s, const ulonglong2 *tw, uint64_t q, uint32_t m0,
-                                         uint32_t row0)
-{
-    using G = Geometry<LOGS, ROLE, CW>;
-    constexpr int R = 1 << K;
-    constexpr int GROUPS_PER = G::S / R;
-    constexpr int GROUPS = G::TILE / R;
-    const uint64_t two_q = 2 * q;
-    const int B = G::S >> s;
-    const int D = B >> K;
-    for (int g = threadIdx.x; g < GROUPS; g += kThreads) {
-        int cc, gg;
-        if (ROLE == kCol) {
-            cc = g % G::C;
-            gg = g / G::C;
-        } else {
-            cc = g / GROUPS_PER;
-            gg = g % GROUPS_PER;
-        }
-        const int blockid = gg / D;
-        const int o = gg - blockid * D;
-        const uint32_t mrow = (ROLE == kRow) ? (m0 + row0 + cc) : m0;
-        uint64_t v[R];
-        int addr[R];
-#pragma unroll
-        for (int t = 0; t < R; t++) {
-            addr[t] = lds_addr<ROLE, G::S, G::C>(cc, blockid * B + o + t * D);
-            v[t] = lds[addr[t]];
-        }
-#pragma unroll
-        for (int d = 0; d < K; d++) {
-            const int h = 1 << (K - 1 - d);
-#pragma unroll
-            for (int j = 0; j < (1 << d); j++) {
-                const uint32_t b = (uint32_t)blockid * (1u << d) + j;
-                const ulonglong2 w = tw[((uint32_t)1 << (s + d)) * mrow + b];
-#pragma unroll
-                for (int u = 0; u < h; u++) {
-                    const int t = j * 2 * h + u;
-                    uint64_t x = v[t];
-                    x = x >= two_q ? x - two_q : x;
-                    const uint64_t y = shoup_lazy(v[t + h], w.x, w.y, q);
-                    v[t] = x + y;
-                    v[t + h] = x - y + two_q;
-                }
-            }
-        }
-#pragma unroll
-        for (int t = 0; t < R; t++) lds[addr[t]] = v[t];
-    }
-}
-
-// Inverse radix-2^K step over local stages s .. s+K-1 (gaps 2^s .. 2^(s+K-1)).
-template <int LOGS, int ROLE, int K, int CW>
-__device__ __forceinline__ void inv_step(uint64_t *lds, int s, const ulonglong2 *tw, uint64_t q, uint32_t n,
-                                         uint32_t mx, uint32_t row0)
-{
-    using G = Geometry<LOGS, ROLE, CW>;
-    constexpr int R = 1 << K;
-    constexpr int GROUPS_PER = G::S / R;
-    constexpr int GROUPS = G::TILE / R;
-    const uint64_t two_q = 2 * q;
-    const int so = 1 << s;
-    for (int g = threadIdx.x; g < GROUPS; g += kThreads) {
-        int cc, gg;
-        if (ROLE == kCol) {
-            cc = g % G::C;
-            gg = g / G::C;
-        } else {
-            cc = g / GROUPS_PER;
-            gg = g % GROUPS_PER;
-        }
-        const int o = gg & (so - 1);
-        const int blockid = gg >> s;
-        const int base = blockid * (so << K) + o;
-        const uint32_t r = row0 + cc;
-        uint64_t v[R];
-        int addr[R];
-#pragma unroll
-        for (int t = 0; t < R; t++) {
-            addr[t] = lds_addr<ROLE, G::S, G::C>(cc, base + t * so);
-            v[t] = lds[addr[t]];
-        }
-#pragma unroll
-        for (int d = 0; d < K; d++) {
-            const int sd = s + d;
-            const uint32_t first = n - (mx >> sd) + 1 + (ROLE == kRow ? r * ((uint32_t)G::S >> (sd + 1)) : 0u);
-#pragma unroll
-            for (int j = 0; j < (R >> (d + 1)); j++) {
-                const uint32_t b = (uint32_t)blockid * (uint32_t)(R >> (d + 1)) + j;
-                const ulonglong2 w = tw[first + b];
-#pragma unroll
-                for (int u = 0; u < (1 << d); u++) {
-                    const int t = j * (2 << d) + u;
-                    const uint64_t x = v[t], y = v[t + (1 << d)];
-                    uint64_t sum = x + y;
-                    v[t] = sum >= two_q ? sum - two_q : sum;
-                    v[t + (1 << d)] = shoup_lazy(x - y + two_q, w.x, w.y, q);
-                }
-            }
-        }
-#pragma unroll
-        for (int t = 0; t < R; t++) lds[addr[t]] = v[t];
-    }
-}
-
-constexpr uint64_t kFpPrimeBound = 1ull << 51;
-
-__device__ __forceinline__ double mulmod_f(double a, double w, double q, double qinv)
-{
-    const double h = a * w;
-    const double e = __builtin_fma(a, w, -h);
-    const double Q = __builtin_rint(h * qinv);
-    return __builtin_fma(-Q, q, h) + e;
-}
-
-__device__ __forceinline__ double reduce_f(double z, double q, double qinv)
-{
-    return __builtin_fma(-__builtin_rint(z * qinv), q, z);
-}
 
 // epi_store in double precision (every prime of the batch below 2^51): the
 // transform value t in [0, q) as a double, the Shoup constants' values (below
@@ -248,229 +105,26 @@ __device__ __forceinline__ void epi_store_f(const NttEpilogue &e, uint32_t p, ui
     const uint64_t off = (uint64_t)i * n + gidx;
     const uint32_t ct = p / e.polys_per, k = p - ct * e.polys_per;
     const uint64_t xv = e.xs[0] ? e.xs[ct][((uint64_t)k * e.x_limbs + i) * n + gidx] : e.x[p * e.x_stride + off];
-    double r = mulmod_f((double)xv - t, (double)e.inv[i].x, q, qinv);
+    double r = mulmod_f(fp_from(xv) - t, fp_from(e.inv[i].x), q, qinv);
     uint64_t *o;
     if (e.out) {
         o = e.out + p * e.out_stride + off;
         if (e.accumulate == 1 || (e.accumulate == 2 && (p & 1) == 0))
-            r += (double)(e.base ? e.base[p * e.base_stride + off] : *o);
+            r += fp_from(e.base ? e.base[p * e.base_stride + off] : *o);
     } else {
         const uint64_t *a0 = e.a0s[0] ? e.a0s[ct] : e.a0;
-        if (a0 && k == 0) r += (double)a0[(uint64_t)i * n + e.perm[ct][gidx]];
-        if (e.d) r += mulmod_f((double)e.d[p * e.d_stride + off], (double)e.inv2[i].x, q, qinv);
+        if (a0 && k == 0) r += fp_from(a0[(uint64_t)i * n + e.perm[ct][gidx]]);
+        if (e.d) r += mulmod_f(fp_from(e.d[p * e.d_stride + off]), fp_from(e.inv2[i].x), q, qinv);
         o = e.outs[ct] + ((uint64_t)k * l + i) * n + gidx;
     }
     r = reduce_f(r, q, qinv);
-    *o = (uint64_t)(r < 0 ? r + q : r);
-}
-
-// The butterflies of one forward radix-2^K group in registers: local stages
-// s .. s+K-1 of block `blockid`, twiddle row mrow (1 for columns).
-template <int K, bool LAZY>
-__device__ __forceinline__ void fwd_group_f(double *v, int s, uint32_t blockid, uint32_t mrow, const double *tw,
-                                            double q, double qinv)
-{
-#pragma unroll
-    for (int d = 0; d < K; d++) {
-        const int h = 1 << (K - 1 - d);
-#pragma unroll
-        for (int j = 0; j < (1 << d); j++) {
-            const uint32_t b = blockid * (1u << d) + j;
-            const double w = tw[((uint32_t)1 << (s + d)) * mrow + b];
-#pragma unroll
-            for (int u = 0; u < h; u++) {
-                const int t = j * 2 * h + u;
-                const double x = v[t];
-                const double y = mulmod_f(v[t + h], w, q, qinv);
-                if (LAZY) {
-                    v[t] = x + y;
-                    v[t + h] = x - y;
-                } else {
-                    v[t] = reduce_f(x + y, q, qinv);
-                    v[t + h] = reduce_f(x - y, q, qinv);
-                }
-            }
-        }
-    }
-}
-
-// Forward radix-2^K step in double precision (values |v| <= q/2 (1 + eps)).
-// LAZY: the sums and differences are left unreduced (see ntt_tile_f).
-template <int LOGS, int ROLE, int K, int CW, bool LAZY, int NT = kThreads>
-__device__ __forceinline__ void fwd_step_f(double *lds, int s, const double *tw, double q, double qinv, uint32_t m0,
-                                           uint32_t row0)
-{
-    using G = Geometry<LOGS, ROLE, CW>;
-    constexpr int R = 1 << K;
-    constexpr int GROUPS_PER = G::S / R;
-    constexpr int GROUPS = G::TILE / R;
-    const int B = G::S >> s;
-    const int D = B >> K;
-    for (int g = threadIdx.x; g < GROUPS; g += NT) {
-        int cc, gg;
-        if (ROLE == kCol) {
-            cc = g % G::C;
-            gg = g / G::C;
-        } else {
-            cc = g / GROUPS_PER;
-            gg = g % GROUPS_PER;
-        }
-        const int blockid = gg / D;
-        const int o = gg - blockid * D;
-        const uint32_t mrow = (ROLE == kRow) ? (m0 + row0 + cc) : m0;
-        double v[R];
-        int addr[R];
-#pragma unroll
-        for (int t = 0; t < R; t++) {
-            addr[t] = lds_addr<ROLE, G::S, G::C>(cc, blockid * B + o + t * D);
-            v[t] = lds[addr[t]];
-        }
-        fwd_group_f<K, LAZY>(v, s, (uint32_t)blockid, mrow, tw, q, qinv);
-#pragma unroll
-        for (int t = 0; t < R; t++) lds[addr[t]] = v[t];
-    }
-}
-
-// Inverse radix-2^K step in double precision.  LAZY: the products are left
-// unreduced (|v| <= 1.07 q; see ntt_tile_f).
-template <int LOGS, int ROLE, int K, int CW, bool LAZY, int NT = kThreads>
-__device__ __forceinline__ void inv_step_f(double *lds, int s, const double *tw, double q, double qinv, uint32_t n,
-                                           uint32_t mx, uint32_t row0)
-{
-    using G = Geometry<LOGS, ROLE, CW>;
-    constexpr int R = 1 << K;
-    constexpr int GROUPS_PER = G::S / R;
-    constexpr int GROUPS = G::TILE / R;
-    const int so = 1 << s;
-    for (int g = threadIdx.x; g < GROUPS; g += NT) {
-        int cc, gg;
-        if (ROLE == kCol) {
-            cc = g % G::C;
-            gg = g / G::C;
-        } else {
-            cc = g / GROUPS_PER;
-            gg = g % GROUPS_PER;
-        }
-        const int o = gg & (so - 1);
-        const int blockid = gg >> s;
-        const int base = blockid * (so << K) + o;
-        const uint32_t r = row0 + cc;
-        double v[R];
-        int addr[R];
-#pragma unroll
-        for (int t = 0; t < R; t++) {
-            addr[t] = lds_addr<ROLE, G::S, G::C>(cc, base + t * so);
-            v[t] = lds[addr[t]];
-        }
-#pragma unroll
-        for (int d = 0; d < K; d++) {
-            const int sd = s + d;
-            const uint32_t first = n - (mx >> sd) + 1 + (ROLE == kRow ? r * ((uint32_t)G::S >> (sd + 1)) : 0u);
-#pragma unroll
-            for (int j = 0; j < (R >> (d + 1)); j++) {
-                const uint32_t b = (uint32_t)blockid * (uint32_t)(R >> (d + 1)) + j;
-                const double w = tw[first + b];
-#pragma unroll
-                for (int u = 0; u < (1 << d); u++) {
-                    const int t = j * (2 << d) + u;
-                    const double x = v[t], y = v[t + (1 << d)];
-                    v[t] = reduce_f(x + y, q, qinv);
-                    const double p = mulmod_f(x - y, w, q, qinv);
-                    v[t + (1 << d)] = LAZY ? p : reduce_f(p, q, qinv);
-                }
-            }
-        }
-#pragma unroll
-        for (int t = 0; t < R; t++) lds[addr[t]] = v[t];
-    }
-}
-
-// The radix steps of one pass in double precision, barrier after each.
-template <int LOGS, int ROLE, bool FWD, int CW, bool LAZY, int NT = kThreads, bool R16 = false>
-__device__ __forceinline__ void stages_f(double *lds, const double *tw, double q, double qinv, uint32_t n,
-                                         uint32_t N1, uint32_t first)
-{
-    if constexpr (R16) {
-        // radix-16 steps (half the LDS passes and barriers of radix-8), then
-        // the remaining 1..3 stages in one step
-        int s = 0;
-        if (FWD) {
-            const uint32_t m0 = ROLE == kRow ? N1 : 1u;
-#pragma unroll
-            for (int st = 0; st < LOGS / 4; st++) {
-                fwd_step_f<LOGS, ROLE, 4, CW, LAZY, NT>(lds, s, tw, q, qinv, m0, first);
-                s += 4;
-                __syncthreads();
-            }
-            if constexpr (LOGS % 4 != 0) {
-                fwd_step_f<LOGS, ROLE, LOGS % 4, CW, LAZY, NT>(lds, s, tw, q, qinv, m0, first);
-                __syncthreads();
-            }
-        } else {
-            const uint32_t mx = ROLE == kCol ? N1 : n;
-#pragma unroll
-            for (int st = 0; st < LOGS / 4; st++) {
-                inv_step_f<LOGS, ROLE, 4, CW, LAZY, NT>(lds, s, tw, q, qinv, n, mx, first);
-                s += 4;
-                __syncthreads();
-            }
-            if constexpr (LOGS % 4 != 0) {
-                inv_step_f<LOGS, ROLE, LOGS % 4, CW, LAZY, NT>(lds, s, tw, q, qinv, n, mx, first);
-                __syncthreads();
-            }
-        }
-        return;
-    }
-    int s = 0;
-    if (FWD) {
-        const uint32_t m0 = ROLE == kRow ? N1 : 1u;
-        if constexpr (LOGS >= 3) {
-#pragma unroll
-            for (int st = 0; st < LOGS / 3; st++) {
-                fwd_step_f<LOGS, ROLE, 3, CW, LAZY, NT>(lds, s, tw, q, qinv, m0, first);
-                s += 3;
-                __syncthreads();
-            }
-        }
-        if constexpr (LOGS % 3 == 2) {
-            fwd_step_f<LOGS, ROLE, 2, CW, LAZY, NT>(lds, s, tw, q, qinv, m0, first);
-            __syncthreads();
-        } else if constexpr (LOGS % 3 == 1) {
-            fwd_step_f<LOGS, ROLE, 1, CW, LAZY, NT>(lds, s, tw, q, qinv, m0, first);
-            __syncthreads();
-        }
-    } else {
-        const uint32_t mx = ROLE == kCol ? N1 : n;
-        if constexpr (LOGS >= 3) {
-#pragma unroll
-            for (int st = 0; st < LOGS / 3; st++) {
-                inv_step_f<LOGS, ROLE, 3, CW, LAZY, NT>(lds, s, tw, q, qinv, n, mx, first);
-                s += 3;
-                __syncthreads();
-            }
-        }
-        if constexpr (LOGS % 3 == 2) {
-            inv_step_f<LOGS, ROLE, 2, CW, LAZY, NT>(lds, s, tw, q, qinv, n, mx, first);
-            __syncthreads();
-        } else if constexpr (LOGS % 3 == 1) {
-            inv_step_f<LOGS, ROLE, 1, CW, LAZY, NT>(lds, s, tw, q, qinv, n, mx, first);
-            __syncthreads();
-        }
-    }
+    *o = fp_to(r < 0 ? r + q : r);
 }
 
 // The whole transform body of one tile in double precision: load (reduced),
 // the radix steps, store in [0, q) (times n^-1 on the inverse's last pass).
 //
-// Lazy reduction, for primes with q (1/2 + 5/4 LOGS) <= 2^50.  Let B bound |v|.
-// mulmod_f(a, w) for |a| <= 2^50, 0 <= w < q: |h / q - a w / q| <= 3.3 2^-53
-// |a w / q| <= 0.41, so |Q - a w / q| <= 0.91 and the result is below 0.91 q
-// (every intermediate stays an integer below 2^53, as for reduced inputs).
-// Forward (Cooley-Tukey): x +- mulmod_f(y, w) grows B by at most 0.91 q a
-// stage from q/2 after the load, so B <= q (1/2 + 0.91 LOGS) <= 2^50 throughout
-// and no sum needs reducing; the store reduces once.  Inverse
-// (Gentleman-Sande): the sums are reduced (|x + y| <= 1.82 q), the products
-// are not (<= 0.91 q); the store (or the n^-1 product) reduces once.  The
+// Lazy reduction: see reduce_step and the inverse step (ntt_steps.h).  The
 // stored words are the fully reduced residues either way.
 template <int LOGS, int ROLE, bool FWD, int CW, bool R16>
 __device__ __forceinline__ void ntt_tile_f(const NttKArgs &a, uint64_t *lds_words, uint64_t *data,
@@ -480,10 +134,9 @@ __device__ __forceinline__ void ntt_tile_f(const NttKArgs &a, uint64_t *lds_word
     using G = Geometry<LOGS, ROLE, CW>;
     const bool epi = FWD && ROLE != kCol && epi_on(a.epi);
     double *lds = reinterpret_cast<double *>(lds_words);
-    const double q = (double)a.mod[prime].q;
-    const double qinv = 1.0 / q;
+    const double q = a.qd[prime].x, qinv = a.qd[prime].y;
     const double *tw = a.twd + (uint64_t)prime * n;
-    const bool lazy = q * (0.5 + 1.25 * LOGS) <= 0x1p50;  // uniform: one prime per workgroup
+    const bool lazy = FWD ? lazy_forward(q, LOGS) : lazy_inverse(q, LOGS);  // uniform: one prime per workgroup
     if constexpr (FWD && ROLE == kRow && LOGS == 8 && G::C == 8 && !R16) {
         // rows of 256, 8 rows per tile, 256 threads: each thread loads one
         // radix-8 group of the first three stages (row g / 32, positions
@@ -494,7 +147,7 @@ __device__ __forceinline__ void ntt_tile_f(const NttKArgs &a, uint64_t *lds_word
             double v[8];
 #pragma unroll
             for (int t = 0; t < 8; t++)
-                v[t] = reduce_f((double)src[(uint64_t)(first + cc) * G::S + o + 32 * t], q, qinv);
+                v[t] = reduce_f(fp_from(src[(uint64_t)(first + cc) * G::S + o + 32 * t]), q, qinv);
             if (lazy)
                 fwd_group_f<3, true>(v, 0, 0, N1 + first + cc, tw, q, qinv);
             else
@@ -524,7 +177,7 @@ __device__ __forceinline__ void ntt_tile_f(const NttKArgs &a, uint64_t *lds_word
             } else {
                 gidx = e;
             }
-            lds[e] = reduce_f((double)src[gidx], q, qinv);
+            lds[e] = reduce_f(fp_from(src[gidx]), q, qinv);
         }
         __syncthreads();
         if (lazy)
@@ -552,11 +205,11 @@ __device__ __forceinline__ void ntt_tile_f(const NttKArgs &a, uint64_t *lds_word
         v = v < 0 ? v + q : v;
         if (epi) {
             if (a.epi_int)
-                epi_store(a.epi, poly, limb, gidx, (uint64_t)v, (uint64_t)q, a.limbs, n);
+                epi_store(a.epi, poly, limb, gidx, fp_to(v), (uint64_t)q, a.limbs, n);
             else
                 epi_store_f(a.epi, poly, limb, gidx, v, q, qinv, a.limbs, n);
         } else {
-            data[gidx] = (uint64_t)v;
+            data[gidx] = fp_to(v);
         }
     }
 }
@@ -694,62 +347,6 @@ __global__ __launch_bounds__(kThreads) void k_ntt(NttKArgs a)
 // products are the exact double-precision ones of the unfused conversion
 // (k_modup_conv_a), and the column stages those of the double-precision pass,
 // so the stored words equal the unfused conversion followed by the column pass.
-// The column stages of one tile whose values v (this thread's positions
-// e = threadIdx.x + NT t, reduced) are in registers, stored column-transformed
-// into out (positions gidx).  For 2^8-row columns, 8-column tiles and 256
-// threads each thread's 8 positions are exactly one radix-8 group of the first
-// three stages, so those run in registers before the values go to LDS, and
-// the last two stages run in registers on the way out: three LDS passes and
-// three barriers instead of eight passes and four.  The words are the same.
-template <int LOGS, int CW, int NT, int PER, bool LAZY>
-__device__ __forceinline__ void col_stages_store(double *v, double *lds, const double *tw, double q, double qinv,
-                                                 uint32_t n, uint32_t N1, uint32_t N2, uint32_t col0, uint64_t *out,
-                                                 const uint32_t *gidx)
-{
-    if constexpr (LOGS == 8 && CW == 8 && NT == 256 && PER == 8) {
-        fwd_group_f<3, LAZY>(v, 0, 0, 1, tw, q, qinv);  // rows gg + 32 t of column threadIdx.x % 8
-#pragma unroll
-        for (int t = 0; t < PER; t++) lds[threadIdx.x + t * NT] = v[t];
-        __syncthreads();
-        fwd_step_f<LOGS, kCol, 3, CW, LAZY, NT>(lds, 3, tw, q, qinv, 1, col0);
-        __syncthreads();
-        double w[2][4];
-#pragma unroll
-        for (int k = 0; k < 2; k++) {
-            const int g = threadIdx.x + k * NT, cc = g % CW, gg = g / CW;
-#pragma unroll
-            for (int t = 0; t < 4; t++) w[k][t] = lds[(4 * gg + t) * CW + cc];
-        }
-        __syncthreads();  // every read of this tile done before the next one is written
-#pragma unroll
-        for (int k = 0; k < 2; k++) {
-            const int g = threadIdx.x + k * NT, cc = g % CW, gg = g / CW;
-            fwd_group_f<2, LAZY>(w[k], 6, (uint32_t)gg, 1, tw, q, qinv);
-#pragma unroll
-            for (int t = 0; t < 4; t++) {
-                double x = w[k][t];
-                if (LAZY) x = reduce_f(x, q, qinv);
-                x = x < 0 ? x + q : x;
-                out[(uint64_t)(4 * gg + t) * N2 + col0 + cc] = (uint64_t)x;
-            }
-        }
-    } else {
-#pragma unroll
-        for (int t = 0; t < PER; t++) lds[threadIdx.x + t * NT] = v[t];
-        __syncthreads();
-        stages_f<LOGS, kCol, true, CW, LAZY, NT>(lds, tw, q, qinv, n, N1, col0);
-#pragma unroll
-        for (int t = 0; t < PER; t++) {
-            double x = lds[threadIdx.x + t * NT];
-            if (LAZY) x = reduce_f(x, q, qinv);
-            x = x < 0 ? x + q : x;
-            out[gidx[t]] = (uint64_t)x;
-        }
-        // each thread rewrites only the LDS words it has just read: the next
-        // tile's stages start after the barrier that follows those writes
-    }
-}
-
 struct ModUpColArgs {
     uint64_t *T;
     const uint64_t *coef;
@@ -761,75 +358,87 @@ struct ModUpColArgs {
     uint32_t outp[kMaxPrimes];  // words: uniform indices take scalar loads
 };
 
-template <int LOGS, int A, int CW, int NT>
-__global__ __launch_bounds__(NT) void k_modup_col(ModUpColArgs a)
+// RAW: the values are left as doubles for k_row_inner instead of as words.
+// S: the inputs of the digit at hand (A, or half of it for a short last digit).
+// The order of the loop hides the latencies behind arithmetic: an output's
+// twiddles are asked for before its conversion, the next output's factors
+// before the current one's stages.
+template <int LOGS, int A, int S, bool RAW>
+__device__ __forceinline__ void modup_tile(const ModUpColArgs &a, double *lds, uint32_t b, uint32_t j, uint32_t s,
+                                           uint32_t r0, uint32_t r1)
 {
-    using G = Geometry<LOGS, kCol, CW>;
-    constexpr int PER = G::TILE / NT;
-    __shared__ double lds[G::TILE];
+    using C = ColTile<LOGS>;
     const uint32_t n = 1u << a.logn;
-    const uint32_t N2 = n >> LOGS, N1 = 1u << LOGS;
+    const uint32_t N2 = n >> LOGS;
+    const uint32_t first = j * A;
+    const uint32_t col0 = xcd_tile(blockIdx.x, gridDim.x) * C::CW;
+    const int tid = threadIdx.x;
+    const uint32_t at = (uint32_t)(tid / C::CW) * N2 + col0 + tid % C::CW;
+    // the digit's products [x Dhat^-1]_q in [0, q) (rows i >= s stay zero)
+    const uint32_t base = (j * A + s - 1) * A;
+    double y[S][8];
+    double qmax = 0.0;
+#pragma unroll
+    for (int i = 0; i < S; i++) {
+        const bool on = (uint32_t)i < s;
+        const uint32_t p = on ? first + i : first;
+        const double q = a.qd[p].x, qinv = a.qd[p].y;
+        qmax = q > qmax ? q : qmax;
+        const double wi = (double)a.w[base + (on ? i : 0)].x;
+        const uint64_t *x = a.coef + ((uint64_t)b * a.l + p) * n;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            double v = reduce_f(mulmod_f(fp_from((x + C::row_step(k) * N2)[at]), wi, q, qinv), q, qinv);
+            v = v < 0 ? v + q : v;
+            y[i][k] = on ? v : 0.0;
+        }
+    }
+    const double *factors = a.convd + (uint64_t)base * a.key_limbs;
+    auto prime = [&](uint32_t r) { return a.outp[r < first ? r : r + s]; };
+    double f[S], q, qinv;
+    auto load_factors = [&](uint32_t kp) {
+#pragma unroll
+        for (int i = 0; i < S; i++) f[i] = table(factors, (uint64_t)i * a.key_limbs + kp);
+        table_prime(a.qd, kp, q, qinv);
+    };
+    load_factors(prime(r0));
+    ColTwiddles<LOGS> tw, next;
+    next.load_lane(a.twd + (uint64_t)prime(r0) * n);
+    uint32_t buf = 0;
+    for (uint32_t r = r0; r < r1; r++, buf ^= 1) {
+        const uint32_t I = r < first ? r : r + s;
+        const double qc = q, qic = qinv;
+        tw = next;
+        tw.load_uniform(a.twd + (uint64_t)prime(r) * n);
+        __builtin_amdgcn_sched_barrier(0);
+        double cv[8];
+        conv_tile<S>(cv, &y[0][0], f, qc, qic, qmax * qc <= 0x1p97);
+        __builtin_amdgcn_sched_barrier(0);
+        const uint32_t kn = prime(min(r + 1, r1 - 1));
+        load_factors(kn);
+        next.load_lane(a.twd + (uint64_t)kn * n);
+        __builtin_amdgcn_sched_barrier(0);
+        col_forward<LOGS, RAW>(cv, lds + buf * C::LDS, tw, qc, qic, (int)a.logn, N2, col0,
+                               a.T + (((uint64_t)b * a.nout + I) * a.digits + j) * n);
+    }
+}
+
+template <int LOGS, int A, bool RAW>
+__global__ __launch_bounds__(kThreads, A <= 9 ? 2 : 1) void k_modup_col(ModUpColArgs a)
+{
+    __shared__ double lds[2 * ColTile<LOGS>::LDS];
     const uint32_t row = blockIdx.y;  // (b * digits + j) * chunks + chunk
     const uint32_t bj = row / a.chunks, chunk = row - bj * a.chunks;
     const uint32_t b = bj / a.digits, j = bj - b * a.digits;
-    const uint32_t first = j * A;
-    const uint32_t s = min((uint32_t)A, a.l - first);
+    const uint32_t s = min((uint32_t)A, a.l - j * A);
     const uint32_t count = a.nout - s;  // output primes outside the digit
     const uint32_t r0 = chunk * a.chunk;
     if (r0 >= count) return;  // uniform, before any barrier
     const uint32_t r1 = min(count, r0 + a.chunk);
-    uint32_t tile = blockIdx.x;
-    if ((gridDim.x & 7) == 0) tile = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-    const uint32_t col0 = tile * G::C;
-    uint32_t gidx[PER];
-#pragma unroll
-    for (int t = 0; t < PER; t++) {
-        const int e = threadIdx.x + t * NT;
-        gidx[t] = (uint32_t)(e / G::C) * N2 + col0 + (uint32_t)(e % G::C);
-    }
-    // the digit's products [x Dhat^-1]_q in [0, q) (rows i >= s stay zero)
-    const uint32_t base = (j * A + s - 1) * A;
-    double y[A][PER];
-#pragma unroll
-    for (int i = 0; i < A; i++) {
-        const bool on = (uint32_t)i < s;
-        const uint32_t p = on ? first + i : first;
-        const double q = a.qd[p].x, qinv = a.qd[p].y;
-        const double wi = (double)a.w[base + (on ? i : 0)].x;
-        const uint64_t *x = a.coef + ((uint64_t)b * a.l + p) * n;
-#pragma unroll
-        for (int t = 0; t < PER; t++) {
-            double v = reduce_f(mulmod_f((double)x[gidx[t]], wi, q, qinv), q, qinv);
-            v = v < 0 ? v + q : v;
-            y[i][t] = on ? v : 0.0;
-        }
-    }
-    for (uint32_t r = r0; r < r1; r++) {
-        const uint32_t I = r < first ? r : r + s;
-        const uint32_t kp = a.outp[I];
-        const double q = a.qd[kp].x, qinv = a.qd[kp].y;
-        const double *fd = a.convd + (uint64_t)base * a.key_limbs + kp;
-        double f[A];
-#pragma unroll
-        for (int i = 0; i < A; i++) f[i] = fd[(uint64_t)i * a.key_limbs];
-        double cv[PER];
-#pragma unroll
-        for (int t = 0; t < PER; t++) {
-            double acc = 0.0;
-#pragma unroll
-            for (int i = 0; i < A; i++) {
-                acc += mulmod_f(y[i][t], f[i], q, qinv);
-                if (i & 1) acc = reduce_f(acc, q, qinv);
-            }
-            cv[t] = reduce_f(acc, q, qinv);  // |v| <= q/2 (1 + eps)
-        }
-        const double *tw = a.twd + (uint64_t)kp * n;
-        uint64_t *out = a.T + (((uint64_t)b * a.nout + I) * a.digits + j) * n;
-        if (q * (0.5 + 1.25 * LOGS) <= 0x1p50)  // uniform
-            col_stages_store<LOGS, CW, NT, PER, true>(cv, lds, tw, q, qinv, n, N1, N2, col0, out, gidx);
-        else
-            col_stages_store<LOGS, CW, NT, PER, false>(cv, lds, tw, q, qinv, n, N1, N2, col0, out, gidx);
-    }
+    if (A > 4 && s <= A / 2)
+        modup_tile<LOGS, A, A / 2, RAW>(a, lds, b, j, s, r0, r1);
+    else
+        modup_tile<LOGS, A, A, RAW>(a, lds, b, j, s, r0, r1);
 }
 
 // ---- ModDown base conversion fused into the forward column pass
@@ -863,40 +472,39 @@ struct CenterColArgs {
 template <int LOGS>
 __global__ __launch_bounds__(kThreads) void k_center_col(CenterColArgs a)
 {
-    using G = Geometry<LOGS, kCol, 8>;
-    constexpr int PER = G::TILE / kThreads;
-    __shared__ double lds[G::TILE];
+    using C = ColTile<LOGS>;
+    __shared__ double lds[2 * C::LDS];
     const uint32_t n = 1u << a.logn;
-    const uint32_t N2 = n >> LOGS, N1 = 1u << LOGS;
+    const uint32_t N2 = n >> LOGS;
     const uint32_t p = blockIdx.y / a.chunks, chunk = blockIdx.y - p * a.chunks;
     const uint32_t i0 = chunk * a.chunk;
     if (i0 >= a.limbs) return;  // uniform, before any barrier
     const uint32_t i1 = min(a.limbs, i0 + a.chunk);
-    uint32_t tile = blockIdx.x;
-    if ((gridDim.x & 7) == 0) tile = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-    const uint32_t col0 = tile * G::C;
-    uint32_t gidx[PER];
-    double v[PER];
+    const uint32_t col0 = xcd_tile(blockIdx.x, gridDim.x) * C::CW;
+    const int tid = threadIdx.x;
+    double v[8];
+    const uint32_t at = (uint32_t)(tid / C::CW) * N2 + col0 + tid % C::CW;
     const uint64_t *x = a.last + (uint64_t)p * a.last_stride;
 #pragma unroll
-    for (int t = 0; t < PER; t++) {
-        const int e = threadIdx.x + t * kThreads;
-        gidx[t] = (uint32_t)(e / G::C) * N2 + col0 + (uint32_t)(e % G::C);
-        uint64_t u = x[gidx[t]] + a.half;
+    for (int k = 0; k < 8; k++) {
+        uint64_t u = (x + C::row_step(k) * N2)[at] + a.half;
         u = u >= a.p ? u - a.p : u;
-        v[t] = (double)u - (double)a.half;
+        v[k] = fp_from(u) - fp_from(a.half);
     }
-    for (uint32_t i = i0; i < i1; i++) {
-        const double q = a.qd[i].x, qinv = a.qd[i].y;
-        double cv[PER];
+    uint32_t buf = 0;
+    ColTwiddles<LOGS> tw, next;
+    next.load_lane(a.twd + (uint64_t)i0 * n);
+    for (uint32_t i = i0; i < i1; i++, buf ^= 1) {
+        double q, qinv;
+        table_prime(a.qd, i, q, qinv);
+        tw = next;
+        tw.load_uniform(a.twd + (uint64_t)i * n);
+        double cv[8];
 #pragma unroll
-        for (int t = 0; t < PER; t++) cv[t] = reduce_f(v[t], q, qinv);
-        const double *tw = a.twd + (uint64_t)i * n;
-        uint64_t *out = a.z + ((uint64_t)p * a.limbs + i) * n;
-        if (q * (0.5 + 1.25 * LOGS) <= 0x1p50)  // uniform
-            col_stages_store<LOGS, 8, kThreads, PER, true>(cv, lds, tw, q, qinv, n, N1, N2, col0, out, gidx);
-        else
-            col_stages_store<LOGS, 8, kThreads, PER, false>(cv, lds, tw, q, qinv, n, N1, N2, col0, out, gidx);
+        for (int k = 0; k < 8; k++) cv[k] = reduce_f(v[k], q, qinv);
+        next.load_lane(a.twd + (uint64_t)min(i + 1, i1 - 1) * n);
+        col_forward<LOGS, false>(cv, lds + buf * C::LDS, tw, q, qinv, (int)a.logn, N2, col0,
+                                 a.z + ((uint64_t)p * a.limbs + i) * n);
     }
 }
 
@@ -913,68 +521,68 @@ struct ModDownColArgs {
     uint32_t inp[kMaxPrimes];
 };
 
-template <int LOGS, int A, int CW, int NT>
-__global__ __launch_bounds__(NT) void k_moddown_col(ModDownColArgs a)
+template <int LOGS, int A>
+__global__ __launch_bounds__(kThreads, A <= 9 ? 2 : 1) void k_moddown_col(ModDownColArgs a)
 {
-    using G = Geometry<LOGS, kCol, CW>;
-    constexpr int PER = G::TILE / NT;
-    __shared__ double lds[G::TILE];
+    using C = ColTile<LOGS>;
+    __shared__ double lds[2 * C::LDS];
     const uint32_t n = 1u << a.logn;
-    const uint32_t N2 = n >> LOGS, N1 = 1u << LOGS;
+    const uint32_t N2 = n >> LOGS;
     const uint32_t p = blockIdx.y / a.chunks, chunk = blockIdx.y - p * a.chunks;
     const uint32_t i0 = chunk * a.chunk;
     if (i0 >= a.lo) return;  // uniform, before any barrier
     const uint32_t i1 = min(a.lo, i0 + a.chunk);
-    uint32_t tile = blockIdx.x;
-    if ((gridDim.x & 7) == 0) tile = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-    const uint32_t col0 = tile * G::C;
-    uint32_t gidx[PER];
-#pragma unroll
-    for (int t = 0; t < PER; t++) {
-        const int e = threadIdx.x + t * NT;
-        gidx[t] = (uint32_t)(e / G::C) * N2 + col0 + (uint32_t)(e % G::C);
-    }
+    const uint32_t col0 = xcd_tile(blockIdx.x, gridDim.x) * C::CW;
+    const int tid = threadIdx.x;
+    const uint32_t at = (uint32_t)(tid / C::CW) * N2 + col0 + tid % C::CW;
     const uint64_t *y = a.acc + (uint64_t)p * a.acc_stride + (uint64_t)a.lo * n;
-    double v[A][PER], rr[PER];
-    double frac[PER];
+    double v[A][8], rr[8];
+    double pmax = 0.0;
 #pragma unroll
-    for (int t = 0; t < PER; t++) frac[t] = 0.0;
+    for (int k = 0; k < 8; k++) rr[k] = 0.0;
 #pragma unroll
-    for (int k = 0; k < A; k++) {
-        const ulonglong2 wk = a.w[k];
-        const uint64_t pk = a.mod[a.inp[k]].q;
+    for (int i = 0; i < A; i++) {
+        const double wi = (double)a.w[i].x;
+        const double pi = a.qd[a.inp[i]].x, pinv = a.qd[a.inp[i]].y;
+        pmax = pi > pmax ? pi : pmax;
 #pragma unroll
-        for (int t = 0; t < PER; t++) {
-            const uint64_t x = shoup(y[(uint64_t)k * n + gidx[t]], wk.x, wk.y, pk);
-            frac[t] += (double)x / (double)pk;
-            v[k][t] = (double)x;
+        for (int k = 0; k < 8; k++) {
+            double x = reduce_f(mulmod_f(fp_from((y + (uint64_t)i * n + C::row_step(k) * N2)[at]), wi, pi, pinv),
+                                pi, pinv);
+            x = x < 0 ? x + pi : x;
+            // x / p_i correctly rounded: pinv is the correctly rounded 1 / p_i, so
+            // one residual step on x pinv gives the quotient a division gives
+            const double d = x * pinv;
+            rr[k] += __builtin_fma(__builtin_fma(-d, pi, x), pinv, d);
+            v[i][k] = x;
         }
     }
 #pragma unroll
-    for (int t = 0; t < PER; t++) rr[t] = (double)(uint32_t)(uint64_t)floor(frac[t] + 0.5);  // <= A
-    for (uint32_t i = i0; i < i1; i++) {
-        const double q = a.qd[i].x, qinv = a.qd[i].y;
-        double f[A + 1];
+    for (int k = 0; k < 8; k++) rr[k] = __builtin_floor(rr[k] + 0.5);  // <= A
+    double f[A + 1], q, qinv;
+    auto load_factors = [&](uint32_t i) {
 #pragma unroll
-        for (int k = 0; k <= A; k++) f[k] = a.convd[(uint64_t)k * a.L + i];
-        double cv[PER];
+        for (int k = 0; k <= A; k++) f[k] = table(a.convd, (uint64_t)k * a.L + i);
+        table_prime(a.qd, i, q, qinv);
+    };
+    load_factors(i0);
+    ColTwiddles<LOGS> tw;
+    uint32_t buf = 0;
+    for (uint32_t i = i0; i < i1; i++, buf ^= 1) {
+        const double qc = q, qic = qinv;
+        tw.load_lane(a.twd + (uint64_t)i * n);
+        tw.load_uniform(a.twd + (uint64_t)i * n);
+        __builtin_amdgcn_sched_barrier(0);
+        double cv[8];
+        conv_tile<A>(cv, &v[0][0], f, qc, qic, pmax * qc <= 0x1p97);
+        // - r (P mod q_i) as r times the centred q_i - P mod q_i
 #pragma unroll
-        for (int t = 0; t < PER; t++) {
-            // - r (P mod q_i) as r (q_i - P mod q_i)
-            double s = mulmod_f(rr[t], f[A], q, qinv);
-#pragma unroll
-            for (int k = 0; k < A; k++) {
-                s += mulmod_f(v[k][t], f[k], q, qinv);
-                if (k & 1) s = reduce_f(s, q, qinv);
-            }
-            cv[t] = reduce_f(s, q, qinv);  // |v| <= q/2 (1 + eps)
-        }
-        const double *tw = a.twd + (uint64_t)i * n;
-        uint64_t *out = a.z + ((uint64_t)p * a.lo + i) * n;
-        if (q * (0.5 + 1.25 * LOGS) <= 0x1p50)  // uniform
-            col_stages_store<LOGS, CW, NT, PER, true>(cv, lds, tw, q, qinv, n, N1, N2, col0, out, gidx);
-        else
-            col_stages_store<LOGS, CW, NT, PER, false>(cv, lds, tw, q, qinv, n, N1, N2, col0, out, gidx);
+        for (int k = 0; k < 8; k++) cv[k] = reduce_f(cv[k] + mulmod_f(rr[k], f[A], qc, qic), qc, qic);
+        __builtin_amdgcn_sched_barrier(0);
+        load_factors(min(i + 1, i1 - 1));
+        __builtin_amdgcn_sched_barrier(0);
+        col_forward<LOGS, false>(cv, lds + buf * C::LDS, tw, qc, qic, (int)a.logn, N2, col0,
+                                 a.z + ((uint64_t)p * a.lo + i) * n);
     }
 }
 
@@ -1123,6 +731,7 @@ NttKArgs make_args(const DeviceTables &t, const NttBatch &b, bool fwd)
     a.poly_period = b.poly_period;
     a.tw = fwd ? t.fwd : t.inv;
     a.mod = t.mod;
+    a.qd = t.qd;
     a.ninv = t.ninv;
     a.twd = fwd ? t.fwd_d : t.inv_d;
     a.ninvd = t.ninv_d;
@@ -1203,9 +812,7 @@ inline double col_flops(int logs) { return logs * (kFlopsProduct + 2.0) / 2.0 + 
 // column pass as separate launches), k > 0 = on with k outputs per workgroup.
 // Process-wide; set by the autotuner.
 static std::atomic<int> g_modup_col[kTuneBuckets];
-constexpr int kColNarrow = 256;  // mode bit: 4-column tiles
 constexpr int kColMaxA = 12;   // largest digit / special-prime count of the fused conversions
-constexpr int kColWide = 512;    // mode bit: 512 threads per workgroup (8-column tiles, half the registers each)
 
 void ks_modup_col_set(uint32_t B, int mode) { g_modup_col[tune_bucket(B)].store(mode); }
 
@@ -1219,7 +826,7 @@ bool ks_modup_col_ok(const DeviceTables &t, uint32_t alpha)
 
 void ks_modup_convert_col(const DeviceTables &t, uint64_t *T, const uint64_t *coef, const ulonglong2 *w,
                           uint32_t B, uint32_t l, uint32_t alpha, uint32_t key_limbs, const uint8_t *out_primes_host,
-                          uint32_t nout, hipStream_t s)
+                          uint32_t nout, hipStream_t s, bool raw)
 {
     if (!ks_modup_col_ok(t, alpha)) throw std::invalid_argument("ks_modup_convert_col: unsupported parameters");
     if (nout > (uint32_t)kMaxPrimes || l < 1 || nout <= alpha) throw std::invalid_argument("ks_modup_convert_col: bad sizes");
@@ -1239,12 +846,9 @@ void ks_modup_convert_col(const DeviceTables &t, uint64_t *T, const uint64_t *co
     int l1, l2;
     split_logn(t.logn, l1, l2);
     const uint32_t n = 1u << t.logn;
-    // mode: outputs per workgroup in its low byte (0: default rule), 4-column
-    // tiles (half the registers per thread) when bit 8 is set
+    // mode: outputs per workgroup (0: default rule)
     const int mode = g_modup_col[tune_bucket(B)].load();
-    const uint32_t cw = (mode > 0 && (mode & kColNarrow)) ? 4u : 8u;
-    const uint32_t nt = (mode > 0 && (mode & kColWide)) ? 512u : 256u;
-    const uint32_t tiles = n / ((1u << l1) * cw);
+    const uint32_t tiles = n / 2048u;
     // outputs per workgroup: enough workgroups to fill the device, at least 4
     // outputs per read of the digit's inputs
     const uint32_t count = nout - std::min(alpha, l);  // most outputs of a digit (a partial digit has more)
@@ -1260,15 +864,13 @@ void ks_modup_convert_col(const DeviceTables &t, uint64_t *T, const uint64_t *co
                    8.0 * n * ((double)B * l + (double)B * outs) + 8.0 * (double)(1u << l1) * B * outs,
                    (double)n * B * ((double)l * kFlopsProduct + outs * (conv_flops(alpha) + col_flops(l1))));
     const dim3 grid(tiles, B * a.digits * a.chunks);
-#define NX_MC(LOGS, A)                                                                          \
-    if (l1 == LOGS && alpha == A) {                                                           \
-        if (cw == 4)                                                                          \
-            hipLaunchKernelGGL((k_modup_col<LOGS, A, 4, 256>), grid, dim3(256), 0, s, a);      \
-        else if (nt == 512 || A > 8)                                                          \
-            hipLaunchKernelGGL((k_modup_col<LOGS, A, 8, 512>), grid, dim3(512), 0, s, a);      \
-        else                                                                                  \
-            hipLaunchKernelGGL((k_modup_col<LOGS, A, 8, (A > 8 ? 512 : 256)>), grid, dim3(A > 8 ? 512 : 256), 0, s, a); \
-        return;                                                                               \
+#define NX_MC(LOGS, A)                                                                      \
+    if (l1 == LOGS && alpha == A) {                                                       \
+        if (raw)                                                                          \
+            hipLaunchKernelGGL((k_modup_col<LOGS, A, true>), grid, dim3(kThreads), 0, s, a);  \
+        else                                                                              \
+            hipLaunchKernelGGL((k_modup_col<LOGS, A, false>), grid, dim3(kThreads), 0, s, a); \
+        return;                                                                           \
     }
     NX_MC(7, 2) NX_MC(7, 3) NX_MC(7, 4) NX_MC(7, 5) NX_MC(7, 6) NX_MC(7, 7) NX_MC(7, 8) NX_MC(7, 9) NX_MC(7, 10)
     NX_MC(7, 11) NX_MC(7, 12)
@@ -1297,7 +899,7 @@ void rns_center_last_col(const DeviceTables &t, uint64_t *z, const uint64_t *las
     int l1, l2;
     split_logn(t.logn, l1, l2);
     const uint32_t n = 1u << t.logn;
-    const uint32_t tiles = n / ((1u << l1) * 8u);
+    const uint32_t tiles = n / 2048u;
     const uint32_t want = (2048u + tiles * polys - 1) / (tiles * polys);
     uint32_t chunk = (limbs + want - 1) / want;
     chunk = std::max(chunk, std::min(4u, limbs));
@@ -1348,9 +950,7 @@ void ks_moddown_convert_col(const DeviceTables &t, uint64_t *z, const uint64_t *
     split_logn(t.logn, l1, l2);
     const uint32_t n = 1u << t.logn;
     const int mode = g_moddown_col[tune_bucket(polys)].load();
-    const uint32_t cw = (mode > 0 && (mode & kColNarrow)) ? 4u : 8u;
-    const uint32_t nt = (mode > 0 && (mode & kColWide)) ? 512u : 256u;
-    const uint32_t tiles = n / ((1u << l1) * cw);
+    const uint32_t tiles = n / 2048u;
     const uint32_t want = (2048u + tiles * polys - 1) / (tiles * polys);
     uint32_t chunk = (lo + want - 1) / want;
     chunk = std::max(chunk, std::min(4u, lo));
@@ -1361,15 +961,10 @@ void ks_moddown_convert_col(const DeviceTables &t, uint64_t *z, const uint64_t *
                    8.0 * n * polys * ((double)A + lo) + 8.0 * (double)(1u << l1) * polys * lo,
                    (double)n * polys * ((double)A * 2.0 + lo * (conv_flops(A + 1) + col_flops(l1))));
     const dim3 grid(tiles, polys * a.chunks);
-#define NX_MD(LOGS, AA)                                                                         \
-    if (l1 == LOGS && A == AA) {                                                              \
-        if (cw == 4)                                                                          \
-            hipLaunchKernelGGL((k_moddown_col<LOGS, AA, 4, 256>), grid, dim3(256), 0, s, a);   \
-        else if (nt == 512 || AA > 9)                                                         \
-            hipLaunchKernelGGL((k_moddown_col<LOGS, AA, 8, 512>), grid, dim3(512), 0, s, a);   \
-        else                                                                                  \
-            hipLaunchKernelGGL((k_moddown_col<LOGS, AA, 8, (AA > 9 ? 512 : 256)>), grid, dim3(AA > 9 ? 512 : 256), 0, s, a); \
-        return;                                                                               \
+#define NX_MD(LOGS, AA)                                                                     \
+    if (l1 == LOGS && A == AA) {                                                          \
+        hipLaunchKernelGGL((k_moddown_col<LOGS, AA>), grid, dim3(kThreads), 0, s, a);       \
+        return;                                                                           \
     }
     NX_MD(7, 2) NX_MD(7, 3) NX_MD(7, 4) NX_MD(7, 5) NX_MD(7, 6) NX_MD(7, 7) NX_MD(7, 8) NX_MD(7, 9) NX_MD(7, 10)
     NX_MD(7, 11) NX_MD(7, 12) NX_MD(7, 13)

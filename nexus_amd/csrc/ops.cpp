@@ -268,6 +268,25 @@ void ks_out_primes(const Context &c, size_t l, uint8_t *outp)
     for (size_t k = 0; k < c.alpha; k++) outp[l + k] = (uint8_t)(c.L + k);
 }
 
+// INTT of the targets ([B][l][n], or B <= kNttSrcMax pointers) into coef
+static void ks_coefficients(Context &c, uint64_t *coef, const uint64_t *targets, const uint64_t *const *target_list,
+                            size_t B, size_t l)
+{
+    if (!target_list) {
+        ntt_inv_from(c, coef, targets, B, l, l * c.n, l * c.n);
+        return;
+    }
+    NttBatch b;
+    b.data = coef;
+    b.poly_stride = l * c.n;
+    b.polys = (uint32_t)B;
+    b.limbs = (uint32_t)l;
+    b.prime_by_poly = 0;
+    for (int i = 0; i < kMaxPrimes; i++) b.prime_of[i] = (uint8_t)i;
+    b.src_list = target_list;
+    ntt_inverse(c.tables, b, c.stream);
+}
+
 static DevBuf ks_modup_impl(Context &c, const uint64_t *targets, const uint64_t *const *target_list, size_t B,
                             size_t l)
 {
@@ -277,19 +296,7 @@ static DevBuf ks_modup_impl(Context &c, const uint64_t *targets, const uint64_t 
     uint8_t outp[kMaxPrimes];
     ks_out_primes(c, l, outp);
     DevBuf coef(&c, B * l * n);
-    if (target_list) {
-        NttBatch b;
-        b.data = coef.get();
-        b.poly_stride = l * n;
-        b.polys = (uint32_t)B;
-        b.limbs = (uint32_t)l;
-        b.prime_by_poly = 0;
-        for (int i = 0; i < kMaxPrimes; i++) b.prime_of[i] = (uint8_t)i;
-        b.src_list = target_list;
-        ntt_inverse(c.tables, b, c.stream);
-    } else {
-        ntt_inv_from(c, coef.get(), targets, B, l, l * n, l * n);
-    }
+    ks_coefficients(c, coef.get(), targets, target_list, B, l);
     DevBuf T(&c, B * nout * digits * n);
     if (c.alpha > 1 && ks_modup_col_ok(c.tables, (uint32_t)c.alpha) && ks_modup_col_get((uint32_t)B) >= 0) {
         // the conversion feeds the forward column pass directly; the digits'
@@ -350,18 +357,89 @@ DevBuf ks_modup_list(Context &c, const uint64_t *const *targets, size_t B, size_
     return ks_modup_impl(c, nullptr, targets, B, l);
 }
 
+bool ks_rows_fused(const Context &c) { return ks_row_inner_ok(c.tables, (uint32_t)c.alpha); }
+
+// Words of digits in flight between the column pass and the inner product (2
+// GiB).  Smaller chunks that stay in the 256 MB last-level cache measured
+// slower (64 fused products at 20 limbs, N = 2^16: 7.12 ms at 256 MB, 6.80 at
+// 768 MB, 6.67 at 1.5 GB and beyond): the kernels are not bound by memory, and
+// shorter launches leave more of the device idle at their ends.
+constexpr size_t kDigitWords = (size_t)1 << 28;
+
+void ks_inner(Context &c, uint64_t *acc, const uint64_t *targets, const uint64_t *const *target_list, size_t B,
+              size_t l, const uint64_t *const *keys, const uint64_t *const *aseeds, const uint32_t *const *perms,
+              bool accumulate)
+{
+    const size_t n = c.n, nout = l + c.alpha, digits = c.digits(l);
+    uint8_t outp[kMaxPrimes];
+    ks_out_primes(c, l, outp);
+    DevBuf coef(&c, B * l * n);
+    ks_coefficients(c, coef.get(), targets, target_list, B, l);
+    KsRowInner p;
+    p.l = (uint32_t)l;
+    p.alpha = (uint32_t)c.alpha;
+    p.digits = (uint32_t)digits;
+    p.nout = (uint32_t)nout;
+    p.key_limbs = (uint32_t)c.key_limbs();
+    p.out_primes = outp;
+    // chunks of inputs; one input alone is cut by output primes where a digit
+    // is cheap to read again (one prime)
+    const size_t per = nout * digits * n, most = kDigitWords;
+    const size_t bc = std::max<size_t>(1, std::min({B, most / per, (size_t)kMaxHoist}));
+    size_t ic = nout;
+    if (c.alpha == 1 && bc == 1) ic = std::max<size_t>(1, std::min(nout, most / (digits * n)));
+    const size_t parts = (nout + ic - 1) / ic;
+    ic = (nout + parts - 1) / parts;
+    DevBuf T(&c, bc * ic * digits * n);
+    for (size_t b0 = 0; b0 < B; b0 += bc) {
+        const size_t cnt = std::min(bc, B - b0);
+        const uint64_t *x = coef.get() + b0 * l * n;
+        p.T = T.get();
+        p.count = (uint32_t)cnt;
+        p.own = targets ? targets + b0 * l * n : nullptr;
+        p.own_list = target_list ? target_list + b0 : nullptr;
+        p.keys = perms ? keys + b0 : keys;
+        p.aseeds = perms ? aseeds + b0 : aseeds;
+        p.perms = perms ? perms + b0 : nullptr;
+        p.acc = perms ? acc : acc + b0 * 2 * nout * n;
+        p.accumulate = perms && (accumulate || b0);
+        for (size_t i0 = 0; i0 < nout; i0 += ic) {
+            p.i0 = (uint32_t)i0;
+            p.icount = (uint32_t)std::min(ic, nout - i0);
+            p.t_stride = p.icount * digits * n;
+            if (c.alpha == 1)
+                ks_lift_col(c.tables, T.get(), x, (uint32_t)cnt, (uint32_t)l, p.i0, p.icount, outp, (uint32_t)nout,
+                            c.stream);
+            else
+                ks_modup_convert_col(c.tables, T.get(), x, c.d_modup_w, (uint32_t)cnt, (uint32_t)l,
+                                     (uint32_t)c.alpha, (uint32_t)c.key_limbs(), outp, (uint32_t)nout, c.stream, true);
+            ks_row_inner(c.tables, p, c.stream);
+        }
+    }
+}
+
+void ks_inner_one_key(Context &c, uint64_t *acc, const uint64_t *targets, size_t B, size_t l, const DevBuf &key,
+                      const uint64_t *aseed)
+{
+    if (ks_rows_fused(c)) {
+        const uint64_t *k = key.get();
+        ks_inner(c, acc, targets, nullptr, B, l, &k, &aseed, nullptr, false);
+        return;
+    }
+    uint8_t outp[kMaxPrimes];
+    ks_out_primes(c, l, outp);
+    DevBuf T = ks_modup(c, targets, B, l);
+    ks_inner_product(c.tables, acc, T.get(), key.get(), (uint32_t)B, (uint32_t)c.digits(l), (uint32_t)c.key_limbs(),
+                     outp, (uint32_t)(l + c.alpha), c.stream, aseed);
+}
+
 void key_switch_batch(Context &c, uint64_t *cts, const uint64_t *targets, size_t B, size_t l, const DevBuf &key,
                       bool zero_c1, const uint64_t *base, const uint64_t *aseed)
 {
     tally("ks", l, (double)B);
-    const size_t n = c.n, nout = l + c.alpha;
-    uint8_t outp[kMaxPrimes];
-    ks_out_primes(c, l, outp);
-    DevBuf T = ks_modup(c, targets, B, l);
-    // inner product with the device-resident key
-    DevBuf acc(&c, B * 2 * nout * n);
-    ks_inner_product(c.tables, acc.get(), T.get(), key.get(), (uint32_t)B, (uint32_t)c.digits(l),
-                     (uint32_t)c.key_limbs(), outp, (uint32_t)nout, c.stream, aseed);
+    // inner product of the digits with the device-resident key
+    DevBuf acc(&c, B * 2 * (l + c.alpha) * c.n);
+    ks_inner_one_key(c, acc.get(), targets, B, l, key, aseed);
     ks_moddown(c, cts, acc.get(), B, l, zero_c1, base);
 }
 
@@ -756,8 +834,6 @@ void op_multiply_relin_rescale_fused_many(const std::vector<const Ciphertext *> 
         require(a[r]->size == 2 && b[r]->size == 2, "multiply expects two size-2 ciphertexts (relinearize first)");
         require(scale_within_bounds(c, a[r]->scale * b[r]->scale, l), "scale out of bounds");
     }
-    uint8_t outp[kMaxPrimes];
-    ks_out_primes(c, l, outp);
     const size_t A = alpha + 1, lo = l - 1;
     std::vector<Ciphertext> res(a.size());
     // every buffer of a chunk is contiguous: up to one epilogue output per product
@@ -772,11 +848,7 @@ void op_multiply_relin_rescale_fused_many(const std::vector<const Ciphertext *> 
         DevBuf c01(&c, cnt * 2 * pw), c2(&c, cnt * pw);
         poly_tensor_many(c.tables, c01.get(), c2.get(), pa.data(), pb.data(), (uint32_t)cnt, (uint32_t)l, c.stream);
         DevBuf acc(&c, cnt * 2 * nout * n);
-        {
-            DevBuf T = ks_modup(c, c2.get(), cnt, l);
-            ks_inner_product(c.tables, acc.get(), T.get(), key.get(), (uint32_t)cnt, (uint32_t)c.digits(l),
-                             (uint32_t)c.key_limbs(), outp, (uint32_t)nout, c.stream, rk.seeds_of(0));
-        }
+        ks_inner_one_key(c, acc.get(), c2.get(), cnt, l, key, rk.seeds_of(0));
         // limb q_(l-1) of Y = acc + P d, then (q_(l-1), p_0..p_(alpha-1)) to coefficients
         rns_add_limb_scaled(c.tables, acc.get(), nout * n, c01.get(), pw, (uint32_t)lo, c.mdr_pmod[l],
                             (uint32_t)(2 * cnt), c.stream);
