@@ -405,8 +405,9 @@ struct PeriodicPlain {
     DevBuf table;
     // device term lists of block_mix, per index pattern (M, K, index)
     struct Terms {
-        DevBuf words;  // first[M + 1] (u32) then (k, entry) int32 pairs, 8-byte aligned
-        uint32_t M = 0, nterms = 0;
+        DevBuf words;  // first[M + 1] (u32, padded), the runs (int32 quads), then block_mix_plan at word `plan`
+        uint32_t M = 0;
+        size_t plan = 0;
     };
     std::map<std::vector<int32_t>, Terms> terms;
     std::mutex mu;

@@ -107,7 +107,7 @@ void periodic_create(Context &c, const double *values, size_t period, size_t cou
     b.prime_by_poly = 0;
     for (int i = 0; i < kMaxPrimes; i++) b.prime_of[i] = (uint8_t)i;
     ntt_forward(c.tables, b, c.stream);
-    periodic_gather(c.tables, table.get(), fl, work.get(), (uint32_t)rows, (uint32_t)B, c.stream);
+    periodic_gather(c.tables, table.get(), fl, work.get(), (uint32_t)count, (uint32_t)limbs, (uint32_t)B, c.stream);
     std::vector<uint8_t> hf(rows * B);
     NX_HIP(hipMemcpyAsync(hf.data(), fl, hf.size(), hipMemcpyDeviceToHost, c.stream));
     NX_HIP(hipStreamSynchronize(c.stream));
@@ -134,7 +134,7 @@ void periodic_expand_entry(const PeriodicPlain &p, size_t index, Plaintext &out)
     r.scale = p.scale;
     r.ntt = true;
     r.data.reset(&c, p.limbs * c.n);
-    periodic_expand(c.tables, r.data.get(), p.table.get() + index * p.limbs * p.blocks, (uint32_t)p.limbs,
+    periodic_expand(c.tables, r.data.get(), p.table.get(), (uint32_t)index, (uint32_t)p.count, (uint32_t)p.limbs,
                     (uint32_t)p.blocks, c.stream);
     out = std::move(r);
 }
@@ -201,15 +201,16 @@ void op_periodic_mix(const std::vector<const Ciphertext *> &in, PeriodicPlain &w
                 }
             }
             h[M] = (int32_t)(runs.size() / 4);
-            const uint32_t nterms = (uint32_t)(runs.size() / 4);
             h.insert(h.end(), runs.begin(), runs.end());
             PeriodicPlain::Terms t;
+            t.plan = h.size();  // a multiple of four words
+            const std::vector<int32_t> plan = block_mix_plan(index, (uint32_t)K, (uint32_t)M);
+            h.insert(h.end(), plan.begin(), plan.end());
             t.words.reset(&c, (h.size() + 1) / 2);
             // stream-ordered: the buffer may come from work still queued on the stream
             NX_HIP(hipMemcpyAsync(t.words.get(), h.data(), h.size() * 4, hipMemcpyHostToDevice, c.stream));
             NX_HIP(hipStreamSynchronize(c.stream));
             t.M = (uint32_t)M;
-            t.nterms = nterms;
             it = w.terms.emplace(std::move(key), std::move(t)).first;
         }
         terms = &it->second;
@@ -230,7 +231,8 @@ void op_periodic_mix(const std::vector<const Ciphertext *> &in, PeriodicPlain &w
     }
     const uint32_t *first = reinterpret_cast<const uint32_t *>(terms->words.get());
     const int32_t *runs = reinterpret_cast<const int32_t *>(first + ((M + 1 + 3) & ~(size_t)3));
-    block_mix(c.tables, p, w.table.get(), runs, first, (uint32_t)K, (uint32_t)M, terms->nterms, (uint32_t)l,
+    const int32_t *plan = reinterpret_cast<const int32_t *>(first) + terms->plan;
+    block_mix(c.tables, p, w.table.get(), runs, first, plan, (uint32_t)K, (uint32_t)M, (uint32_t)l,
               (uint32_t)w.count, (uint32_t)w.blocks, c.stream);
     for (size_t m = 0; m < M; m++) *out[m] = std::move(res[m]);
 }
