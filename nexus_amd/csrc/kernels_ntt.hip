@@ -8,7 +8,8 @@
 // Outputs are fully reduced, so they are bit-identical to SEAL's however the
 // lazy reductions inside are scheduled.
 //
-// Mapping.  n <= 2^13: one workgroup holds a whole limb in LDS.  n >= 2^14: the
+// Mapping.  n <= 2^13: one workgroup holds a whole limb in LDS (a few limbs of
+// 2^13: two passes, see two_passes).  n >= 2^14: the
 // limb is viewed as an N1 x N2 matrix (index = t * N2 + c).  The first log2(N1)
 // forward stages only pair elements of the same column c (gap >= N2), the last
 // log2(N2) stages only pair elements of the same row t; the inverse runs rows
@@ -126,7 +127,7 @@ __device__ __forceinline__ void epi_store_f(const NttEpilogue &e, uint32_t p, ui
 //
 // Lazy reduction: see reduce_step and the inverse step (ntt_steps.h).  The
 // stored words are the fully reduced residues either way.
-template <int LOGS, int ROLE, bool FWD, int CW, bool R16>
+template <int LOGS, int ROLE, bool FWD, int CW, bool R16, int NT>
 __device__ __forceinline__ void ntt_tile_f(const NttKArgs &a, uint64_t *lds_words, uint64_t *data,
                                            const uint64_t *src, uint32_t prime, uint32_t n, uint32_t N2, uint32_t N1,
                                            uint32_t first, uint32_t poly, uint32_t limb)
@@ -167,7 +168,7 @@ __device__ __forceinline__ void ntt_tile_f(const NttKArgs &a, uint64_t *lds_word
         }
         __syncthreads();
     } else {
-        for (int e = threadIdx.x; e < G::TILE; e += kThreads) {
+        for (int e = threadIdx.x; e < G::TILE; e += NT) {
             uint64_t gidx;
             if (ROLE == kCol) {
                 const int k = e / G::C, cc = e % G::C;
@@ -181,13 +182,13 @@ __device__ __forceinline__ void ntt_tile_f(const NttKArgs &a, uint64_t *lds_word
         }
         __syncthreads();
         if (lazy)
-            stages_f<LOGS, ROLE, FWD, CW, true, kThreads, R16>(lds, tw, q, qinv, n, N1, first);
+            stages_f<LOGS, ROLE, FWD, CW, true, NT, R16>(lds, tw, q, qinv, n, N1, first);
         else
-            stages_f<LOGS, ROLE, FWD, CW, false, kThreads, R16>(lds, tw, q, qinv, n, N1, first);
+            stages_f<LOGS, ROLE, FWD, CW, false, NT, R16>(lds, tw, q, qinv, n, N1, first);
     }
     const bool scale_out = !FWD && ROLE != kRow;  // the inverse's last pass
     const double ni = a.ninvd[prime];
-    for (int e = threadIdx.x; e < G::TILE; e += kThreads) {
+    for (int e = threadIdx.x; e < G::TILE; e += NT) {
         uint64_t gidx;
         if (ROLE == kCol) {
             const int k = e / G::C, cc = e % G::C;
@@ -214,7 +215,7 @@ __device__ __forceinline__ void ntt_tile_f(const NttKArgs &a, uint64_t *lds_word
     }
 }
 
-template <int LOGS, int ROLE, bool FWD, int CW, bool R16>
+template <int LOGS, int ROLE, bool FWD, int CW, bool R16, int NT>
 __device__ __forceinline__ void ntt_pass(const NttKArgs &a)
 {
     using G = Geometry<LOGS, ROLE, CW>;
@@ -242,12 +243,12 @@ __device__ __forceinline__ void ntt_pass(const NttKArgs &a)
     if (ROLE == kCol && (gridDim.x & 7) == 0) tile = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
     const uint32_t first = tile * G::C;  // first column / row of the tile
     if (q < kFpPrimeBound) {
-        ntt_tile_f<LOGS, ROLE, FWD, CW, R16>(a, lds, data, src, prime, n, N2, N1, first, poly, limb);
+        ntt_tile_f<LOGS, ROLE, FWD, CW, R16, NT>(a, lds, data, src, prime, n, N2, N1, first, poly, limb);
         return;
     }
 
     // ---- load
-    for (int e = threadIdx.x; e < G::TILE; e += kThreads) {
+    for (int e = threadIdx.x; e < G::TILE; e += NT) {
         uint64_t gidx;
         if (ROLE == kCol) {
             const int k = e / G::C, cc = e % G::C;
@@ -267,16 +268,16 @@ __device__ __forceinline__ void ntt_pass(const NttKArgs &a)
         if constexpr (LOGS >= 3) {
 #pragma unroll
             for (int st = 0; st < LOGS / 3; st++) {
-                fwd_step<LOGS, ROLE, 3, CW>(lds, s, tw, q, m0, first);
+                fwd_step<LOGS, ROLE, 3, CW, NT>(lds, s, tw, q, m0, first);
                 s += 3;
                 __syncthreads();
             }
         }
         if constexpr (LOGS % 3 == 2) {
-            fwd_step<LOGS, ROLE, 2, CW>(lds, s, tw, q, m0, first);
+            fwd_step<LOGS, ROLE, 2, CW, NT>(lds, s, tw, q, m0, first);
             __syncthreads();
         } else if constexpr (LOGS % 3 == 1) {
-            fwd_step<LOGS, ROLE, 1, CW>(lds, s, tw, q, m0, first);
+            fwd_step<LOGS, ROLE, 1, CW, NT>(lds, s, tw, q, m0, first);
             __syncthreads();
         }
     } else {
@@ -285,16 +286,16 @@ __device__ __forceinline__ void ntt_pass(const NttKArgs &a)
         if constexpr (LOGS >= 3) {
 #pragma unroll
             for (int st = 0; st < LOGS / 3; st++) {
-                inv_step<LOGS, ROLE, 3, CW>(lds, s, tw, q, n, mx, first);
+                inv_step<LOGS, ROLE, 3, CW, NT>(lds, s, tw, q, n, mx, first);
                 s += 3;
                 __syncthreads();
             }
         }
         if constexpr (LOGS % 3 == 2) {
-            inv_step<LOGS, ROLE, 2, CW>(lds, s, tw, q, n, mx, first);
+            inv_step<LOGS, ROLE, 2, CW, NT>(lds, s, tw, q, n, mx, first);
             __syncthreads();
         } else if constexpr (LOGS % 3 == 1) {
-            inv_step<LOGS, ROLE, 1, CW>(lds, s, tw, q, n, mx, first);
+            inv_step<LOGS, ROLE, 1, CW, NT>(lds, s, tw, q, n, mx, first);
             __syncthreads();
         }
     }
@@ -303,7 +304,7 @@ __device__ __forceinline__ void ntt_pass(const NttKArgs &a)
     const bool last_pass = FWD ? (ROLE != kCol) : (ROLE != kRow);
     const bool epi = FWD && ROLE != kCol && epi_on(a.epi);
     const ulonglong2 ni = a.ninv[prime];
-    for (int e = threadIdx.x; e < G::TILE; e += kThreads) {
+    for (int e = threadIdx.x; e < G::TILE; e += NT) {
         uint64_t gidx;
         if (ROLE == kCol) {
             const int k = e / G::C, cc = e % G::C;
@@ -329,10 +330,10 @@ __device__ __forceinline__ void ntt_pass(const NttKArgs &a)
     }
 }
 
-template <int LOGS, int ROLE, bool FWD, int CW, bool R16>
-__global__ __launch_bounds__(kThreads) void k_ntt(NttKArgs a)
+template <int LOGS, int ROLE, bool FWD, int CW, bool R16, int NT>
+__global__ __launch_bounds__(NT) void k_ntt(NttKArgs a)
 {
-    ntt_pass<LOGS, ROLE, FWD, CW, R16>(a);
+    ntt_pass<LOGS, ROLE, FWD, CW, R16, NT>(a);
 }
 
 // ---- ModUp base conversion fused into the forward column pass
@@ -591,7 +592,7 @@ __global__ __launch_bounds__(kThreads, A <= 9 ? 2 : 1) void k_moddown_col(ModDow
 template <int LOGS, int ROLE, bool FWD, int CW, bool R16>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_ntt_w8(NttKArgs a)
 {
-    ntt_pass<LOGS, ROLE, FWD, CW, R16>(a);
+    ntt_pass<LOGS, ROLE, FWD, CW, R16, kThreads>(a);
 }
 
 template <int LOGS, int ROLE, bool FWD, int CW = 16, bool R16 = false>
@@ -614,10 +615,14 @@ void launch_one(const NttKArgs &a, uint32_t batch, hipStream_t s)
     const double epi_bytes = epi ? 8.0 * n * (1.0 + epi_reads) : 0.0;
     ProfScope prof(epi ? "ntt_fwd_sub_mul" : names[FWD ? 1 : 0][ROLE], s,
                    (double)(batch - a.skipped) * (16.0 * n + a.tw_bytes * tw + epi_bytes));
+    // a whole limb of 2^13 words leaves room for two workgroups on a CU: one
+    // radix-8 group a thread fills it (177 limbs of 60 bits: 22.4 us, with 512
+    // threads 26.3; 256 threads took 40 us for any number up to 256)
+    constexpr int NT = ROLE != kWhole || LOGS < 12 ? kThreads : (LOGS == 12 ? 512 : 1024);
     if constexpr (ROLE == kCol && FWD && CW == 8 && !R16)
         hipLaunchKernelGGL((k_ntt_w8<LOGS, ROLE, FWD, CW, R16>), grid, dim3(kThreads), 0, s, a);
     else
-        hipLaunchKernelGGL((k_ntt<LOGS, ROLE, FWD, CW, R16>), grid, dim3(kThreads), 0, s, a);
+        hipLaunchKernelGGL((k_ntt<LOGS, ROLE, FWD, CW, R16, NT>), grid, dim3(NT), 0, s, a);
 }
 
 template <bool FWD>
@@ -682,6 +687,7 @@ template <int ROLE, bool FWD>
 void launch_pass(int logs, const NttKArgs &a, uint32_t batch, hipStream_t s)
 {
     switch (logs) {
+    case 6: launch_one<6, ROLE, FWD, 8>(a, batch, s); break;
     case 7: launch_sized<7, ROLE, FWD>(a, batch, s); break;
     case 8: launch_sized<8, ROLE, FWD>(a, batch, s); break;
     case 9: launch_sized<9, ROLE, FWD>(a, batch, s); break;
@@ -780,12 +786,20 @@ int ntt_get_tile(int logn, int pass, bool fwd, uint32_t batch)
     return g_tile[li][pass][fwd ? 1 : 0][tune_bucket(batch)].load();
 }
 
+// Rings of 2^14 and above always run in two passes.  A limb of 2^13 words held
+// by one workgroup takes its time on one CU however few limbs there are (60-bit
+// primes: 17 us, 46-bit: 12.5 us for 3 to 48 limbs); cut into passes of 64 x 128
+// it takes 11.6 and 9.6 us.  The two cross between 48 limbs (17.9 / 14.2 us and
+// 13.3 / 11.9 us) and 96 (18.7 / 17.6, 13.8 / 15.4).  At 2^12 one workgroup is
+// never behind (10.3 us against 10.1 for 3 limbs, 11.2 against 12.4 for 96).
+static bool two_passes(int logn, uint32_t batch) { return logn >= 14 || (logn == 13 && batch <= 64); }
+
 void ntt_forward(const DeviceTables &t, const NttBatch &b, hipStream_t s)
 {
     const uint32_t batch = b.polys * b.limbs;
     if (!batch) return;
     NttKArgs a = make_args(t, b, true);
-    if (t.logn <= 13) {
+    if (!two_passes(t.logn, batch)) {
         launch_whole<true>(a, batch, s);
     } else {
         int l1, l2;
@@ -979,7 +993,7 @@ void ntt_inverse(const DeviceTables &t, const NttBatch &b, hipStream_t s)
     const uint32_t batch = b.polys * b.limbs;
     if (!batch) return;
     NttKArgs a = make_args(t, b, false);
-    if (t.logn <= 13) {
+    if (!two_passes(t.logn, batch)) {
         launch_whole<false>(a, batch, s);
     } else {
         int l1, l2;

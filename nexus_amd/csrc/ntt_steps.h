@@ -35,7 +35,7 @@ __device__ __forceinline__ int lds_addr(int cc, int pos)
 }
 
 // Forward radix-2^K step over local stages s .. s+K-1.
-template <int LOGS, int ROLE, int K, int CW>
+template <int LOGS, int ROLE, int K, int CW, int NT = kThreads>
 __device__ __forceinline__ void fwd_step(uint64_t *lds, int s, const ulonglong2 *tw, uint64_t q, uint32_t m0,
                                          uint32_t row0)
 {
@@ -46,7 +46,7 @@ __device__ __forceinline__ void fwd_step(uint64_t *lds, int s, const ulonglong2 
     const uint64_t two_q = 2 * q;
     const int B = G::S >> s;
     const int D = B >> K;
-    for (int g = threadIdx.x; g < GROUPS; g += kThreads) {
+    for (int g = threadIdx.x; g < GROUPS; g += NT) {
         int cc, gg;
         if (ROLE == kCol) {
             cc = g % G::C;
@@ -89,7 +89,7 @@ __device__ __forceinline__ void fwd_step(uint64_t *lds, int s, const ulonglong2 
 }
 
 // Inverse radix-2^K step over local stages s .. s+K-1 (gaps 2^s .. 2^(s+K-1)).
-template <int LOGS, int ROLE, int K, int CW>
+template <int LOGS, int ROLE, int K, int CW, int NT = kThreads>
 __device__ __forceinline__ void inv_step(uint64_t *lds, int s, const ulonglong2 *tw, uint64_t q, uint32_t n,
                                          uint32_t mx, uint32_t row0)
 {
@@ -99,7 +99,7 @@ __device__ __forceinline__ void inv_step(uint64_t *lds, int s, const ulonglong2 
     constexpr int GROUPS = G::TILE / R;
     const uint64_t two_q = 2 * q;
     const int so = 1 << s;
-    for (int g = threadIdx.x; g < GROUPS; g += kThreads) {
+    for (int g = threadIdx.x; g < GROUPS; g += NT) {
         int cc, gg;
         if (ROLE == kCol) {
             cc = g % G::C;
