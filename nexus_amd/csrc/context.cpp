@@ -539,11 +539,14 @@ void ntt_fwd(Context &c, uint64_t *data, size_t polys, size_t limbs, size_t poly
 }
 
 void ntt_fwd_epi(Context &c, uint64_t *data, size_t polys, size_t limbs, size_t poly_stride, const NttEpilogue &epi,
-                 bool rows_only)
+                 const FwdInput &in)
 {
     NttBatch b = make_batch(data, polys, limbs, poly_stride);
     b.epi = epi;
-    b.rows_only = rows_only ? 1 : 0;
+    b.rows_only = in.rows_only ? 1 : 0;
+    b.center = in.center;
+    b.center_stride = in.center_stride;
+    b.center_prime = in.center_prime;
     ntt_forward(c.tables, b, c.stream);
 }
 

@@ -248,10 +248,18 @@ private:
 // ---------------------------------------------------------------- operations
 // NTT of a [polys][limbs][n] buffer whose limb i uses prime i.
 void ntt_fwd(Context &c, uint64_t *data, size_t polys, size_t limbs, size_t poly_stride);
+// What ntt_fwd_epi finds in data: the limbs; limbs whose column pass has already
+// run (rows_only, after a fused conversion); or nothing yet, every limb being
+// the centred residues of a limb of another prime (NttBatch::center)
+struct FwdInput {
+    bool rows_only = false;
+    const uint64_t *center = nullptr;
+    uint64_t center_stride = 0;
+    uint32_t center_prime = 0;
+};
 // forward NTT whose last pass stores through epi instead of into data
-// rows_only: the column pass has already run on data (a fused conversion)
 void ntt_fwd_epi(Context &c, uint64_t *data, size_t polys, size_t limbs, size_t poly_stride, const NttEpilogue &epi,
-                 bool rows_only = false);
+                 const FwdInput &in);
 void ntt_inv(Context &c, uint64_t *data, size_t polys, size_t limbs, size_t poly_stride);
 // out of place: src (poly stride src_stride) -> dst (poly stride dst_stride)
 void ntt_fwd_from(Context &c, uint64_t *dst, const uint64_t *src, size_t polys, size_t limbs, size_t dst_stride,
@@ -356,15 +364,11 @@ void ks_inner(Context &c, uint64_t *acc, const uint64_t *targets, const uint64_t
 // acc[B][2][l+alpha][n]: the same with one key, on any ring
 void ks_inner_one_key(Context &c, uint64_t *acc, const uint64_t *targets, size_t B, size_t l, const DevBuf &key,
                       const uint64_t *aseed);
-// ModDown up to the final combination: INTT of the special limbs of acc
-// [B][2][l+alpha][n], conversion, NTT; returns tmp [B][2][l][n] for
-// out = (acc - tmp) P^-1.
-// col_done non-null: the conversion may run fused into the forward column
-// pass, and *col_done says whether it did (the caller's forward NTT of the
-// result then runs its row pass only).  transform: the whole forward NTT runs
-// here.
-DevBuf ks_moddown_prepare(Context &c, uint64_t *acc, size_t B, size_t l, bool transform = true,
-                          bool *col_done = nullptr);
+// ModDown up to the forward transform: INTT of the special limbs of acc
+// [B][2][l+alpha][n] in place and the conversion, as far as it is not part of
+// the transform; returns tmp [B][2][l][n], and in `in` what the caller's forward
+// NTT of it (ntt_fwd_epi, for out = (acc - NTT(tmp)) P^-1) starts from.
+DevBuf ks_moddown_prepare(Context &c, uint64_t *acc, size_t B, size_t l, FwdInput &in);
 // base (optional, [B][2][l][n]): the accumulated terms are read from base instead of cts.
 void ks_moddown(Context &c, uint64_t *cts, uint64_t *acc, size_t B, size_t l, bool zero_c1,
                 const uint64_t *base = nullptr);

@@ -91,6 +91,16 @@ struct NttBatch {
     // forward, n >= 2^14: the column pass has already run (ks_modup_convert_col);
     // only the row pass is launched
     uint32_t rows_only = 0;
+    // Forward, instead of words below each limb's prime:
+    //  lift: limb j of poly p is lift[(p / poly_period) limbs + j] (limbs of n
+    //        words of any primes), taken mod the limb's prime;
+    //  center: every limb i of poly p is SEAL's centred residue of one limb of
+    //        prime p_c = center_prime at center + p * center_stride,
+    //        ((x + p_c/2) mod p_c) - p_c/2 mod the limb's prime.
+    const uint64_t *lift = nullptr;
+    const uint64_t *center = nullptr;
+    uint64_t center_stride = 0;
+    uint32_t center_prime = 0;
 };
 constexpr int kNttSrcMax = 32;
 constexpr int kMaxHoist = 32;  // rotations of one hoisted inner product
@@ -175,22 +185,14 @@ void poly_add_scalar(const DeviceTables &t, uint64_t *out, const uint64_t *a, co
 // Rescale / ModDown tail, SEAL-exact rounding.
 //  last: coefficient-domain limb (already INTT'd) of prime `last_prime`, one per poly
 //  out[p][i] = (x[p][i] - NTT_i(centered(last[p]) mod q_i)) * inv[i]   for i < limbs
-// This writes the centred residues mod q_i into tmp[p][i]; the caller's forward
-// NTT of tmp combines them with x through an NttEpilogue.
-void rns_center_last(const DeviceTables &t, uint64_t *tmp, const uint64_t *last, uint64_t last_stride,
-                     uint32_t last_prime, uint32_t polys, uint32_t limbs, hipStream_t s);
-// rns_center_last fused into the forward NTT's column pass: tmp[p][i] holds the
-// column-transformed centred residues; the caller's forward NTT runs its row
-// pass only (NttBatch::rows_only).  Needs center_col_ok: every prime below
-// 2^51, 2^14 <= n <= 2^17.
+// The centring is the forward NTT's load (NttBatch::center) and the combination
+// its store (NttEpilogue).  Where every prime is below 2^51 and
+// 2^14 <= n <= 2^17 (center_col_ok), one read of the last limb serves several
+// limbs: tmp[p][i] receives the column-transformed centred residues, and the
+// caller's forward NTT runs its row pass only (NttBatch::rows_only).
 bool center_col_ok(const DeviceTables &t);
 void rns_center_last_col(const DeviceTables &t, uint64_t *tmp, const uint64_t *last, uint64_t last_stride,
                          uint32_t last_prime, uint32_t polys, uint32_t limbs, hipStream_t s);
-// Key-switch ModUp over a batch of B targets: for ciphertext b, every output
-// prime I in out_primes (count = nout) and digit j < l,
-// T[b][I][j] = coef[b][j] mod q_I  (coef = INTT of the target, [B][l][n]).
-void ks_modup_expand(const DeviceTables &t, uint64_t *T, const uint64_t *coef, uint32_t B, uint32_t l,
-                     const uint8_t *out_primes_host, uint32_t nout, hipStream_t s);
 // Inner product: acc[b][k][I][c] = sum_j T[b][I][j][c] * key[j][k][kp(I)][c] mod q_kp(I)
 // key layout [digits][2][key_limbs][n], shared by the batch.
 // aseed (device array, one seed per digit) non-null: poly 1 of every key digit

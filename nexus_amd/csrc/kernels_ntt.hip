@@ -62,6 +62,9 @@ struct NttKArgs {
     uint32_t skip_l, skip_alpha, skipped;  // NttBatch::skip_*; skipped: limbs left out
     NttEpilogue epi;                        // applied by the forward transform's last pass
     uint32_t epi_int;                       // double-precision path: the epilogue in 64-bit integers
+    const uint64_t *in;                     // NttBatch::lift / center (LOAD kLift / kCenter): the words read,
+    uint64_t in_stride;                     // words from a poly's to the next one's (kCenter),
+    uint32_t in_prime;                      // and their prime (kCenter)
     uint8_t prime_of[kMaxPrimes];
 };
 
@@ -122,12 +125,33 @@ __device__ __forceinline__ void epi_store_f(const NttEpilogue &e, uint32_t p, ui
     *o = fp_to(r < 0 ? r + q : r);
 }
 
+// What the first pass of a forward transform reads (NttBatch::lift, center).
+// Taking the words mod the limb's prime here saves the key switch and the
+// rescale a pass that only wrote them out for this one to read back: bound by
+// memory traffic on large rings (16 degree-7 products at N = 2^16 with 60-bit
+// primes: 14.3 to 13.4 ms), by launches on small ones (multiply, relinearise and
+// rescale at 2^13: 83 to 75 us).
+enum Load { kPlain = 0, kLift = 1, kCenter = 2 };
+
+template <int LOAD>
+__device__ __forceinline__ uint64_t load_word(uint64_t v, const NttKArgs &a, const ModConst &m)
+{
+    if constexpr (LOAD == kLift) return v >= m.q ? barrett64(v, m) : v;
+    if constexpr (LOAD == kCenter) {
+        const uint64_t p = a.mod[a.in_prime].q, half = p >> 1;
+        v += half;
+        v = v >= p ? v - p : v;  // (x + (p - 1) / 2) mod p
+        return sub_mod(barrett64(v, m), barrett64(half, m), m.q);
+    }
+    return v;
+}
+
 // The whole transform body of one tile in double precision: load (reduced),
 // the radix steps, store in [0, q) (times n^-1 on the inverse's last pass).
 //
 // Lazy reduction: see reduce_step and the inverse step (ntt_steps.h).  The
 // stored words are the fully reduced residues either way.
-template <int LOGS, int ROLE, bool FWD, int CW, bool R16, int NT>
+template <int LOGS, int ROLE, bool FWD, int CW, bool R16, int NT, int LOAD>
 __device__ __forceinline__ void ntt_tile_f(const NttKArgs &a, uint64_t *lds_words, uint64_t *data,
                                            const uint64_t *src, uint32_t prime, uint32_t n, uint32_t N2, uint32_t N1,
                                            uint32_t first, uint32_t poly, uint32_t limb)
@@ -178,7 +202,10 @@ __device__ __forceinline__ void ntt_tile_f(const NttKArgs &a, uint64_t *lds_word
             } else {
                 gidx = e;
             }
-            lds[e] = reduce_f(fp_from(src[gidx]), q, qinv);
+            if constexpr (LOAD == kPlain)
+                lds[e] = reduce_f(fp_from(src[gidx]), q, qinv);
+            else
+                lds[e] = reduce_f(fp_from(load_word<LOAD>(src[gidx], a, a.mod[prime])), q, qinv);
         }
         __syncthreads();
         if (lazy)
@@ -215,7 +242,7 @@ __device__ __forceinline__ void ntt_tile_f(const NttKArgs &a, uint64_t *lds_word
     }
 }
 
-template <int LOGS, int ROLE, bool FWD, int CW, bool R16, int NT>
+template <int LOGS, int ROLE, bool FWD, int CW, bool R16, int NT, int LOAD>
 __device__ __forceinline__ void ntt_pass(const NttKArgs &a)
 {
     using G = Geometry<LOGS, ROLE, CW>;
@@ -232,6 +259,8 @@ __device__ __forceinline__ void ntt_pass(const NttKArgs &a)
     uint64_t *data = a.data + poly * a.poly_stride + (uint64_t)limb * n;
     const uint64_t *src = a.nsrcs ? a.srcs[poly] + (uint64_t)limb * n
                                   : (a.src ? a.src + poly * a.src_poly_stride + (uint64_t)limb * n : data);
+    if (LOAD == kLift) src = a.in + ((uint64_t)(poly / a.poly_period) * a.limbs + limb) * n;
+    if (LOAD == kCenter) src = a.in + poly * a.in_stride;
     const ulonglong2 *tw = a.tw + (uint64_t)prime * n;
     const uint64_t q = a.mod[prime].q;
     const uint32_t N2 = ROLE == kCol ? (n >> LOGS) : (ROLE == kRow ? (uint32_t)G::S : n);
@@ -243,7 +272,7 @@ __device__ __forceinline__ void ntt_pass(const NttKArgs &a)
     if (ROLE == kCol && (gridDim.x & 7) == 0) tile = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
     const uint32_t first = tile * G::C;  // first column / row of the tile
     if (q < kFpPrimeBound) {
-        ntt_tile_f<LOGS, ROLE, FWD, CW, R16, NT>(a, lds, data, src, prime, n, N2, N1, first, poly, limb);
+        ntt_tile_f<LOGS, ROLE, FWD, CW, R16, NT, LOAD>(a, lds, data, src, prime, n, N2, N1, first, poly, limb);
         return;
     }
 
@@ -258,7 +287,7 @@ __device__ __forceinline__ void ntt_pass(const NttKArgs &a)
         } else {
             gidx = e;
         }
-        lds[e] = src[gidx];
+        lds[e] = LOAD == kPlain ? src[gidx] : load_word<LOAD>(src[gidx], a, a.mod[prime]);
     }
     __syncthreads();
 
@@ -330,10 +359,10 @@ __device__ __forceinline__ void ntt_pass(const NttKArgs &a)
     }
 }
 
-template <int LOGS, int ROLE, bool FWD, int CW, bool R16, int NT>
+template <int LOGS, int ROLE, bool FWD, int CW, bool R16, int NT, int LOAD>
 __global__ __launch_bounds__(NT) void k_ntt(NttKArgs a)
 {
-    ntt_pass<LOGS, ROLE, FWD, CW, R16, NT>(a);
+    ntt_pass<LOGS, ROLE, FWD, CW, R16, NT, LOAD>(a);
 }
 
 // ---- ModUp base conversion fused into the forward column pass
@@ -592,10 +621,10 @@ __global__ __launch_bounds__(kThreads, A <= 9 ? 2 : 1) void k_moddown_col(ModDow
 template <int LOGS, int ROLE, bool FWD, int CW, bool R16>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_ntt_w8(NttKArgs a)
 {
-    ntt_pass<LOGS, ROLE, FWD, CW, R16, kThreads>(a);
+    ntt_pass<LOGS, ROLE, FWD, CW, R16, kThreads, kPlain>(a);
 }
 
-template <int LOGS, int ROLE, bool FWD, int CW = 16, bool R16 = false>
+template <int LOGS, int ROLE, bool FWD, int CW = 16, bool R16 = false, int LOAD = kPlain>
 void launch_one(const NttKArgs &a, uint32_t batch, hipStream_t s)
 {
     using G = Geometry<LOGS, ROLE, CW>;
@@ -619,18 +648,18 @@ void launch_one(const NttKArgs &a, uint32_t batch, hipStream_t s)
     // radix-8 group a thread fills it (177 limbs of 60 bits: 22.4 us, with 512
     // threads 26.3; 256 threads took 40 us for any number up to 256)
     constexpr int NT = ROLE != kWhole || LOGS < 12 ? kThreads : (LOGS == 12 ? 512 : 1024);
-    if constexpr (ROLE == kCol && FWD && CW == 8 && !R16)
+    if constexpr (ROLE == kCol && FWD && CW == 8 && !R16 && LOAD == kPlain)
         hipLaunchKernelGGL((k_ntt_w8<LOGS, ROLE, FWD, CW, R16>), grid, dim3(kThreads), 0, s, a);
     else
-        hipLaunchKernelGGL((k_ntt<LOGS, ROLE, FWD, CW, R16, NT>), grid, dim3(NT), 0, s, a);
+        hipLaunchKernelGGL((k_ntt<LOGS, ROLE, FWD, CW, R16, NT, LOAD>), grid, dim3(NT), 0, s, a);
 }
 
-template <bool FWD>
+template <bool FWD, int LOAD = kPlain>
 void launch_whole(const NttKArgs &a, uint32_t batch, hipStream_t s)
 {
     switch (a.logn) {
 #define NX_CASE(L) \
-    case L: launch_one<L, kWhole, FWD>(a, batch, s); break;
+    case L: launch_one<L, kWhole, FWD, 16, false, LOAD>(a, batch, s); break;
         NX_CASE(1) NX_CASE(2) NX_CASE(3) NX_CASE(4) NX_CASE(5) NX_CASE(6) NX_CASE(7)
         NX_CASE(8) NX_CASE(9) NX_CASE(10) NX_CASE(11) NX_CASE(12) NX_CASE(13)
 #undef NX_CASE
@@ -695,6 +724,19 @@ void launch_pass(int logs, const NttKArgs &a, uint32_t batch, hipStream_t s)
     }
 }
 
+// The first pass of a forward transform with a load of its own: tiles of 8, radix 8
+// (the words do not depend on either).
+template <int LOAD>
+void launch_load_col(int logs, const NttKArgs &a, uint32_t batch, hipStream_t s)
+{
+    switch (logs) {
+    case 6: launch_one<6, kCol, true, 8, false, LOAD>(a, batch, s); break;
+    case 7: launch_one<7, kCol, true, 8, false, LOAD>(a, batch, s); break;
+    case 8: launch_one<8, kCol, true, 8, false, LOAD>(a, batch, s); break;
+    default: break;
+    }
+}
+
 NttKArgs make_args(const DeviceTables &t, const NttBatch &b, bool fwd)
 {
     NttKArgs a;
@@ -720,6 +762,9 @@ NttKArgs make_args(const DeviceTables &t, const NttBatch &b, bool fwd)
     }
     a.epi = b.epi;
     a.epi_int = (uint32_t)g_epi_int.load();
+    a.in = nullptr;
+    a.in_stride = 0;
+    a.in_prime = 0;
     if (!fwd) {
         a.epi.out = nullptr;
         a.epi.outs[0] = nullptr;
@@ -799,12 +844,30 @@ void ntt_forward(const DeviceTables &t, const NttBatch &b, hipStream_t s)
     const uint32_t batch = b.polys * b.limbs;
     if (!batch) return;
     NttKArgs a = make_args(t, b, true);
+    const int load = b.lift ? kLift : b.center ? kCenter : kPlain;
+    if (load == kLift && (!b.prime_by_poly || !b.poly_period || b.polys % b.poly_period))
+        throw std::invalid_argument("ntt: a lift needs a prime per poly of a period");
+    if (load != kPlain && (b.rows_only || b.src || b.src_list || b.skip_alpha))
+        throw std::invalid_argument("ntt: a lift or centring is the only source of a whole transform");
+    a.in = b.lift ? b.lift : b.center;
+    a.in_stride = b.center_stride;
+    a.in_prime = b.center_prime;
     if (!two_passes(t.logn, batch)) {
-        launch_whole<true>(a, batch, s);
+        if (load == kLift)
+            launch_whole<true, kLift>(a, batch, s);
+        else if (load == kCenter)
+            launch_whole<true, kCenter>(a, batch, s);
+        else
+            launch_whole<true>(a, batch, s);
     } else {
         int l1, l2;
         split_logn(t.logn, l1, l2);
-        if (!b.rows_only) launch_pass<kCol, true>(l1, a, batch, s);
+        if (load == kLift)
+            launch_load_col<kLift>(l1, a, batch, s);
+        else if (load == kCenter)
+            launch_load_col<kCenter>(l1, a, batch, s);
+        else if (!b.rows_only)
+            launch_pass<kCol, true>(l1, a, batch, s);
         a.src = nullptr;  // the second pass runs in place on the output
         a.nsrcs = 0;
         launch_pass<kRow, true>(l2, a, batch, s);

@@ -260,37 +260,7 @@ __global__ void k_add_scalar(uint64_t *out, const uint64_t *a, LimbWords v, cons
     out[idx] = add_mod(a[idx], v.v[limb], mod[limb].q);
 }
 
-// ---- rescale / ModDown
-__global__ void k_center_last(uint64_t *tmp, const uint64_t *last, uint64_t last_stride, const ModConst *mod,
-                              uint32_t last_prime, uint32_t limbs, uint32_t n)
-{
-    const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
-    if (c >= n) return;
-    const uint32_t row = blockIdx.y;
-    const uint32_t poly = row / limbs, limb = row - poly * limbs;
-    const uint64_t p = mod[last_prime].q;
-    const uint64_t half = p >> 1;
-    uint64_t v = last[poly * last_stride + c] + half;
-    v = v >= p ? v - p : v;  // [0, p): (x + (p-1)/2) mod p
-    const ModConst mi = mod[limb];
-    const uint64_t r = sub_mod(barrett64(v, mi), barrett64(half, mi), mi.q);
-    tmp[(uint64_t)row * n + c] = r;
-}
-
 // ---- key switching
-__global__ void k_modup_expand(uint64_t *T, const uint64_t *coef, const ModConst *mod, PrimeMap outp, uint32_t l,
-                               uint32_t nout, uint32_t n)
-{
-    const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
-    if (c >= n) return;
-    const uint32_t row = blockIdx.y;  // (b * nout + I) * l + j
-    const uint32_t bi = row / l, j = row - bi * l;
-    const uint32_t b = bi / nout, I = bi - b * nout;
-    const ModConst m = mod[outp.p[I]];
-    const uint64_t v = coef[((uint64_t)b * l + j) * n + c];
-    T[(uint64_t)row * n + c] = v >= m.q ? barrett64(v, m) : v;
-}
-
 // aseed non-null: poly 1 of key digit j (uniform) is ctr_uniform(aseed[j], kp n + c, q_kp), regenerated
 // instead of read
 // qd non-null (every prime below 2^51): exact double-precision products (fp_mulmod); same words
@@ -552,21 +522,6 @@ void poly_add_scalar(const DeviceTables &t, uint64_t *out, const uint64_t *a, co
     LimbWords v;
     for (uint32_t i = 0; i < kMaxPrimes; i++) v.v[i] = i < limbs ? host_v[i] : 0;
     hipLaunchKernelGGL(k_add_scalar, grid_for(t.logn, limbs), dim3(kBlock), 0, s, out, a, v, t.mod, 1u << t.logn);
-}
-
-void rns_center_last(const DeviceTables &t, uint64_t *tmp, const uint64_t *last, uint64_t last_stride,
-                     uint32_t last_prime, uint32_t polys, uint32_t limbs, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_center_last, grid_for(t.logn, polys * limbs), dim3(kBlock), 0, s, tmp, last, last_stride,
-                       t.mod, last_prime, limbs, 1u << t.logn);
-}
-
-void ks_modup_expand(const DeviceTables &t, uint64_t *T, const uint64_t *coef, uint32_t B, uint32_t l,
-                     const uint8_t *out_primes_host, uint32_t nout, hipStream_t s)
-{
-    ProfScope prof("ks_modup", s, 8.0 * (1u << t.logn) * B * ((double)l + (double)nout * l));
-    hipLaunchKernelGGL(k_modup_expand, grid_for(t.logn, B * nout * l), dim3(kBlock), 0, s, T, coef, t.mod,
-                       make_map(out_primes_host, nout), l, nout, 1u << t.logn);
 }
 
 void ks_inner_product(const DeviceTables &t, uint64_t *acc, const uint64_t *T, const uint64_t *key, uint32_t B,

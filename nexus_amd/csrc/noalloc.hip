@@ -73,14 +73,17 @@ void rescale_noalloc(Context &c, const uint64_t *in, size_t polys, size_t limbs,
     b.src = in + (l - 1) * n;
     b.src_poly_stride = l * n;
     ntt_inverse(c.tables, b, c.stream);
-    rns_center_last(c.tables, tmp, last, n, (uint32_t)(l - 1), (uint32_t)P, (uint32_t)(l - 1), c.stream);
     NttEpilogue e;
     e.out = out;
     e.out_stride = (l - 1) * n;
     e.x = in;
     e.x_stride = l * n;
     e.inv = c.rescale_inv(l);
-    ntt_fwd_epi(c, tmp, P, l - 1, (l - 1) * n, e);
+    FwdInput center;
+    center.center = last;
+    center.center_stride = n;
+    center.center_prime = (uint32_t)(l - 1);
+    ntt_fwd_epi(c, tmp, P, l - 1, (l - 1) * n, e, center);
 }
 
 }  // namespace nx

@@ -319,15 +319,15 @@ static DevBuf ks_modup_impl(Context &c, const uint64_t *targets, const uint64_t 
         ntt_forward(c.tables, b, c.stream);
         return T;
     }
+    NttBatch b;
     if (c.alpha == 1)
-        ks_modup_expand(c.tables, T.get(), coef.get(), (uint32_t)B, (uint32_t)l, outp, (uint32_t)nout, c.stream);
+        b.lift = coef.get();  // T[b][I][j] = coef[b][j] mod q_I, taken as the transform loads it
     else if (ks_conv_fused_ok((uint32_t)c.alpha))
         ks_modup_convert_fused(c.tables, T.get(), coef.get(), c.d_modup_w, c.d_modup_conv, (uint32_t)B, (uint32_t)l,
                                (uint32_t)c.alpha, (uint32_t)c.key_limbs(), outp, (uint32_t)nout, c.stream);
     else
         ks_modup_convert(c.tables, T.get(), coef.get(), c.d_modup_w, c.d_modup_conv, (uint32_t)B, (uint32_t)l,
                          (uint32_t)c.alpha, (uint32_t)c.key_limbs(), outp, (uint32_t)nout, c.stream);
-    NttBatch b;
     if (c.alpha > 1) {
         // digit j on its own primes is its input: copied in NTT form, not transformed
         ks_modup_copy_own(c.tables, T.get(), targets, target_list, (uint32_t)B, (uint32_t)l, (uint32_t)c.alpha,
@@ -443,7 +443,7 @@ void key_switch_batch(Context &c, uint64_t *cts, const uint64_t *targets, size_t
     ks_moddown(c, cts, acc.get(), B, l, zero_c1, base);
 }
 
-DevBuf ks_moddown_prepare(Context &c, uint64_t *acc, size_t B, size_t l, bool transform, bool *col_done)
+DevBuf ks_moddown_prepare(Context &c, uint64_t *acc, size_t B, size_t l, FwdInput &in)
 {
     const size_t n = c.n, L = c.L, alpha = c.alpha;
     const size_t nout = l + alpha;
@@ -460,37 +460,34 @@ DevBuf ks_moddown_prepare(Context &c, uint64_t *acc, size_t B, size_t l, bool tr
         ntt_inverse(c.tables, b, c.stream);
     }
     DevBuf tmp(&c, B * 2 * l * n);
-    if (col_done) *col_done = false;
-    if (alpha > 1 && (col_done || transform) && c.d_moddown_conv_d && ks_moddown_col_ok(c.tables, (uint32_t)alpha) &&
+    if (alpha > 1 && c.d_moddown_conv_d && ks_moddown_col_ok(c.tables, (uint32_t)alpha) &&
         ks_moddown_col_get((uint32_t)(2 * B)) >= 0) {
         // the centred conversion feeds the forward column pass directly
         uint8_t inp[kMaxPrimes];
         for (size_t k = 0; k < alpha; k++) inp[k] = (uint8_t)(L + k);
         ks_moddown_convert_col(c.tables, tmp.get(), acc, nout * n, c.d_moddown_w, c.d_moddown_conv_d, inp,
                                (uint32_t)alpha, (uint32_t)(2 * B), (uint32_t)l, (uint32_t)L, c.stream);
-        if (transform) ntt_fwd_epi(c, tmp.get(), 2 * B, l, l * n, NttEpilogue(), true);
-        if (col_done) *col_done = !transform;
+        in.rows_only = true;
         return tmp;
     }
-    if (alpha == 1 && (col_done || transform) && center_col_ok(c.tables)) {
+    if (alpha == 1 && center_col_ok(c.tables)) {
         // SEAL's centring inside the forward column pass
         rns_center_last_col(c.tables, tmp.get(), acc + l * n, nout * n, (uint32_t)L, (uint32_t)(2 * B), (uint32_t)l,
                             c.stream);
-        if (transform) ntt_fwd_epi(c, tmp.get(), 2 * B, l, l * n, NttEpilogue(), true);
-        if (col_done) *col_done = !transform;
+        in.rows_only = true;
         return tmp;
     }
-    if (alpha == 1)  // SEAL: centred (rounded) division by p
-        rns_center_last(c.tables, tmp.get(), acc + l * n, nout * n, (uint32_t)L, (uint32_t)(2 * B), (uint32_t)l,
-                        c.stream);
-    else if (ks_conv_fused_ok((uint32_t)alpha))  // hybrid: centred conversion of the P part
+    if (alpha == 1) {  // SEAL: centred (rounded) division by p, centred as the transform loads it
+        in.center = acc + l * n;
+        in.center_stride = nout * n;
+        in.center_prime = (uint32_t)L;
+    } else if (ks_conv_fused_ok((uint32_t)alpha))  // hybrid: centred conversion of the P part
         ks_moddown_convert_fused(c.tables, tmp.get(), acc, nout * n, c.d_moddown_w, c.d_moddown_conv,
                                  c.d_moddown_conv_d, (uint32_t)(2 * B), (uint32_t)l, (uint32_t)alpha, (uint32_t)L,
                                  c.stream);
     else
         ks_moddown_convert(c.tables, tmp.get(), acc, nout * n, c.d_moddown_w, c.d_moddown_conv, (uint32_t)(2 * B),
                            (uint32_t)l, (uint32_t)alpha, (uint32_t)L, c.stream);
-    if (transform) ntt_fwd(c, tmp.get(), 2 * B, l, l * n);
     return tmp;
 }
 
@@ -499,8 +496,8 @@ void ks_moddown(Context &c, uint64_t *cts, uint64_t *acc, size_t B, size_t l, bo
     // cts = (acc - NTT(conversion)) P^-1 (+ base or cts): the combination is the
     // forward transform's last pass
     const size_t n = c.n, nout = l + c.alpha;
-    bool col_done = false;
-    DevBuf tmp = ks_moddown_prepare(c, acc, B, l, false, &col_done);
+    FwdInput in;
+    DevBuf tmp = ks_moddown_prepare(c, acc, B, l, in);
     NttEpilogue e;
     e.out = cts;
     e.out_stride = l * n;
@@ -510,7 +507,7 @@ void ks_moddown(Context &c, uint64_t *cts, uint64_t *acc, size_t B, size_t l, bo
     e.accumulate = zero_c1 ? 2 : 1;
     e.base = base;
     e.base_stride = l * n;
-    ntt_fwd_epi(c, tmp.get(), 2 * B, l, l * n, e, col_done);
+    ntt_fwd_epi(c, tmp.get(), 2 * B, l, l * n, e, in);
 }
 
 static void key_switch_impl(Context &c, Ciphertext &ct, const uint64_t *target, const DevBuf &key, bool zero_c1,
@@ -621,6 +618,23 @@ void op_conjugate(const Ciphertext &a, const KSwitchKeys &gk, Ciphertext &dst)
 }
 
 // ---------------------------------------------------------------- rescale & level
+// The centring of a rescale from l limbs: inside the forward column pass, one
+// read of `last` ([P][n]) for several limbs of z ([P][l-1][n]), or left to the
+// transform's load.
+static FwdInput rescale_center(Context &c, uint64_t *z, const uint64_t *last, size_t P, size_t l)
+{
+    FwdInput in;
+    if (center_col_ok(c.tables)) {
+        rns_center_last_col(c.tables, z, last, c.n, (uint32_t)(l - 1), (uint32_t)P, (uint32_t)(l - 1), c.stream);
+        in.rows_only = true;
+    } else {
+        in.center = last;
+        in.center_stride = c.n;
+        in.center_prime = (uint32_t)(l - 1);
+    }
+    return in;
+}
+
 void op_rescale_to_next(const Ciphertext &a, Ciphertext &dst)
 {
     // evaluator.cpp:1402-1481 + util/rns.cpp:830-905
@@ -645,13 +659,7 @@ void op_rescale_to_next(const Ciphertext &a, Ciphertext &dst)
         ntt_inverse(c.tables, b, c.stream);
     }
     DevBuf tmp(&c, P * (l - 1) * n);
-    const bool col = center_col_ok(c.tables);  // centring inside the forward column pass
-    if (col)
-        rns_center_last_col(c.tables, tmp.get(), last.get(), n, (uint32_t)(l - 1), (uint32_t)P, (uint32_t)(l - 1),
-                            c.stream);
-    else
-        rns_center_last(c.tables, tmp.get(), last.get(), n, (uint32_t)(l - 1), (uint32_t)P, (uint32_t)(l - 1),
-                        c.stream);
+    const FwdInput in_tmp = rescale_center(c, tmp.get(), last.get(), P, l);
     // out = (a - NTT(centred last limb)) q_(l-1)^-1, stored by the transform's last pass
     DevBuf out(&c, P * (l - 1) * n);
     NttEpilogue e;
@@ -660,7 +668,7 @@ void op_rescale_to_next(const Ciphertext &a, Ciphertext &dst)
     e.x = a.data.get();
     e.x_stride = l * n;
     e.inv = c.rescale_inv(l);
-    ntt_fwd_epi(c, tmp.get(), P, l - 1, (l - 1) * n, e, col);
+    ntt_fwd_epi(c, tmp.get(), P, l - 1, (l - 1) * n, e, in_tmp);
     const double scale = a.scale / (double)c.moduli[l - 1];
     Ciphertext r;
     r.ctx = &c;
@@ -697,13 +705,7 @@ static void rescale_batch(Context &c, const std::vector<const uint64_t *> &x, si
         ntt_inverse(c.tables, b, c.stream);
     }
     DevBuf tmp(&c, P * (l - 1) * n);
-    const bool col = center_col_ok(c.tables);  // centring inside the forward column pass
-    if (col)
-        rns_center_last_col(c.tables, tmp.get(), last.get(), n, (uint32_t)(l - 1), (uint32_t)P, (uint32_t)(l - 1),
-                            c.stream);
-    else
-        rns_center_last(c.tables, tmp.get(), last.get(), n, (uint32_t)(l - 1), (uint32_t)P, (uint32_t)(l - 1),
-                        c.stream);
+    const FwdInput in_tmp = rescale_center(c, tmp.get(), last.get(), P, l);
     NttEpilogue e;  // outs[r] = (x[r] - NTT(centred last limbs)) q_(l-1)^-1
     for (size_t r = 0; r < B; r++) {
         e.outs[r] = outs[r];
@@ -712,7 +714,7 @@ static void rescale_batch(Context &c, const std::vector<const uint64_t *> &x, si
     e.x_limbs = (uint32_t)l;
     e.polys_per = (uint32_t)polys;
     e.inv = c.rescale_inv(l);
-    ntt_fwd_epi(c, tmp.get(), P, l - 1, (l - 1) * n, e, col);
+    ntt_fwd_epi(c, tmp.get(), P, l - 1, (l - 1) * n, e, in_tmp);
 }
 
 void op_rescale_many(const std::vector<const Ciphertext *> &in, const std::vector<Ciphertext *> &out)
@@ -864,7 +866,7 @@ void op_multiply_relin_rescale_fused_many(const std::vector<const Ciphertext *> 
             ntt_inverse(c.tables, nb, c.stream);
         }
         DevBuf tmp(&c, cnt * 2 * lo * n);  // conversion, then the transform's first pass
-        bool col_done = false;
+        FwdInput in_tmp;
         if (ks_moddown_col_ok(c.tables, (uint32_t)A) && ks_moddown_col_get((uint32_t)(2 * cnt)) >= 0) {
             // the conversion feeds the forward column pass directly
             uint8_t inp[kMaxPrimes];
@@ -872,7 +874,7 @@ void op_multiply_relin_rescale_fused_many(const std::vector<const Ciphertext *> 
             ks_moddown_convert_col(c.tables, tmp.get(), acc.get(), nout * n, c.d_mdr_w + l * A,
                                    c.d_mdr_conv_d + l * (A + 1) * c.L, inp, (uint32_t)A, (uint32_t)(2 * cnt),
                                    (uint32_t)lo, (uint32_t)c.L, c.stream);
-            col_done = true;
+            in_tmp.rows_only = true;
         } else {
             ks_moddown_rescale_convert(c.tables, tmp.get(), acc.get(), nout * n, c.d_mdr_w + l * A,
                                        c.d_mdr_conv + l * (A + 1) * c.L, c.d_mdr_conv_d + l * (A + 1) * c.L,
@@ -895,7 +897,7 @@ void op_multiply_relin_rescale_fused_many(const std::vector<const Ciphertext *> 
         e.d = c01.get();
         e.d_stride = pw;
         e.inv2 = c.rescale_inv(l);
-        ntt_fwd_epi(c, tmp.get(), 2 * cnt, lo, lo * n, e, col_done);
+        ntt_fwd_epi(c, tmp.get(), 2 * cnt, lo, lo * n, e, in_tmp);
     }
     for (size_t r = 0; r < a.size(); r++) *out[r] = std::move(res[r]);
 }
