@@ -384,13 +384,22 @@ void poly_mul_add(const DeviceTables &t, uint64_t *out, const uint64_t *a, const
 // out[c] += a[c] * w (mod q_prime) for one limb; w = {value, Shoup quotient}
 void limb_add_scaled(const DeviceTables &t, uint64_t *out, const uint64_t *a, ulonglong2 w, uint32_t prime,
                      hipStream_t s);
-// out[p][i] = a[p][i] * P[i] + b[p][i] * Q[i]  (NTT-domain, limb i uses prime i)
-void poly_mul2_add(const DeviceTables &t, uint64_t *out, const uint64_t *a, const uint64_t *P, const uint64_t *b,
-                   const uint64_t *Q, uint32_t polys, uint32_t limbs, hipStream_t s);
-// out[i][p][l] = sum_{j < inner} E[i * inner + j][p][l] * A[j][l]  for i < cols, p < 2
-// (E: [cols*inner][2][limbs][n] expanded ciphertexts, A: [inner][limbs][n] plaintexts)
-void mm_accumulate(const DeviceTables &t, uint64_t *out, const uint64_t *E, const uint64_t *A, uint32_t cols,
-                   uint32_t inner, uint32_t limbs, hipStream_t s);
+// Expansion round of the matrix product, NTT domain, limb i uses prime i:
+// sum = x + r, mix[p][i] = x[p][i] * P[i] + r[p][i] * Q[i]
+void mm_combine(const DeviceTables &t, uint64_t *sum, uint64_t *mix, const uint64_t *x, const uint64_t *P,
+                const uint64_t *r, const uint64_t *Q, uint32_t polys, uint32_t limbs, hipStream_t s);
+// count ciphertexts a [2][limbs][n], words c from perm[c]: poly 0 into cts (same layout), poly 1 into tgt
+// [count][limbs][n]
+void mm_permute(const DeviceTables &t, uint64_t *cts, uint64_t *tgt, const uint64_t *a, const uint32_t *perm,
+                uint32_t count, uint32_t limbs, hipStream_t s);
+// outs[i][p][l] = sum_{j < inner} e[i * inner + j][p][l] * A[j][l]  for i < cols, p < 2, where e counts through
+// the batches E[k] of counts[k] expanded ciphertexts [2][limbs][n] (A[j]: [limbs][n] plaintexts; host arrays)
+constexpr int kMmTerms = 256;   // plaintext pointers of one launch
+constexpr int kMmBatches = 48;  // batches of one launch
+constexpr int kMmCols = 64;     // result pointers of one launch
+void mm_accumulate(const DeviceTables &t, uint64_t *const *outs, const uint64_t *const *E, const size_t *counts,
+                   uint32_t batches, const uint64_t *const *A, uint32_t cols, uint32_t inner, uint32_t limbs,
+                   hipStream_t s);
 // ModRaise: in0 = coefficient-domain q0 limb of each poly ([polys][n]) -> out [polys][limbs][n]
 void mod_raise(const DeviceTables &t, uint64_t *out, const uint64_t *in0, uint32_t polys, uint32_t limbs,
                hipStream_t s);

@@ -624,70 +624,135 @@ namespace nx {
 
 namespace {
 
-__global__ void k_mul2_add(uint64_t *out, const uint64_t *a, const uint64_t *P, const uint64_t *b, const uint64_t *Q,
-                           const ModConst *mod, uint32_t limbs, uint32_t n)
+// One expansion round's end: x + r and x P + r Q from one read of x and r.
+__global__ void k_mm_combine(uint64_t *sum, uint64_t *mix, const uint64_t *x, const uint64_t *P, const uint64_t *r,
+                             const uint64_t *Q, const ModConst *mod, uint32_t limbs, uint32_t n)
 {
     const uint32_t c = blockIdx.x * 256 + threadIdx.x;
     if (c >= n) return;
     const uint32_t row = blockIdx.y, limb = row % limbs;
     const ModConst m = mod[limb];
     const uint64_t idx = (uint64_t)row * n + c, pidx = (uint64_t)limb * n + c;
-    const uint64_t x = a[idx], y = P[pidx], u = b[idx], v = Q[pidx];
-    uint64_t lo1 = x * y, hi1 = mulhi64(x, y);
+    const uint64_t a = x[idx], y = P[pidx], u = r[idx], v = Q[pidx];
+    uint64_t lo1 = a * y, hi1 = mulhi64(a, y);
     uint64_t lo2 = u * v, hi2 = mulhi64(u, v);
     uint64_t lo = lo1 + lo2;
     uint64_t hi = hi1 + hi2 + (lo < lo1);
-    out[idx] = barrett128(hi, lo, m);
+    sum[idx] = add_mod(a, u, m.q);
+    mix[idx] = barrett128(hi, lo, m);
 }
 
-// One lane per (output column, poly, limb, coefficient); 128-bit accumulation,
-// folded back below q every 32 products (each product < 2^122, so 33 terms
-// stay below 2^128).
-__global__ void k_mm_acc(uint64_t *out, const uint64_t *E, const uint64_t *A, const ModConst *mod, uint32_t inner,
-                         uint32_t limbs, uint32_t n)
+// sigma of both polys of every ciphertext: poly 0 in place in `cts`' layout
+// ([2][limbs][n] a ciphertext), poly 1 into tgt ([limbs][n] a ciphertext)
+__global__ void k_mm_permute(uint64_t *cts, uint64_t *tgt, const uint64_t *a, const uint32_t *perm, uint32_t limbs,
+                             uint32_t n)
 {
     const uint32_t c = blockIdx.x * 256 + threadIdx.x;
     if (c >= n) return;
+    const uint32_t row = blockIdx.y;  // (ct * 2 + p) * limbs + limb
+    const uint32_t poly = row / limbs, limb = row - poly * limbs;
+    uint64_t *o = poly & 1 ? tgt + ((uint64_t)(poly >> 1) * limbs + limb) * n : cts + (uint64_t)row * n;
+    o[c] = a[(uint64_t)row * n + perm[c]];
+}
+
+// One lane per (output column, poly, limb, coefficient); 128-bit accumulation,
+// folded back below q every 32 products (each product < 2^122, so 32 of them
+// and a folded sum stay below 2^128).  Bound by the read of E.  Plaintexts,
+// expanded batches and results are addressed where they lie, by pointers in the
+// arguments: gathered by copies first, the 768 plaintexts of 128 KB alone cost
+// 2.2 ms beside 0.5 ms here (10 columns, N = 2^13).
+struct MmAccArgs {
+    const uint64_t *A[kMmTerms];
+    const uint64_t *E[kMmBatches];
+    uint32_t first[kMmBatches + 1];  // index of each batch's first ciphertext
+    uint64_t *out[kMmCols];
+    uint32_t j0, j1;                 // terms of this launch
+    uint32_t col0;                   // its first column
+    uint32_t inner, limbs, n;
+};
+
+__global__ void k_mm_acc(MmAccArgs a, const ModConst *mod)
+{
+    const uint32_t c = blockIdx.x * 256 + threadIdx.x;
+    if (c >= a.n) return;
     const uint32_t row = blockIdx.y;  // (i * 2 + p) * limbs + l
-    const uint32_t limb = row % limbs;
-    const uint32_t ip = row / limbs, i = ip >> 1, p = ip & 1;
+    const uint32_t limb = row % a.limbs;
+    const uint32_t ip = row / a.limbs, i = ip >> 1, p = ip & 1;
     const ModConst m = mod[limb];
-    const uint64_t ct_words = 2ull * limbs * n;
-    const uint64_t *e = E + (uint64_t)i * inner * ct_words + ((uint64_t)p * limbs + limb) * n + c;
-    const uint64_t *aa = A + (uint64_t)limb * n + c;
-    const uint64_t a_stride = (uint64_t)limbs * n;
-    uint64_t lo = 0, hi = 0;
-    for (uint32_t j = 0; j < inner; j++) {
-        const uint64_t x = e[(uint64_t)j * ct_words], y = aa[(uint64_t)j * a_stride];
-        const uint64_t plo = x * y, phi = mulhi64(x, y);
-        lo += plo;
-        hi += phi + (lo < plo);
-        if ((j & 31) == 31) {
-            lo = barrett128(hi, lo, m);
-            hi = 0;
+    const uint64_t ct_words = 2ull * a.limbs * a.n;
+    const uint64_t poly_at = (uint64_t)limb * a.n + c, ct_at = (uint64_t)p * a.limbs * a.n + poly_at;
+    uint64_t *out = a.out[i] + ct_at;
+    uint64_t lo = a.j0 ? *out : 0, hi = 0;
+    uint32_t j = a.j0, k = 0;
+    const uint32_t base = (a.col0 + i) * a.inner;
+    while (j < a.j1) {
+        while (base + j >= a.first[k + 1]) k++;
+        // up to 32 terms of one batch
+        const uint32_t stop = min(min(a.j1, j + 32), a.first[k + 1] - base);
+        const uint64_t *e = a.E[k] + (uint64_t)(base + j - a.first[k]) * ct_words + ct_at;
+#pragma unroll 4
+        for (; j < stop; j++, e += ct_words) {
+            const uint64_t x = *e, y = a.A[j - a.j0][poly_at];
+            const uint64_t plo = x * y, phi = mulhi64(x, y);
+            lo += plo;
+            hi += phi + (lo < plo);
         }
+        lo = barrett128(hi, lo, m);
+        hi = 0;
     }
-    out[(uint64_t)row * n + c] = barrett128(hi, lo, m);
+    *out = lo;
 }
 
 }  // namespace
 
-void poly_mul2_add(const DeviceTables &t, uint64_t *out, const uint64_t *a, const uint64_t *P, const uint64_t *b,
-                   const uint64_t *Q, uint32_t polys, uint32_t limbs, hipStream_t s)
+void mm_combine(const DeviceTables &t, uint64_t *sum, uint64_t *mix, const uint64_t *x, const uint64_t *P,
+                const uint64_t *r, const uint64_t *Q, uint32_t polys, uint32_t limbs, hipStream_t s)
 {
     const uint32_t n = 1u << t.logn;
-    ProfScope prof("mul2_add", s, 8.0 * n * ((double)polys * limbs * 3 + 2.0 * limbs));
-    hipLaunchKernelGGL(k_mul2_add, dim3((n + 255) / 256, polys * limbs), dim3(256), 0, s, out, a, P, b, Q, t.mod,
+    ProfScope prof("mm_combine", s, 8.0 * n * ((double)polys * limbs * 4 + 2.0 * limbs));
+    hipLaunchKernelGGL(k_mm_combine, dim3((n + 255) / 256, polys * limbs), dim3(256), 0, s, sum, mix, x, P, r, Q,
+                       t.mod, limbs, n);
+}
+
+void mm_permute(const DeviceTables &t, uint64_t *cts, uint64_t *tgt, const uint64_t *a, const uint32_t *perm,
+                uint32_t count, uint32_t limbs, hipStream_t s)
+{
+    const uint32_t n = 1u << t.logn;
+    ProfScope prof("mm_permute", s, 8.0 * n * count * limbs * 4.0);
+    hipLaunchKernelGGL(k_mm_permute, dim3((n + 255) / 256, count * 2 * limbs), dim3(256), 0, s, cts, tgt, a, perm,
                        limbs, n);
 }
 
-void mm_accumulate(const DeviceTables &t, uint64_t *out, const uint64_t *E, const uint64_t *A, uint32_t cols,
-                   uint32_t inner, uint32_t limbs, hipStream_t s)
+void mm_accumulate(const DeviceTables &t, uint64_t *const *outs, const uint64_t *const *E, const size_t *counts,
+                   uint32_t batches, const uint64_t *const *A, uint32_t cols, uint32_t inner, uint32_t limbs,
+                   hipStream_t s)
 {
+    if (batches < 1 || batches > (uint32_t)kMmBatches)
+        throw std::invalid_argument("mm_accumulate: too many batches");
     const uint32_t n = 1u << t.logn;
     ProfScope prof("mm_acc", s, 8.0 * n * limbs * ((double)cols * inner * 2 + inner + cols * 2.0));
-    hipLaunchKernelGGL(k_mm_acc, dim3((n + 255) / 256, cols * 2 * limbs), dim3(256), 0, s, out, E, A, t.mod, inner,
-                       limbs, n);
+    MmAccArgs a;
+    a.inner = inner;
+    a.limbs = limbs;
+    a.n = n;
+    uint64_t first = 0;
+    for (uint32_t k = 0; k < (uint32_t)kMmBatches; k++) {
+        a.E[k] = k < batches ? E[k] : nullptr;
+        a.first[k] = (uint32_t)first;
+        if (k < batches) first += counts[k];
+    }
+    a.first[kMmBatches] = (uint32_t)first;
+    if (first < (uint64_t)cols * inner || first >> 32)
+        throw std::invalid_argument("mm_accumulate: not enough expanded ciphertexts");
+    for (a.col0 = 0; a.col0 < cols; a.col0 += kMmCols) {
+        const uint32_t cnt = std::min((uint32_t)kMmCols, cols - a.col0);
+        for (uint32_t i = 0; i < (uint32_t)kMmCols; i++) a.out[i] = i < cnt ? outs[a.col0 + i] : nullptr;
+        for (a.j0 = 0; a.j0 < inner; a.j0 = a.j1) {
+            a.j1 = std::min(inner, a.j0 + (uint32_t)kMmTerms);
+            for (uint32_t j = 0; j < (uint32_t)kMmTerms; j++) a.A[j] = a.j0 + j < a.j1 ? A[a.j0 + j] : nullptr;
+            hipLaunchKernelGGL(k_mm_acc, dim3((n + 255) / 256, cnt * 2 * limbs), dim3(256), 0, s, a, t.mod);
+        }
+    }
 }
 
 }  // namespace nx

@@ -113,12 +113,7 @@ void mm_expand(Context &c, const Ciphertext &ct, uint32_t m, const uint32_t *elt
         // rot = tau_elt(cur): permute both polys, key-switch the permuted c1
         const uint32_t *perm = c.galois_table(elt);
         DevBuf rot(&c, S * ctw), tgt(&c, S * l * n);
-        // c0 of every ciphertext -> rot, c1 -> tgt: permute a [S][2][l] view
-        // row by row (rows of one ciphertext are contiguous)
-        DevBuf perm_all(&c, S * ctw);
-        poly_permute(perm_all.get(), cur.data.get(), perm, (uint32_t)(2 * S), (uint32_t)l, c.logn, c.stream);
-        poly_copy_limbs(c.tables, rot.get(), ctw, perm_all.get(), ctw, (uint32_t)S, (uint32_t)l, c.stream);
-        poly_copy_limbs(c.tables, tgt.get(), l * n, perm_all.get() + l * n, ctw, (uint32_t)S, (uint32_t)l, c.stream);
+        mm_permute(c.tables, rot.get(), tgt.get(), cur.data.get(), perm, (uint32_t)S, (uint32_t)l, c.stream);
         key_switch_batch(c, rot.get(), tgt.get(), S, l, it->second, true, nullptr, gk.seeds_of(elt));
         // next round: [cur + rot | cur * x^(2n - 2^i) + rot * x^((2n - 2^i) * elt mod 2n)]
         CtBatch nxt;
@@ -127,13 +122,12 @@ void mm_expand(Context &c, const Ciphertext &ct, uint32_t m, const uint32_t *elt
         nxt.limbs = l;
         nxt.scale = ct.scale;
         nxt.data.reset(&c, 2 * S * ctw);
-        poly_add(c.tables, nxt.data.get(), cur.data.get(), rot.get(), (uint32_t)(2 * S), (uint32_t)l, c.stream);
         const uint64_t two_n = 2 * (uint64_t)n;
         const uint32_t k_raw = (uint32_t)(two_n - (1ull << i));
         const uint32_t k_idx = (uint32_t)(((uint64_t)k_raw * elt) % two_n);
         const uint64_t *P = power_of_x_ntt(c, k_raw, l), *Q = power_of_x_ntt(c, k_idx, l);
-        poly_mul2_add(c.tables, nxt.data.get() + S * ctw, cur.data.get(), P, rot.get(), Q, (uint32_t)(2 * S),
-                      (uint32_t)l, c.stream);
+        mm_combine(c.tables, nxt.data.get(), nxt.data.get() + S * ctw, cur.data.get(), P, rot.get(), Q,
+                   (uint32_t)(2 * S), (uint32_t)l, c.stream);
         cur = std::move(nxt);
     }
     out = std::move(cur);
@@ -153,26 +147,39 @@ void mm_accumulate_cts(Context &c, const std::vector<const Plaintext *> &a, cons
     }
     require(total >= cols * inner, "not enough expanded ciphertexts");
     for (auto *p : a) require(p->limbs == l && p->ntt, "plaintext level mismatch");
-    // gather: expanded ciphertexts and plaintexts into contiguous operands
-    DevBuf Ebuf, Abuf(&c, inner * l * n);
-    const uint64_t *Eptr;
-    if (E.size() == 1) {
-        Eptr = E[0]->data.get();
-    } else {
-        Ebuf.reset(&c, cols * inner * ctw);
+    // operands are read where they lie; copied first: those of another context
+    // (which may be another device's), and batches beyond what a launch names
+    std::vector<const uint64_t *> A, Ep;
+    std::vector<size_t> counts;
+    std::vector<DevBuf> copies;
+    for (auto *p : a) {
+        A.push_back(p->data.get());
+        if (p->ctx == &c) continue;
+        copies.emplace_back(&c, l * n);
+        d2d(c, copies.back().get(), p->data.get(), l * n);
+        A.back() = copies.back().get();
+    }
+    bool gather = E.size() > (size_t)kMmBatches;
+    for (auto *e : E) gather = gather || e->ctx != &c;
+    if (gather) {
+        copies.emplace_back(&c, cols * inner * ctw);
         size_t off = 0;
         for (auto *e : E) {
             const size_t take = std::min(e->B, cols * inner - off);
             if (!take) break;
-            d2d(c, Ebuf.get() + off * ctw, e->data.get(), take * ctw);
+            d2d(c, copies.back().get() + off * ctw, e->data.get(), take * ctw);
             off += take;
         }
-        Eptr = Ebuf.get();
+        Ep.push_back(copies.back().get());
+        counts.push_back(cols * inner);
+    } else {
+        for (auto *e : E) {
+            Ep.push_back(e->data.get());
+            counts.push_back(e->B);
+        }
     }
-    for (size_t j = 0; j < inner; j++) d2d(c, Abuf.get() + j * l * n, a[j]->data.get(), l * n);
-    DevBuf res(&c, cols * ctw);
-    mm_accumulate(c.tables, res.get(), Eptr, Abuf.get(), (uint32_t)cols, (uint32_t)inner, (uint32_t)l, c.stream);
     out.resize(cols);
+    std::vector<uint64_t *> outs;
     const double scale = E[0]->scale * a[0]->scale;
     for (size_t i = 0; i < cols; i++) {
         Ciphertext r;
@@ -182,9 +189,11 @@ void mm_accumulate_cts(Context &c, const std::vector<const Plaintext *> &a, cons
         r.scale = scale;
         r.ntt = true;
         r.data.reset(&c, ctw);
-        d2d(c, r.data.get(), res.get() + i * ctw, ctw);
+        outs.push_back(r.data.get());
         out[i] = std::move(r);
     }
+    mm_accumulate(c.tables, outs.data(), Ep.data(), counts.data(), (uint32_t)Ep.size(), A.data(), (uint32_t)cols,
+                  (uint32_t)inner, (uint32_t)l, c.stream);
 }
 
 }  // namespace nx
