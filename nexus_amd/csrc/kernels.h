@@ -297,7 +297,7 @@ constexpr int kMaxDot = 64;
 // g < rows <= kMultiDotG, k < 2, count <= kMultiDotK (pts entries may be null:
 // no term); each ciphertext is read once for all rows.  accumulate adds into
 // the outputs instead of writing them.
-constexpr int kMultiDotG = 4, kMultiDotK = 32;
+constexpr int kMultiDotG = 8, kMultiDotK = 32;
 void poly_dot_plain_multi(const DeviceTables &t, uint64_t *const *outs, const uint64_t *const *cts,
                           const uint64_t *const *pts, uint32_t rows, uint32_t count, uint32_t limbs, bool accumulate,
                           hipStream_t s);

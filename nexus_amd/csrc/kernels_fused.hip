@@ -365,56 +365,81 @@ struct MultiDotArgs {
     uint64_t *out[kMultiDotG];                    // null: unused row
 };
 
-// out_g[k][limb][c] (+)= sum_r ct_r[k][limb][c] * pt_g,r[limb][c] for the rows g
+// V adjacent words
+template <int V>
+__device__ __forceinline__ void load_words(uint64_t *v, const uint64_t *p)
+{
+    if constexpr (V == 2) {
+        const ulonglong2 x = *reinterpret_cast<const ulonglong2 *>(p);
+        v[0] = x.x;
+        v[1] = x.y;
+    } else {
+        v[0] = *p;
+    }
+}
+
+// out_g[k][limb][c] (+)= sum_r ct_r[k][limb][c] * pt_g,r[limb][c] for the G rows
 // of one launch (k < 2, count <= kMultiDotK, so no intermediate fold): every
-// ciphertext word is read once for all rows.  Two adjacent coefficients of one
-// limb per thread, 16-byte loads, as k_dot_plain.
+// ciphertext word is read once for all rows.  Bound by those reads: with up to
+// eight rows a launch the ciphertexts of a product with eight giant steps are
+// read once instead of twice.  One and two rows take two adjacent coefficients a
+// thread (16-byte loads); more take one, which keeps the sums (G V 2 of 128 bits)
+// in as many registers.  Where every plaintext is there (!HOLES) the loads of a
+// term carry no branch between them and are in flight together.  Sixteen
+// ciphertexts of 34 limbs at N = 2^16 times eight rows: 744 us in two launches of
+// four rows, 640 us in one.
+template <int G, int V, bool HOLES>
 __global__ __launch_bounds__(kBlock) void k_dot_plain_multi(MultiDotArgs args, uint32_t count, const ModConst *mod,
                                                             uint32_t limbs, uint32_t n, int accumulate)
 {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;  // coefficient pair
-    if (2 * i >= n) return;
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (V * i >= n) return;
     const uint32_t limb = blockIdx.y;
     const ModConst m = mod[limb];
-    const uint64_t poff = (uint64_t)limb * n + 2 * i, off1 = poff + (uint64_t)limbs * n;
-    uint64_t lo[kMultiDotG][4] = {}, hi[kMultiDotG][4] = {};
+    const uint64_t poff = (uint64_t)limb * n + V * i, off1 = poff + (uint64_t)limbs * n;
+    uint64_t lo[G][2 * V] = {}, hi[G][2 * V] = {};
     for (uint32_t r = 0; r < count; r++) {
-        const ulonglong2 a = *reinterpret_cast<const ulonglong2 *>(args.ct[r] + poff);
-        const ulonglong2 b = *reinterpret_cast<const ulonglong2 *>(args.ct[r] + off1);
-        const uint64_t xs[4] = {a.x, a.y, b.x, b.y};
+        uint64_t x[2 * V], y[G][V];
+        load_words<V>(x, args.ct[r] + poff);
+        load_words<V>(x + V, args.ct[r] + off1);
+        if (!HOLES) {
 #pragma unroll
-        for (int g = 0; g < kMultiDotG; g++) {
-            const uint64_t *p = args.pt[g][r];
-            if (!p) continue;  // uniform across the launch
-            const ulonglong2 y = *reinterpret_cast<const ulonglong2 *>(p + poff);
-            const uint64_t ys[4] = {y.x, y.y, y.x, y.y};
+            for (int g = 0; g < G; g++) load_words<V>(y[g], args.pt[g][r] + poff);
+        }
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const uint64_t plo = xs[k] * ys[k], phi = mulhi64(xs[k], ys[k]);
+        for (int g = 0; g < G; g++) {
+            if (HOLES) {
+                const uint64_t *p = args.pt[g][r];
+                if (!p) continue;  // uniform across the launch
+                load_words<V>(y[g], p + poff);
+            }
+#pragma unroll
+            for (int k = 0; k < 2 * V; k++) {
+                const uint64_t plo = x[k] * y[g][k % V], phi = mulhi64(x[k], y[g][k % V]);
                 lo[g][k] += plo;
                 hi[g][k] += phi + (lo[g][k] < plo);
             }
         }
     }
 #pragma unroll
-    for (int g = 0; g < kMultiDotG; g++) {
-        uint64_t *o = args.out[g];
-        if (!o) continue;
-        ulonglong2 o0, o1;
-        o0.x = barrett128(hi[g][0], lo[g][0], m);
-        o0.y = barrett128(hi[g][1], lo[g][1], m);
-        o1.x = barrett128(hi[g][2], lo[g][2], m);
-        o1.y = barrett128(hi[g][3], lo[g][3], m);
+    for (int g = 0; g < G; g++) {
+        uint64_t o[2 * V];
+#pragma unroll
+        for (int k = 0; k < 2 * V; k++) o[k] = barrett128(hi[g][k], lo[g][k], m);
         if (accumulate) {
-            const ulonglong2 p0 = *reinterpret_cast<const ulonglong2 *>(o + poff);
-            const ulonglong2 p1 = *reinterpret_cast<const ulonglong2 *>(o + off1);
-            o0.x = add_mod(o0.x, p0.x, m.q);
-            o0.y = add_mod(o0.y, p0.y, m.q);
-            o1.x = add_mod(o1.x, p1.x, m.q);
-            o1.y = add_mod(o1.y, p1.y, m.q);
+            uint64_t old[2 * V];
+            load_words<V>(old, args.out[g] + poff);
+            load_words<V>(old + V, args.out[g] + off1);
+#pragma unroll
+            for (int k = 0; k < 2 * V; k++) o[k] = add_mod(o[k], old[k], m.q);
         }
-        *reinterpret_cast<ulonglong2 *>(o + poff) = o0;
-        *reinterpret_cast<ulonglong2 *>(o + off1) = o1;
+        if constexpr (V == 2) {
+            *reinterpret_cast<ulonglong2 *>(args.out[g] + poff) = make_ulonglong2(o[0], o[1]);
+            *reinterpret_cast<ulonglong2 *>(args.out[g] + off1) = make_ulonglong2(o[2], o[3]);
+        } else {
+            args.out[g][poff] = o[0];
+            args.out[g][off1] = o[1];
+        }
     }
 }
 
@@ -546,8 +571,21 @@ void poly_dot_plain_multi(const DeviceTables &t, uint64_t *const *outs, const ui
     }
     ProfScope prof("dot_plain", s,
                    8.0 * n * limbs * (2.0 * count + terms + 2.0 * rows * (accumulate ? 2.0 : 1.0)));
-    hipLaunchKernelGGL(k_dot_plain_multi, dim3((n / 2 + kBlock - 1) / kBlock, limbs), dim3(kBlock), 0, s, a, count,
-                       t.mod, limbs, n, accumulate ? 1 : 0);
+    const bool holes = terms < rows * count;
+#define NX_DOT(G, V)                                                                                             \
+    case G:                                                                                                      \
+        if (holes)                                                                                               \
+            hipLaunchKernelGGL((k_dot_plain_multi<G, V, true>), dim3((n / V + kBlock - 1) / kBlock, limbs),        \
+                               dim3(kBlock), 0, s, a, count, t.mod, limbs, n, accumulate ? 1 : 0);               \
+        else                                                                                                     \
+            hipLaunchKernelGGL((k_dot_plain_multi<G, V, false>), dim3((n / V + kBlock - 1) / kBlock, limbs),       \
+                               dim3(kBlock), 0, s, a, count, t.mod, limbs, n, accumulate ? 1 : 0);               \
+        break;
+    switch (rows) {
+        NX_DOT(1, 2) NX_DOT(2, 2) NX_DOT(3, 1) NX_DOT(4, 1) NX_DOT(5, 1) NX_DOT(6, 1) NX_DOT(7, 1) NX_DOT(8, 1)
+    default: break;
+    }
+#undef NX_DOT
 }
 
 void poly_dot_plain(const DeviceTables &t, uint64_t *out, const uint64_t *const *cts, const uint64_t *const *pts,
