@@ -65,9 +65,10 @@ void op_rotate_hoisted(const Ciphertext &a, const std::vector<int> &steps, const
         for (size_t base = 0; base < p.keys.size(); base += kMaxHoist) {
             const size_t cnt = std::min<size_t>(kMaxHoist, p.keys.size() - base);
             DevBuf acc(&c, cnt * 2 * nout * n);
-            ks_inner_product_rot(c.tables, acc.get(), T.get(), p.keys.data() + base, p.perms.data() + base,
+            const uint64_t *t = T.get();
+            ks_inner_product_rot(c.tables, acc.get(), &t, 1, p.keys.data() + base, p.perms.data() + base,
                                  (uint32_t)cnt, (uint32_t)c.digits(l), (uint32_t)c.key_limbs(), outp, (uint32_t)nout,
-                                 c.stream, nullptr, p.seeds.data() + base);
+                                 c.stream, p.seeds.data() + base);
             FwdInput in_tmp;
             DevBuf tmp = ks_moddown_prepare(c, acc.get(), cnt, l, in_tmp);
             // each result written in place by the transform's last pass:
@@ -132,43 +133,37 @@ void op_rotate_hoisted_many(const std::vector<const Ciphertext *> &in, const std
             Ts.push_back(ks_modup_list(c, c1s.data(), cnt, l));
             for (size_t b = 0; b < cnt; b++) tp[b0 + b] = Ts.back().get() + b * tstride;
         }
-        // (input, rotation) pairs in chunks of kMaxHoist
-        const size_t P = B * R;
-        for (size_t base = 0; base < P; base += (size_t)kMaxHoist) {
-            const size_t cnt = std::min<size_t>((size_t)kMaxHoist, P - base);
-            std::vector<const uint64_t *> keys(cnt), tps(cnt), seeds(cnt);
-            std::vector<const uint32_t *> perms(cnt);
-            for (size_t r = 0; r < cnt; r++) {
-                const size_t b = (base + r) / R, k = (base + r) % R;
-                keys[r] = p.keys[k];
-                seeds[r] = p.seeds[k];
-                perms[r] = p.perms[k];
-                tps[r] = tp[b];
+        // (step, input) pairs, up to kMaxHoist a launch: whole steps, whose inputs
+        // share a key
+        for (size_t b0 = 0; b0 < B; b0 += (size_t)kMaxHoist) {
+            const size_t nb = std::min<size_t>((size_t)kMaxHoist, B - b0), most = (size_t)kMaxHoist / nb;
+            for (size_t k0 = 0; k0 < R; k0 += most) {
+                const size_t nk = std::min(most, R - k0), cnt = nk * nb;
+                DevBuf acc(&c, cnt * 2 * nout * n);
+                ks_inner_product_rot(c.tables, acc.get(), tp.data() + b0, (uint32_t)nb, p.keys.data() + k0,
+                                     p.perms.data() + k0, (uint32_t)nk, (uint32_t)digits, (uint32_t)c.key_limbs(), outp,
+                                     (uint32_t)nout, c.stream, p.seeds.data() + k0);
+                FwdInput in_tmp;
+                DevBuf tmp = ks_moddown_prepare(c, acc.get(), cnt, l, in_tmp);
+                NttEpilogue e;
+                for (size_t r = 0; r < cnt; r++) {
+                    const size_t b = b0 + r % nb, k = k0 + r / nb;
+                    Ciphertext &o = out[b][p.index[k]];
+                    o.ctx = &c;
+                    o.size = 2;
+                    o.limbs = l;
+                    o.scale = in[b]->scale;
+                    o.ntt = true;
+                    o.data.reset(&c, 2 * pw);
+                    e.outs[r] = o.data.get();
+                    e.perm[r] = p.perms[k];
+                    e.a0s[r] = in[b]->data.get();
+                }
+                e.x = acc.get();
+                e.x_stride = nout * n;
+                e.inv = c.d_p_inv;
+                ntt_fwd_epi(c, tmp.get(), 2 * cnt, l, l * n, e, in_tmp);
             }
-            DevBuf acc(&c, cnt * 2 * nout * n);
-            ks_inner_product_rot(c.tables, acc.get(), nullptr, keys.data(), perms.data(), (uint32_t)cnt,
-                                 (uint32_t)digits, (uint32_t)c.key_limbs(), outp, (uint32_t)nout, c.stream,
-                                 tps.data(), seeds.data());
-            FwdInput in_tmp;
-            DevBuf tmp = ks_moddown_prepare(c, acc.get(), cnt, l, in_tmp);
-            NttEpilogue e;
-            for (size_t r = 0; r < cnt; r++) {
-                const size_t b = (base + r) / R, k = (base + r) % R;
-                Ciphertext &o = out[b][p.index[k]];
-                o.ctx = &c;
-                o.size = 2;
-                o.limbs = l;
-                o.scale = in[b]->scale;
-                o.ntt = true;
-                o.data.reset(&c, 2 * pw);
-                e.outs[r] = o.data.get();
-                e.perm[r] = perms[r];
-                e.a0s[r] = in[b]->data.get();
-            }
-            e.x = acc.get();
-            e.x_stride = nout * n;
-            e.inv = c.d_p_inv;
-            ntt_fwd_epi(c, tmp.get(), 2 * cnt, l, l * n, e, in_tmp);
         }
     }
     dst = std::move(out);

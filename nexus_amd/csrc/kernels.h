@@ -341,15 +341,15 @@ void block_mix(const DeviceTables &t, const MixPtrs &p, const uint64_t *table, c
 constexpr int kQuadWords = 8, kSingleWords = 8;
 std::vector<int32_t> block_mix_plan(const int32_t *index, uint32_t K, uint32_t M);
 
-// Hoisted variants over one shared ModUp T[nout][l][n] (B = 1): rotation r
-// reads digit values through the NTT-domain Galois permutation perms[r]
-// (T[I][j][perms[r][c]]) and uses key keys[r].  _rot writes one result per
-// rotation, acc[r][2][nout][n]; _rot_sum writes (or adds to acc) their sum,
-// acc[2][nout][n].
-void ks_inner_product_rot(const DeviceTables &t, uint64_t *acc, const uint64_t *T, const uint64_t *const *keys,
-                          const uint32_t *const *perms, uint32_t count, uint32_t l, uint32_t key_limbs,
-                          const uint8_t *out_primes_host, uint32_t nout, hipStream_t s,
-                          const uint64_t *const *Ts = nullptr, const uint64_t *const *aseeds = nullptr);
+// Hoisted variants over ModUps T[nout][l][n]: rotation r reads digit values
+// through the NTT-domain Galois permutation perms[r] (T[I][j][perms[r][c]]) and
+// uses key keys[r].  _rot writes one result per step r and input b (at most
+// kMaxHoist of each), acc[r inputs + b][2][nout][n]; _rot_sum writes (or adds to
+// acc) the sum of the rotations of one T, acc[2][nout][n].
+void ks_inner_product_rot(const DeviceTables &t, uint64_t *acc, const uint64_t *const *Ts, uint32_t inputs,
+                          const uint64_t *const *keys, const uint32_t *const *perms, uint32_t steps, uint32_t l,
+                          uint32_t key_limbs, const uint8_t *out_primes_host, uint32_t nout, hipStream_t s,
+                          const uint64_t *const *aseeds = nullptr);
 // t_stride > 0: rotation r reads its own ModUp at T + r t_stride (a sum of
 // rotations of different inputs) instead of the shared T.
 void ks_inner_product_rot_sum(const DeviceTables &t, uint64_t *acc, const uint64_t *T, const uint64_t *const *keys,
