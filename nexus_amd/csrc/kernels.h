@@ -88,8 +88,9 @@ struct NttBatch {
     // when I = p % poly_period < skip_l and I / skip_alpha == j (0: none)
     uint32_t skip_l = 0, skip_alpha = 0;
     NttEpilogue epi;  // forward transforms only
-    // forward, n >= 2^14: the column pass has already run (ks_modup_convert_col);
-    // only the row pass is launched
+    // n >= 2^14, only the row pass is launched: forward, the column pass has
+    // already run (ks_modup_convert_col); inverse, it runs in the conversion that
+    // follows (ks_modup_col_inverse)
     uint32_t rows_only = 0;
     // Forward, instead of words below each limb's prime:
     //  lift: limb j of poly p is lift[(p / poly_period) limbs + j] (limbs of n
@@ -249,7 +250,10 @@ void ks_modup_col_set(uint32_t B, int mode);
 int ks_modup_col_get(uint32_t B);
 void ks_modup_convert_col(const DeviceTables &t, uint64_t *T, const uint64_t *coef, const ulonglong2 *w,
                           uint32_t B, uint32_t l, uint32_t alpha, uint32_t key_limbs, const uint8_t *out_primes_host,
-                          uint32_t nout, hipStream_t s, bool raw = false);
+                          uint32_t nout, hipStream_t s, bool raw = false, bool inverse = false);
+// whether coef had better come from the inverse's row pass alone, its column pass
+// being left to ks_modup_convert_col (raw and inverse set)
+bool ks_modup_col_inverse(const DeviceTables &t, uint32_t B, uint32_t l, uint32_t alpha);
 // The digits of a key switch from the column pass to the inner product
 // (kernels_ks.hip): T[b][I - i0][j] for the output primes i0 .. i0 + icount - 1
 // outside digit j holds column-transformed values as ks_row_inner reads them
@@ -283,7 +287,9 @@ void ks_row_inner(const DeviceTables &t, const KsRowInner &p, hipStream_t s);
 bool ks_moddown_col_ok(const DeviceTables &t, uint32_t A);
 void ks_moddown_convert_col(const DeviceTables &t, uint64_t *z, const uint64_t *acc, uint64_t acc_stride,
                             const ulonglong2 *w, const double *convd, const uint8_t *in_primes_host, uint32_t A,
-                            uint32_t polys, uint32_t lo, uint32_t L, hipStream_t s);
+                            uint32_t polys, uint32_t lo, uint32_t L, hipStream_t s, bool inverse = false);
+// as ks_modup_col_inverse, for the limbs of acc
+bool ks_moddown_col_inverse(const DeviceTables &t, uint32_t polys);
 // per power-of-two bucket of the poly count: as ks_modup_col_set
 void ks_moddown_col_set(uint32_t polys, int mode);
 int ks_moddown_col_get(uint32_t polys);

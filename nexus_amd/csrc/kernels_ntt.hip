@@ -377,7 +377,28 @@ __global__ __launch_bounds__(NT) void k_ntt(NttKArgs a)
 // products are the exact double-precision ones of the unfused conversion
 // (k_modup_conv_a), and the column stages those of the double-precision pass,
 // so the stored words equal the unfused conversion followed by the column pass.
+// The inverse's column pass of a tile, on the 8 words of a thread in the order the
+// conversions hold them; fully reduced to [0, q).  lds: 2048 doubles that no
+// other thread still reads.
+template <int LOGS>
+__device__ __forceinline__ void col_inverse(double *x, double *lds, const double *tw, double ninv, double q,
+                                            double qinv, uint32_t n, uint32_t col0)
+{
+    using C = ColTile<LOGS>;
+    const int tid = threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < 8; k++) lds[C::row_in(tid, k) * C::CW + tid % C::CW] = reduce_f(x[k], q, qinv);
+    __syncthreads();
+    stages_f<LOGS, kCol, false, C::CW, false, kThreads, false>(lds, tw, q, qinv, n, 1u << LOGS, col0);
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const double v = reduce_f(mulmod_f(lds[C::row_in(tid, k) * C::CW + tid % C::CW], ninv, q, qinv), q, qinv);
+        x[k] = v < 0 ? v + q : v;
+    }
+}
+
 struct ModUpColArgs {
+    const double *invd, *ninvd;  // the inverse's tables (INV)
     uint64_t *T;
     const uint64_t *coef;
     const ulonglong2 *w;
@@ -393,7 +414,8 @@ struct ModUpColArgs {
 // The order of the loop hides the latencies behind arithmetic: an output's
 // twiddles are asked for before its conversion, the next output's factors
 // before the current one's stages.
-template <int LOGS, int A, int S, bool RAW>
+// INV: the inputs come from the inverse's row pass; its column pass runs here.
+template <int LOGS, int A, int S, bool RAW, bool INV>
 __device__ __forceinline__ void modup_tile(const ModUpColArgs &a, double *lds, uint32_t b, uint32_t j, uint32_t s,
                                            uint32_t r0, uint32_t r1)
 {
@@ -417,12 +439,17 @@ __device__ __forceinline__ void modup_tile(const ModUpColArgs &a, double *lds, u
         const double wi = (double)a.w[base + (on ? i : 0)].x;
         const uint64_t *x = a.coef + ((uint64_t)b * a.l + p) * n;
 #pragma unroll
+        for (int k = 0; k < 8; k++) y[i][k] = fp_from((x + C::row_step(k) * N2)[at]);
+        if (INV && on)  // uniform
+            col_inverse<LOGS>(y[i], lds + (i & 1) * C::LDS, a.invd + (uint64_t)p * n, a.ninvd[p], q, qinv, n, col0);
+#pragma unroll
         for (int k = 0; k < 8; k++) {
-            double v = reduce_f(mulmod_f(fp_from((x + C::row_step(k) * N2)[at]), wi, q, qinv), q, qinv);
+            double v = reduce_f(mulmod_f(y[i][k], wi, q, qinv), q, qinv);
             v = v < 0 ? v + q : v;
             y[i][k] = on ? v : 0.0;
         }
     }
+    if (INV) __syncthreads();  // the last input's buffer may be the first output's
     const double *factors = a.convd + (uint64_t)base * a.key_limbs;
     auto prime = [&](uint32_t r) { return a.outp[r < first ? r : r + s]; };
     double f[S], q, qinv;
@@ -453,7 +480,7 @@ __device__ __forceinline__ void modup_tile(const ModUpColArgs &a, double *lds, u
     }
 }
 
-template <int LOGS, int A, bool RAW>
+template <int LOGS, int A, bool RAW, bool INV>
 __global__ __launch_bounds__(kThreads, A <= 9 ? 2 : 1) void k_modup_col(ModUpColArgs a)
 {
     __shared__ double lds[2 * ColTile<LOGS>::LDS];
@@ -466,9 +493,9 @@ __global__ __launch_bounds__(kThreads, A <= 9 ? 2 : 1) void k_modup_col(ModUpCol
     if (r0 >= count) return;  // uniform, before any barrier
     const uint32_t r1 = min(count, r0 + a.chunk);
     if (A > 4 && s <= A / 2)
-        modup_tile<LOGS, A, A / 2, RAW>(a, lds, b, j, s, r0, r1);
+        modup_tile<LOGS, A, A / 2, RAW, INV>(a, lds, b, j, s, r0, r1);
     else
-        modup_tile<LOGS, A, A, RAW>(a, lds, b, j, s, r0, r1);
+        modup_tile<LOGS, A, A, RAW, INV>(a, lds, b, j, s, r0, r1);
 }
 
 // ---- ModDown base conversion fused into the forward column pass
@@ -539,6 +566,7 @@ __global__ __launch_bounds__(kThreads) void k_center_col(CenterColArgs a)
 }
 
 struct ModDownColArgs {
+    const double *invd, *ninvd;  // the inverse's tables (INV)
     uint64_t *z;
     const uint64_t *acc;
     uint64_t acc_stride;
@@ -551,7 +579,7 @@ struct ModDownColArgs {
     uint32_t inp[kMaxPrimes];
 };
 
-template <int LOGS, int A>
+template <int LOGS, int A, bool INV>
 __global__ __launch_bounds__(kThreads, A <= 9 ? 2 : 1) void k_moddown_col(ModDownColArgs a)
 {
     using C = ColTile<LOGS>;
@@ -576,9 +604,13 @@ __global__ __launch_bounds__(kThreads, A <= 9 ? 2 : 1) void k_moddown_col(ModDow
         const double pi = a.qd[a.inp[i]].x, pinv = a.qd[a.inp[i]].y;
         pmax = pi > pmax ? pi : pmax;
 #pragma unroll
+        for (int k = 0; k < 8; k++) v[i][k] = fp_from((y + (uint64_t)i * n + C::row_step(k) * N2)[at]);
+        if (INV)
+            col_inverse<LOGS>(v[i], lds + (i & 1) * C::LDS, a.invd + (uint64_t)a.inp[i] * n, a.ninvd[a.inp[i]], pi,
+                              pinv, n, col0);
+#pragma unroll
         for (int k = 0; k < 8; k++) {
-            double x = reduce_f(mulmod_f(fp_from((y + (uint64_t)i * n + C::row_step(k) * N2)[at]), wi, pi, pinv),
-                                pi, pinv);
+            double x = reduce_f(mulmod_f(v[i][k], wi, pi, pinv), pi, pinv);
             x = x < 0 ? x + pi : x;
             // x / p_i correctly rounded: pinv is the correctly rounded 1 / p_i, so
             // one residual step on x pinv gives the quotient a division gives
@@ -589,6 +621,7 @@ __global__ __launch_bounds__(kThreads, A <= 9 ? 2 : 1) void k_moddown_col(ModDow
     }
 #pragma unroll
     for (int k = 0; k < 8; k++) rr[k] = __builtin_floor(rr[k] + 0.5);  // <= A
+    if (INV) __syncthreads();  // the last input's buffer may be the first output's
     double f[A + 1], q, qinv;
     auto load_factors = [&](uint32_t i) {
 #pragma unroll
@@ -901,9 +934,36 @@ bool ks_modup_col_ok(const DeviceTables &t, uint32_t alpha)
            t.modup_conv_d != nullptr;
 }
 
+// Outputs per workgroup: enough workgroups to fill the device, at least 4
+// outputs per read of the digit's inputs.
+static uint32_t modup_col_chunk(const DeviceTables &t, uint32_t B, uint32_t l, uint32_t alpha, uint32_t nout)
+{
+    const uint32_t tiles = (1u << t.logn) / 2048u, digits = (l + alpha - 1) / alpha;
+    const uint32_t count = nout - std::min(alpha, l);  // most outputs of a digit (a partial digit has more)
+    const uint32_t want = (2048u + tiles * B * digits - 1) / (tiles * B * digits);
+    uint32_t chunk = std::max((count + want - 1) / want, std::min(4u, count));
+    const int mode = g_modup_col[tune_bucket(B)].load();  // 0: this rule
+    if (mode > 0 && (mode & 255)) chunk = std::min((uint32_t)(mode & 255), count);
+    return chunk;
+}
+
+// The inverse's column pass belongs in the conversion where one workgroup can
+// make all outputs of a digit and there are still kInverseBlocks of them (two
+// rounds of the two a CU holds): it saves a read and a write of every input.
+// With the outputs cut up each part would repeat it.
+// 64 fused products at 20 limbs, N = 2^16: 6.37 ms with the column pass apart,
+// 5.99 with it here; with the line at 2048 workgroups and outputs cut up below
+// that, 6.14.  Six sums of sixteen rotations: 4.94, 4.80 and 4.91 ms.
+constexpr uint32_t kInverseBlocks = 1024;
+bool ks_modup_col_inverse(const DeviceTables &t, uint32_t B, uint32_t l, uint32_t alpha)
+{
+    return ks_modup_col_ok(t, alpha) && l >= 1 && g_modup_col[tune_bucket(B)].load() == 0 &&
+           (1u << t.logn) / 2048u * B * ((l + alpha - 1) / alpha) >= kInverseBlocks;
+}
+
 void ks_modup_convert_col(const DeviceTables &t, uint64_t *T, const uint64_t *coef, const ulonglong2 *w,
                           uint32_t B, uint32_t l, uint32_t alpha, uint32_t key_limbs, const uint8_t *out_primes_host,
-                          uint32_t nout, hipStream_t s, bool raw)
+                          uint32_t nout, hipStream_t s, bool raw, bool inverse)
 {
     if (!ks_modup_col_ok(t, alpha)) throw std::invalid_argument("ks_modup_convert_col: unsupported parameters");
     if (nout > (uint32_t)kMaxPrimes || l < 1 || nout <= alpha) throw std::invalid_argument("ks_modup_convert_col: bad sizes");
@@ -923,16 +983,10 @@ void ks_modup_convert_col(const DeviceTables &t, uint64_t *T, const uint64_t *co
     int l1, l2;
     split_logn(t.logn, l1, l2);
     const uint32_t n = 1u << t.logn;
-    // mode: outputs per workgroup (0: default rule)
-    const int mode = g_modup_col[tune_bucket(B)].load();
     const uint32_t tiles = n / 2048u;
-    // outputs per workgroup: enough workgroups to fill the device, at least 4
-    // outputs per read of the digit's inputs
-    const uint32_t count = nout - std::min(alpha, l);  // most outputs of a digit (a partial digit has more)
-    const uint32_t want = (2048u + tiles * B * a.digits - 1) / (tiles * B * a.digits);
-    uint32_t chunk = (count + want - 1) / want;
-    chunk = std::max(chunk, std::min(4u, count));
-    if (mode > 0 && (mode & 255)) chunk = std::min((uint32_t)(mode & 255), count);
+    const uint32_t chunk = inverse ? nout - 1 : modup_col_chunk(t, B, l, alpha, nout);
+    a.invd = t.inv_d;
+    a.ninvd = t.ninv_d;
     a.chunk = chunk;
     a.chunks = (nout - 1 + chunk - 1) / chunk;  // covers a partial last digit (nout - s <= nout - 1 outputs)
     uint32_t outs = 0;
@@ -943,10 +997,12 @@ void ks_modup_convert_col(const DeviceTables &t, uint64_t *T, const uint64_t *co
     const dim3 grid(tiles, B * a.digits * a.chunks);
 #define NX_MC(LOGS, A)                                                                      \
     if (l1 == LOGS && alpha == A) {                                                       \
-        if (raw)                                                                          \
-            hipLaunchKernelGGL((k_modup_col<LOGS, A, true>), grid, dim3(kThreads), 0, s, a);  \
+        if (raw && inverse)                                                               \
+            hipLaunchKernelGGL((k_modup_col<LOGS, A, true, true>), grid, dim3(kThreads), 0, s, a);   \
+        else if (raw)                                                                     \
+            hipLaunchKernelGGL((k_modup_col<LOGS, A, true, false>), grid, dim3(kThreads), 0, s, a);  \
         else                                                                              \
-            hipLaunchKernelGGL((k_modup_col<LOGS, A, false>), grid, dim3(kThreads), 0, s, a); \
+            hipLaunchKernelGGL((k_modup_col<LOGS, A, false, false>), grid, dim3(kThreads), 0, s, a); \
         return;                                                                           \
     }
     NX_MC(7, 2) NX_MC(7, 3) NX_MC(7, 4) NX_MC(7, 5) NX_MC(7, 6) NX_MC(7, 7) NX_MC(7, 8) NX_MC(7, 9) NX_MC(7, 10)
@@ -1004,9 +1060,24 @@ bool ks_moddown_col_ok(const DeviceTables &t, uint32_t A)
     return t.max_bits <= 51 && A >= 2 && A <= kColMaxA + 1 && t.logn >= 14 && t.logn <= 17;
 }
 
+static uint32_t moddown_col_chunk(const DeviceTables &t, uint32_t polys, uint32_t lo)
+{
+    const uint32_t tiles = (1u << t.logn) / 2048u;
+    const uint32_t want = (2048u + tiles * polys - 1) / (tiles * polys);
+    uint32_t chunk = std::max((lo + want - 1) / want, std::min(4u, lo));
+    const int mode = g_moddown_col[tune_bucket(polys)].load();
+    if (mode > 0 && (mode & 255)) chunk = std::min((uint32_t)(mode & 255), lo);
+    return chunk;
+}
+
+bool ks_moddown_col_inverse(const DeviceTables &t, uint32_t polys)
+{
+    return g_moddown_col[tune_bucket(polys)].load() == 0 && (1u << t.logn) / 2048u * polys >= kInverseBlocks;
+}
+
 void ks_moddown_convert_col(const DeviceTables &t, uint64_t *z, const uint64_t *acc, uint64_t acc_stride,
                             const ulonglong2 *w, const double *convd, const uint8_t *in_primes_host, uint32_t A,
-                            uint32_t polys, uint32_t lo, uint32_t L, hipStream_t s)
+                            uint32_t polys, uint32_t lo, uint32_t L, hipStream_t s, bool inverse)
 {
     if (!ks_moddown_col_ok(t, A) || !convd) throw std::invalid_argument("ks_moddown_convert_col: unsupported parameters");
     if (lo < 1 || lo + A > (uint32_t)kMaxPrimes) throw std::invalid_argument("ks_moddown_convert_col: bad sizes");
@@ -1026,12 +1097,10 @@ void ks_moddown_convert_col(const DeviceTables &t, uint64_t *z, const uint64_t *
     int l1, l2;
     split_logn(t.logn, l1, l2);
     const uint32_t n = 1u << t.logn;
-    const int mode = g_moddown_col[tune_bucket(polys)].load();
     const uint32_t tiles = n / 2048u;
-    const uint32_t want = (2048u + tiles * polys - 1) / (tiles * polys);
-    uint32_t chunk = (lo + want - 1) / want;
-    chunk = std::max(chunk, std::min(4u, lo));
-    if (mode > 0 && (mode & 255)) chunk = std::min((uint32_t)(mode & 255), lo);
+    const uint32_t chunk = inverse ? lo : moddown_col_chunk(t, polys, lo);
+    a.invd = t.inv_d;
+    a.ninvd = t.ninv_d;
     a.chunk = chunk;
     a.chunks = (lo + chunk - 1) / chunk;
     ProfScope prof("ks_moddown_col", s,
@@ -1040,7 +1109,10 @@ void ks_moddown_convert_col(const DeviceTables &t, uint64_t *z, const uint64_t *
     const dim3 grid(tiles, polys * a.chunks);
 #define NX_MD(LOGS, AA)                                                                     \
     if (l1 == LOGS && A == AA) {                                                          \
-        hipLaunchKernelGGL((k_moddown_col<LOGS, AA>), grid, dim3(kThreads), 0, s, a);       \
+        if (inverse)                                                                      \
+            hipLaunchKernelGGL((k_moddown_col<LOGS, AA, true>), grid, dim3(kThreads), 0, s, a);  \
+        else                                                                              \
+            hipLaunchKernelGGL((k_moddown_col<LOGS, AA, false>), grid, dim3(kThreads), 0, s, a); \
         return;                                                                           \
     }
     NX_MD(7, 2) NX_MD(7, 3) NX_MD(7, 4) NX_MD(7, 5) NX_MD(7, 6) NX_MD(7, 7) NX_MD(7, 8) NX_MD(7, 9) NX_MD(7, 10)
@@ -1062,6 +1134,7 @@ void ntt_inverse(const DeviceTables &t, const NttBatch &b, hipStream_t s)
         int l1, l2;
         split_logn(t.logn, l1, l2);
         launch_pass<kRow, false>(l2, a, batch, s);
+        if (b.rows_only) return;
         a.src = nullptr;
         a.nsrcs = 0;
         launch_pass<kCol, false>(l1, a, batch, s);

@@ -270,12 +270,8 @@ void ks_out_primes(const Context &c, size_t l, uint8_t *outp)
 
 // INTT of the targets ([B][l][n], or B <= kNttSrcMax pointers) into coef
 static void ks_coefficients(Context &c, uint64_t *coef, const uint64_t *targets, const uint64_t *const *target_list,
-                            size_t B, size_t l)
+                            size_t B, size_t l, bool rows_only = false)
 {
-    if (!target_list) {
-        ntt_inv_from(c, coef, targets, B, l, l * c.n, l * c.n);
-        return;
-    }
     NttBatch b;
     b.data = coef;
     b.poly_stride = l * c.n;
@@ -283,7 +279,10 @@ static void ks_coefficients(Context &c, uint64_t *coef, const uint64_t *targets,
     b.limbs = (uint32_t)l;
     b.prime_by_poly = 0;
     for (int i = 0; i < kMaxPrimes; i++) b.prime_of[i] = (uint8_t)i;
-    b.src_list = target_list;
+    b.src = targets;
+    b.src_poly_stride = l * c.n;
+    b.src_list = targets ? nullptr : target_list;
+    b.rows_only = rows_only ? 1 : 0;
     ntt_inverse(c.tables, b, c.stream);
 }
 
@@ -374,7 +373,12 @@ void ks_inner(Context &c, uint64_t *acc, const uint64_t *targets, const uint64_t
     uint8_t outp[kMaxPrimes];
     ks_out_primes(c, l, outp);
     DevBuf coef(&c, B * l * n);
-    ks_coefficients(c, coef.get(), targets, target_list, B, l);
+    const size_t per = nout * digits * n, most = kDigitWords;
+    size_t bc = std::max<size_t>(1, std::min({B, most / per, (size_t)kMaxHoist}));
+    bc = (B + (B + bc - 1) / bc - 1) / ((B + bc - 1) / bc);  // even chunks: no short last launch
+    // several special primes, large batches: the inverse's column pass in the conversion
+    const bool inverse = c.alpha > 1 && ks_modup_col_inverse(c.tables, (uint32_t)bc, (uint32_t)l, (uint32_t)c.alpha);
+    ks_coefficients(c, coef.get(), targets, target_list, B, l, inverse);
     KsRowInner p;
     p.l = (uint32_t)l;
     p.alpha = (uint32_t)c.alpha;
@@ -384,8 +388,6 @@ void ks_inner(Context &c, uint64_t *acc, const uint64_t *targets, const uint64_t
     p.out_primes = outp;
     // chunks of inputs; one input alone is cut by output primes where a digit
     // is cheap to read again (one prime)
-    const size_t per = nout * digits * n, most = kDigitWords;
-    const size_t bc = std::max<size_t>(1, std::min({B, most / per, (size_t)kMaxHoist}));
     size_t ic = nout;
     if (c.alpha == 1 && bc == 1) ic = std::max<size_t>(1, std::min(nout, most / (digits * n)));
     const size_t parts = (nout + ic - 1) / ic;
@@ -412,7 +414,8 @@ void ks_inner(Context &c, uint64_t *acc, const uint64_t *targets, const uint64_t
                             c.stream);
             else
                 ks_modup_convert_col(c.tables, T.get(), x, c.d_modup_w, (uint32_t)cnt, (uint32_t)l,
-                                     (uint32_t)c.alpha, (uint32_t)c.key_limbs(), outp, (uint32_t)nout, c.stream, true);
+                                     (uint32_t)c.alpha, (uint32_t)c.key_limbs(), outp, (uint32_t)nout, c.stream, true,
+                                     inverse);
             ks_row_inner(c.tables, p, c.stream);
         }
     }
@@ -447,6 +450,9 @@ DevBuf ks_moddown_prepare(Context &c, uint64_t *acc, size_t B, size_t l, FwdInpu
 {
     const size_t n = c.n, L = c.L, alpha = c.alpha;
     const size_t nout = l + alpha;
+    const bool col = alpha > 1 && c.d_moddown_conv_d && ks_moddown_col_ok(c.tables, (uint32_t)alpha) &&
+                     ks_moddown_col_get((uint32_t)(2 * B)) >= 0;
+    const bool inverse = col && ks_moddown_col_inverse(c.tables, (uint32_t)(2 * B));
     // The special-prime limbs of acc are transformed in place: INTT of the
     // special limbs of every poly.
     {
@@ -457,16 +463,16 @@ DevBuf ks_moddown_prepare(Context &c, uint64_t *acc, size_t B, size_t l, FwdInpu
         b.limbs = (uint32_t)alpha;
         b.prime_by_poly = 0;
         for (int i = 0; i < kMaxPrimes; i++) b.prime_of[i] = (uint8_t)(L + (i < (int)alpha ? i : 0));
+        b.rows_only = inverse ? 1 : 0;
         ntt_inverse(c.tables, b, c.stream);
     }
     DevBuf tmp(&c, B * 2 * l * n);
-    if (alpha > 1 && c.d_moddown_conv_d && ks_moddown_col_ok(c.tables, (uint32_t)alpha) &&
-        ks_moddown_col_get((uint32_t)(2 * B)) >= 0) {
+    if (col) {
         // the centred conversion feeds the forward column pass directly
         uint8_t inp[kMaxPrimes];
         for (size_t k = 0; k < alpha; k++) inp[k] = (uint8_t)(L + k);
         ks_moddown_convert_col(c.tables, tmp.get(), acc, nout * n, c.d_moddown_w, c.d_moddown_conv_d, inp,
-                               (uint32_t)alpha, (uint32_t)(2 * B), (uint32_t)l, (uint32_t)L, c.stream);
+                               (uint32_t)alpha, (uint32_t)(2 * B), (uint32_t)l, (uint32_t)L, c.stream, inverse);
         in.rows_only = true;
         return tmp;
     }
@@ -854,6 +860,8 @@ void op_multiply_relin_rescale_fused_many(const std::vector<const Ciphertext *> 
         // limb q_(l-1) of Y = acc + P d, then (q_(l-1), p_0..p_(alpha-1)) to coefficients
         rns_add_limb_scaled(c.tables, acc.get(), nout * n, c01.get(), pw, (uint32_t)lo, c.mdr_pmod[l],
                             (uint32_t)(2 * cnt), c.stream);
+        const bool col = ks_moddown_col_ok(c.tables, (uint32_t)A) && ks_moddown_col_get((uint32_t)(2 * cnt)) >= 0;
+        const bool inverse = col && ks_moddown_col_inverse(c.tables, (uint32_t)(2 * cnt));
         {
             NttBatch nb;
             nb.data = acc.get() + lo * n;
@@ -863,17 +871,18 @@ void op_multiply_relin_rescale_fused_many(const std::vector<const Ciphertext *> 
             nb.prime_by_poly = 0;
             for (int i = 0; i < kMaxPrimes; i++)
                 nb.prime_of[i] = (uint8_t)(i == 0 ? lo : c.L + (i - 1 < (int)alpha ? i - 1 : 0));
+            nb.rows_only = inverse ? 1 : 0;
             ntt_inverse(c.tables, nb, c.stream);
         }
         DevBuf tmp(&c, cnt * 2 * lo * n);  // conversion, then the transform's first pass
         FwdInput in_tmp;
-        if (ks_moddown_col_ok(c.tables, (uint32_t)A) && ks_moddown_col_get((uint32_t)(2 * cnt)) >= 0) {
+        if (col) {
             // the conversion feeds the forward column pass directly
             uint8_t inp[kMaxPrimes];
             for (size_t k = 0; k < A; k++) inp[k] = (uint8_t)(k == 0 ? lo : c.L + k - 1);
             ks_moddown_convert_col(c.tables, tmp.get(), acc.get(), nout * n, c.d_mdr_w + l * A,
                                    c.d_mdr_conv_d + l * (A + 1) * c.L, inp, (uint32_t)A, (uint32_t)(2 * cnt),
-                                   (uint32_t)lo, (uint32_t)c.L, c.stream);
+                                   (uint32_t)lo, (uint32_t)c.L, c.stream, inverse);
             in_tmp.rows_only = true;
         } else {
             ks_moddown_rescale_convert(c.tables, tmp.get(), acc.get(), nout * n, c.d_mdr_w + l * A,
