@@ -353,17 +353,19 @@ DevBuf ks_modup(Context &c, const uint64_t *targets, size_t B, size_t l);
 DevBuf ks_modup_list(Context &c, const uint64_t *const *targets, size_t B, size_t l);
 // Whether key switches run without a stored ModUp (kernels_ks.hip).
 bool ks_rows_fused(const Context &c);
-// Inner products of the digits of B targets ([B][l][n] NTT form, or B <=
-// kNttSrcMax pointers) with keys, the digits in chunks (ks_rows_fused only):
-// acc[B][2][l+alpha][n] with the one key keys[0]; or with perms, target b
-// rotated by perms[b] under keys[b] and summed into acc[2][l+alpha][n] (added
-// to it with accumulate).  aseeds as KSwitchKeys::seeds_of, one per key.
-void ks_inner(Context &c, uint64_t *acc, const uint64_t *targets, const uint64_t *const *target_list, size_t B,
-              size_t l, const uint64_t *const *keys, const uint64_t *const *aseeds, const uint32_t *const *perms,
-              bool accumulate);
-// acc[B][2][l+alpha][n]: the same with one key, on any ring
+// acc[B][2][l+alpha][n]: inner products of the digits of B targets ([B][l][n]
+// NTT form) with one key.  aseed as KSwitchKeys::seeds_of.
 void ks_inner_one_key(Context &c, uint64_t *acc, const uint64_t *targets, size_t B, size_t l, const DevBuf &key,
                       const uint64_t *aseed);
+// acc[sum][2][l+alpha][n] for every sum that `in` names (inputs of one sum side
+// by side): the sum over its inputs of the inner products of their digits,
+// rotated by perm, with their keys.
+struct KsRotated {
+    const uint64_t *target, *key, *aseed;  // target: [l][n] NTT form; aseed as KSwitchKeys::seeds_of
+    const uint32_t *perm;
+    uint32_t sum;
+};
+void ks_inner_sums(Context &c, uint64_t *acc, const std::vector<KsRotated> &in, size_t l);
 // ModDown up to the forward transform: INTT of the special limbs of acc
 // [B][2][l+alpha][n] in place and the conversion, as far as it is not part of
 // the transform; returns tmp [B][2][l][n], and in `in` what the caller's forward

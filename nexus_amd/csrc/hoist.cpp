@@ -180,20 +180,13 @@ void op_rotate_sum_many(const std::vector<std::vector<const Ciphertext *>> &grou
     const Ciphertext &a0 = *groups[0].at(0);
     check_input(a0, gk);
     Context &c = *a0.ctx;
-    const size_t n = c.n, l = a0.limbs, nout = l + c.alpha, pw = l * n, digits = c.digits(l);
+    const size_t n = c.n, l = a0.limbs, nout = l + c.alpha, pw = l * n;
     const size_t G = groups.size();
     DevBuf outs(&c, G * 2 * pw), acc(&c, G * 2 * nout * n);
-    uint8_t outp[kMaxPrimes];
-    ks_out_primes(c, l, outp);
-    // the switched inputs of every group, in group order: their ModUps run in
-    // chunks of up to kMaxHoist inputs across group boundaries, and each group's
-    // inner products read its inputs' digits from the chunks that hold them
-    struct Sw {
-        size_t g;
-        const uint64_t *key, *seed, *c1;
-        const uint32_t *perm;
-    };
-    std::vector<Sw> sw;
+    // the switched inputs of every group, in group order: their key switches run
+    // together, in chunks across group boundaries (ks_inner_sums)
+    std::vector<KsRotated> sw;
+    std::vector<char> switched(G, 0);
     for (size_t g = 0; g < G; g++) {
         const auto &in = groups[g];
         require(!in.empty() && in.size() == steps[g].size(), "inputs and steps must match");
@@ -211,7 +204,8 @@ void op_rotate_sum_many(const std::vector<std::vector<const Ciphertext *>> &grou
             Prepared p = prepare(c, std::vector<int>{steps[g][i]}, gk);
             tally("ks_hoisted", l);
             perms.push_back(p.perms[0]);
-            sw.push_back({g, p.keys[0], p.seeds[0], in[i]->data.get() + pw, p.perms[0]});
+            sw.push_back({in[i]->data.get() + pw, p.keys[0], p.seeds[0], p.perms[0], (uint32_t)g});
+            switched[g] = 1;
         }
         uint64_t *og = outs.get() + g * 2 * pw;
         DevBuf part;
@@ -222,39 +216,9 @@ void op_rotate_sum_many(const std::vector<std::vector<const Ciphertext *>> &grou
             if (base) poly_add(c.tables, og, og, o, 2, (uint32_t)l, c.stream);
         }
     }
-    std::vector<char> started(G, 0);
-    const bool fused = ks_rows_fused(c);
-    for (size_t base = 0; base < sw.size(); base += kMaxHoist) {
-        const size_t cnt = std::min<size_t>(kMaxHoist, sw.size() - base);
-        std::vector<const uint64_t *> c1s(cnt);
-        for (size_t r = 0; r < cnt; r++) c1s[r] = sw[base + r].c1;
-        DevBuf T;
-        if (!fused) T = ks_modup_list(c, c1s.data(), cnt, l);
-        for (size_t r0 = 0; r0 < cnt;) {
-            const size_t g = sw[base + r0].g;
-            size_t r1 = r0;
-            while (r1 < cnt && sw[base + r1].g == g) r1++;
-            std::vector<const uint64_t *> keys, seeds;
-            std::vector<const uint32_t *> rperms;
-            for (size_t r = r0; r < r1; r++) {
-                keys.push_back(sw[base + r].key);
-                seeds.push_back(sw[base + r].seed);
-                rperms.push_back(sw[base + r].perm);
-            }
-            if (fused)
-                ks_inner(c, acc.get() + g * 2 * nout * n, nullptr, c1s.data() + r0, r1 - r0, l, keys.data(),
-                         seeds.data(), rperms.data(), started[g] != 0);
-            else
-                ks_inner_product_rot_sum(c.tables, acc.get() + g * 2 * nout * n, T.get() + r0 * nout * digits * n,
-                                         keys.data(), rperms.data(), (uint32_t)(r1 - r0), (uint32_t)digits,
-                                         (uint32_t)c.key_limbs(), outp, (uint32_t)nout, started[g] != 0, c.stream,
-                                         nout * digits * n, seeds.data());
-            started[g] = 1;
-            r0 = r1;
-        }
-    }
+    ks_inner_sums(c, acc.get(), sw, l);
     for (size_t g = 0; g < G; g++)
-        if (!started[g]) {
+        if (!switched[g]) {
             // no switched term: a zero accumulator leaves the base unchanged
             std::vector<uint64_t> zeros(nout, 0);
             poly_fill_limbs(acc.get() + g * 2 * nout * n, zeros.data(), 2, (uint32_t)nout, c.logn, c.stream);
@@ -333,7 +297,7 @@ void op_rotate_sum(const std::vector<const Ciphertext *> &in, const std::vector<
     const Ciphertext &a0 = *in[0];
     check_input(a0, gk);
     Context &c = *a0.ctx;
-    const size_t n = c.n, l = a0.limbs, nout = l + c.alpha, pw = l * n, digits = c.digits(l);
+    const size_t n = c.n, l = a0.limbs, nout = l + c.alpha, pw = l * n;
     for (const Ciphertext *a : in) {
         check_input(*a, gk);
         require(a->ctx == &c && a->limbs == l, "inputs must share the level");
@@ -347,8 +311,9 @@ void op_rotate_sum(const std::vector<const Ciphertext *> &in, const std::vector<
     out.ntt = true;
     out.data.reset(&c, 2 * pw);
     // data-basis part: sigma_i(c0_i), and (c0, c1) of the identity terms
-    std::vector<const uint64_t *> ins, c1s, keys, seeds;
-    std::vector<const uint32_t *> perms, rperms;
+    std::vector<const uint64_t *> ins;
+    std::vector<const uint32_t *> perms;
+    std::vector<KsRotated> sw;
     for (size_t i = 0; i < in.size(); i++) {
         ins.push_back(in[i]->data.get());
         if (steps[i] == 0) {
@@ -358,10 +323,7 @@ void op_rotate_sum(const std::vector<const Ciphertext *> &in, const std::vector<
         Prepared p = prepare(c, std::vector<int>{steps[i]}, gk);
         tally("ks_hoisted", l);
         perms.push_back(p.perms[0]);
-        rperms.push_back(p.perms[0]);
-        keys.push_back(p.keys[0]);
-        seeds.push_back(p.seeds[0]);
-        c1s.push_back(in[i]->data.get() + pw);
+        sw.push_back({in[i]->data.get() + pw, p.keys[0], p.seeds[0], p.perms[0], 0});
     }
     {
         DevBuf part;
@@ -372,22 +334,9 @@ void op_rotate_sum(const std::vector<const Ciphertext *> &in, const std::vector<
             if (base) poly_add(c.tables, out.data.get(), out.data.get(), o, 2, (uint32_t)l, c.stream);
         }
     }
-    if (!keys.empty()) {
-        uint8_t outp[kMaxPrimes];
-        ks_out_primes(c, l, outp);
+    if (!sw.empty()) {
         DevBuf acc(&c, 2 * nout * n);
-        for (size_t base = 0; base < keys.size(); base += kMaxHoist) {
-            const size_t cnt = std::min<size_t>(kMaxHoist, keys.size() - base);
-            if (ks_rows_fused(c)) {
-                ks_inner(c, acc.get(), nullptr, c1s.data() + base, cnt, l, keys.data() + base, seeds.data() + base,
-                         rperms.data() + base, base > 0);
-                continue;
-            }
-            DevBuf T = ks_modup_list(c, c1s.data() + base, cnt, l);
-            ks_inner_product_rot_sum(c.tables, acc.get(), T.get(), keys.data() + base, rperms.data() + base,
-                                     (uint32_t)cnt, (uint32_t)digits, (uint32_t)c.key_limbs(), outp, (uint32_t)nout,
-                                     base > 0, c.stream, nout * digits * n, seeds.data() + base);
-        }
+        ks_inner_sums(c, acc.get(), sw, l);
         ks_moddown(c, out.data.get(), acc.get(), 1, l, false);
     }
     dst = std::move(out);

@@ -255,25 +255,25 @@ void ks_modup_convert_col(const DeviceTables &t, uint64_t *T, const uint64_t *co
 // being left to ks_modup_convert_col (raw and inverse set)
 bool ks_modup_col_inverse(const DeviceTables &t, uint32_t B, uint32_t l, uint32_t alpha);
 // The digits of a key switch from the column pass to the inner product
-// (kernels_ks.hip): T[b][I - i0][j] for the output primes i0 .. i0 + icount - 1
-// outside digit j holds column-transformed values as ks_row_inner reads them
-// (doubles below 2^51, lazily reduced words above), written by ks_lift_col
-// (one special prime) or ks_modup_convert_col with raw set (i0 = 0, icount =
-// nout).  ks_row_inner runs the row pass and multiplies by the keys.
+// (kernels_ks.hip): T[b][I][j] for the output primes I outside digit j holds
+// column-transformed values as ks_row_inner reads them (doubles below 2^51,
+// lazily reduced words above), written by ks_lift_col (one special prime) or
+// ks_modup_convert_col with raw set.  ks_row_inner runs the row pass and
+// multiplies by the keys.
 bool ks_row_inner_ok(const DeviceTables &t, uint32_t alpha);
-void ks_lift_col(const DeviceTables &t, uint64_t *T, const uint64_t *coef, uint32_t B, uint32_t l, uint32_t i0,
-                 uint32_t icount, const uint8_t *out_primes_host, uint32_t nout, hipStream_t s);
+void ks_lift_col(const DeviceTables &t, uint64_t *T, const uint64_t *coef, uint32_t B, uint32_t l,
+                 const uint8_t *out_primes_host, uint32_t nout, hipStream_t s);
 struct KsRowInner {
-    uint64_t *acc = nullptr;       // [count][2][nout][n], or [2][nout][n] for a sum of rotations
-    const uint64_t *T = nullptr;   // [count][icount][digits][n], t_stride words per input
-    uint64_t t_stride = 0;
+    uint64_t *acc = nullptr;       // [count][2][nout][n], or [sum][2][nout][n] for sums of rotations
+    const uint64_t *T = nullptr;   // [count][nout][digits][n]
     const uint64_t *own = nullptr;             // the inputs in NTT form, [count][l][n] ...
     const uint64_t *const *own_list = nullptr; // ... or a pointer each (count <= kMaxHoist)
     const uint64_t *const *keys = nullptr;     // one key, or one per rotation
     const uint64_t *const *aseeds = nullptr;   // per key: its uniform half's digit seeds, or null
-    const uint32_t *const *perms = nullptr;    // set: acc (+)= the sum over the inputs of their rotations
-    uint32_t count = 0, l = 0, alpha = 0, digits = 0, nout = 0, i0 = 0, icount = 0, key_limbs = 0;
-    bool accumulate = false;       // sums of rotations: add to acc
+    const uint32_t *const *perms = nullptr;    // set: input i is rotated by perms[i] ...
+    const uint32_t *sum = nullptr;             // ... and belongs to acc[sum[i]], inputs of one sum side by side
+    uint32_t count = 0, l = 0, alpha = 0, digits = 0, nout = 0, key_limbs = 0;
+    bool accumulate = false;       // rotations: the first input's sum is added to acc
     const uint8_t *out_primes = nullptr;
 };
 void ks_row_inner(const DeviceTables &t, const KsRowInner &p, hipStream_t s);

@@ -28,13 +28,13 @@ namespace {
 // ---- lift of one-prime digits (one special prime) in the column pass
 
 struct LiftColArgs {
-    uint64_t *T;           // [B][icount][l][n]
+    uint64_t *T;           // [B][nout][l][n]
     const uint64_t *coef;  // [B][l][n]
     const ulonglong2 *tw;
     const double *twd;
     const ModConst *mod;
     const double2 *qd;
-    uint32_t l, i0, icount, logn, chunk, chunks, listed;
+    uint32_t l, nout, logn, chunk, chunks, listed;
     uint32_t list[kMaxPrimes];  // the output primes I of this launch
     uint32_t outp[kMaxPrimes];
 };
@@ -92,7 +92,7 @@ __global__ __launch_bounds__(kThreads, INT ? 2 : 4) void k_lift_col(LiftColArgs 
         const uint32_t I = a.list[r];
         if (I == j) continue;  // the input's own limb
         const uint32_t kp = a.outp[I];
-        uint64_t *out = a.T + (((uint64_t)b * a.icount + I - a.i0) * a.l + j) * n;
+        uint64_t *out = a.T + (((uint64_t)b * a.nout + I) * a.l + j) * n;
         if constexpr (INT) {
             const ModConst m = table_mod(a.mod, kp);
 #pragma unroll
@@ -124,9 +124,8 @@ __global__ __launch_bounds__(kThreads, INT ? 2 : 4) void k_lift_col(LiftColArgs 
 // ---- row pass and inner product
 
 struct RowInnerArgs {
-    uint64_t *acc;          // [B][2][nout][n] ([2][nout][n] for a sum of rotations)
-    const uint64_t *T;      // [B][icount][digits][n]
-    uint64_t t_stride;      // words per input of T
+    uint64_t *acc;          // [B][2][nout][n] (sums of rotations: [sum[s]][2][nout][n])
+    const uint64_t *T;      // [inputs][nout][digits][n]
     const uint64_t *own;    // the inputs in NTT form: [B][l][n], or ownp[b]
     const uint64_t *ownp[kMaxHoist];
     const uint64_t *key[kMaxHoist];    // per rotation; key[0] without rotations
@@ -136,7 +135,10 @@ struct RowInnerArgs {
     const double *twd;
     const ModConst *mod;
     const double2 *qd;
-    uint32_t B, l, alpha, digits, nout, i0, key_limbs, logn, log_cw, accumulate;
+    uint32_t B, l, alpha, digits, nout, key_limbs, logn, log_cw;  // B: inputs, or sums of rotations
+    uint32_t accumulate;           // the first sum is added to acc
+    uint32_t sum[kMaxHoist];       // sum b: its index in acc and inputs first[b] .. first[b + 1] - 1
+    uint8_t first[kMaxHoist + 1];
     uint32_t outp[kMaxPrimes];
 };
 
@@ -289,9 +291,9 @@ __device__ __forceinline__ void store_row(const uint64_t *v, uint64_t *row, int 
         *reinterpret_cast<ulonglong2 *>(row + P::out(o, k)) = make_ulonglong2(v[k], v[k + 1]);
 }
 
-// acc[b][k][I] = sum_j NTT(digit j)[I] key[j][k][I] (ROT: acc[k][I] (+)= the
-// sum over the rotations r of sigma_r(NTT(digit j of input r))[I] key_r[j][k][I]).
-// Workgroup: one output prime I (and input b), four waves, each of
+// acc[b][k][I] = sum_j NTT(digit j)[I] key[j][k][I] (ROT: acc[b][k][I] (+)= the
+// sum over the rotations r of sum b of sigma_r(NTT(digit j of input r))[I] key_r[j][k][I]).
+// Workgroup: one output prime I and input or sum b, four waves, each of
 // which owns its rows for the whole sum.  The automorphism maps rows onto rows (row and
 // position in the row are the low and high bits of the bit-reversed exponent,
 // and exponents are multiplied by an odd number), so a wave transforms the
@@ -307,10 +309,9 @@ __global__ __launch_bounds__(kThreads) void k_row_inner(RowInnerArgs a)
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const int cc = (int)lane / P::LPR, o = (int)lane % P::LPR;
     uint64_t *wlds = words + wave * P::LDS + cc * P::SP;
-    // neighbours in y: the same output prime of consecutive inputs, whose key
-    // words are then in this XCD's L2
-    const uint32_t r = ROT ? blockIdx.y : blockIdx.y / a.B, b = ROT ? 0u : blockIdx.y - r * a.B;
-    const uint32_t I = a.i0 + r;
+    // neighbours in y: the same output prime of consecutive inputs or sums, whose
+    // key words are then in this XCD's L2
+    const uint32_t I = blockIdx.y / a.B, b = blockIdx.y - I * a.B;
     const uint32_t kp = a.outp[I];
     const uint32_t row = (blockIdx.x * (kThreads / 64) + wave) * P::ROWS + cc;
     const uint64_t base = (uint64_t)row * P::S;
@@ -318,9 +319,10 @@ __global__ __launch_bounds__(kThreads) void k_row_inner(RowInnerArgs a)
     const uint64_t kstride = (uint64_t)a.key_limbs * n;
     const uint64_t koff = (uint64_t)kp * n + base;
     const uint32_t own_digit = I < a.l ? I / a.alpha : ~0u;
-    uint64_t *out = a.acc + (uint64_t)b * 2 * a.nout * n + (uint64_t)I * n + base;
+    uint64_t *out = a.acc + (uint64_t)(ROT ? a.sum[b] : b) * 2 * a.nout * n + (uint64_t)I * n + base;
     const uint64_t poly1 = (uint64_t)a.nout * n;
-    const uint32_t count = ROT ? a.B : 1u;
+    const uint32_t begin = ROT ? a.first[b] : b, end = ROT ? a.first[b + 1] : b + 1;
+    const bool accumulate = ROT && a.accumulate && b == 0;
 
     if (m.q < kFpPrimeBound) {
         const double q = a.qd[kp].x, qinv = a.qd[kp].y;
@@ -336,7 +338,7 @@ __global__ __launch_bounds__(kThreads) void k_row_inner(RowInnerArgs a)
             s0[k].start(M);
             s1[k].start(M);
         }
-        if (ROT && a.accumulate) {
+        if (accumulate) {
             uint64_t v0[W], v1[W];
             load_row<LOGS>(v0, out, o);
             load_row<LOGS>(v1, out + poly1, o);
@@ -354,10 +356,9 @@ __global__ __launch_bounds__(kThreads) void k_row_inner(RowInnerArgs a)
         RowTwiddles<LOGS> w;
         if (!ROT) w.load(tw, N1 + row, o);
         uint32_t left = terms;
-        for (uint32_t i = 0; i < count; i++) {
-            const uint32_t in = ROT ? i : b;
-            const uint64_t *t0 = a.T + in * a.t_stride + (uint64_t)r * a.digits * n;
-            const uint64_t *own = (a.own ? a.own + (uint64_t)in * a.l * n : a.ownp[in]) + (uint64_t)I * n;
+        for (uint32_t i = begin; i < end; i++) {
+            const uint64_t *t0 = a.T + ((uint64_t)i * a.nout + I) * a.digits * n;
+            const uint64_t *own = (a.own ? a.own + (uint64_t)i * a.l * n : a.ownp[i]) + (uint64_t)I * n;
             const uint64_t *key = a.key[ROT ? i : 0] + koff;
             const uint64_t *seed = a.aseed[ROT ? i : 0];
             uint32_t src[W];
@@ -464,15 +465,14 @@ __global__ __launch_bounds__(kThreads) void k_row_inner(RowInnerArgs a)
     // between two reductions
     const ulonglong2 *tw = a.tw + (uint64_t)kp * n;
     uint64_t lo0[W] = {}, hi0[W] = {}, lo1[W] = {}, hi1[W] = {};
-    if (ROT && a.accumulate) {
+    if (accumulate) {
         load_row<LOGS>(lo0, out, o);
         load_row<LOGS>(lo1, out + poly1, o);
     }
     uint32_t sum = 1;
-    for (uint32_t i = 0; i < count; i++) {
-        const uint32_t in = ROT ? i : b;
-        const uint64_t *t0 = a.T + in * a.t_stride + (uint64_t)r * a.digits * n;
-        const uint64_t *own = (a.own ? a.own + (uint64_t)in * a.l * n : a.ownp[in]) + (uint64_t)I * n;
+    for (uint32_t i = begin; i < end; i++) {
+        const uint64_t *t0 = a.T + ((uint64_t)i * a.nout + I) * a.digits * n;
+        const uint64_t *own = (a.own ? a.own + (uint64_t)i * a.l * n : a.ownp[i]) + (uint64_t)I * n;
         const uint64_t *key = a.key[ROT ? i : 0] + koff;
         const uint64_t *seed = a.aseed[ROT ? i : 0];
         uint32_t src[W];
@@ -559,10 +559,10 @@ bool ks_row_inner_ok(const DeviceTables &t, uint32_t alpha)
     return t.logn >= 14 && t.logn <= 17 && t.max_bits <= 61 && (alpha == 1 || ks_modup_col_ok(t, alpha));
 }
 
-void ks_lift_col(const DeviceTables &t, uint64_t *T, const uint64_t *coef, uint32_t B, uint32_t l, uint32_t i0,
-                 uint32_t icount, const uint8_t *out_primes_host, uint32_t nout, hipStream_t s)
+void ks_lift_col(const DeviceTables &t, uint64_t *T, const uint64_t *coef, uint32_t B, uint32_t l,
+                 const uint8_t *out_primes_host, uint32_t nout, hipStream_t s)
 {
-    if (t.logn < 14 || t.logn > 17 || nout > (uint32_t)kMaxPrimes || i0 + icount > nout || !icount || !l || !B)
+    if (t.logn < 14 || t.logn > 17 || nout > (uint32_t)kMaxPrimes || !nout || !l || !B)
         throw std::invalid_argument("ks_lift_col: unsupported parameters");
     LiftColArgs a;
     a.T = T;
@@ -572,16 +572,15 @@ void ks_lift_col(const DeviceTables &t, uint64_t *T, const uint64_t *coef, uint3
     a.mod = t.mod;
     a.qd = t.qd;
     a.l = l;
-    a.i0 = i0;
-    a.icount = icount;
+    a.nout = nout;
     a.logn = (uint32_t)t.logn;
     for (int i = 0; i < kMaxPrimes; i++) a.outp[i] = i < (int)nout ? out_primes_host[i] : 0;
     const int l1 = t.logn / 2;
     const uint32_t n = 1u << t.logn, tiles = n / 2048;
-    ProfScope prof("ks_lift_col", s, 8.0 * n * B * l * (1.0 + icount) + 8.0 * (double)(1u << l1) * B * l * icount);
+    ProfScope prof("ks_lift_col", s, 8.0 * n * B * l * (1.0 + nout) + 8.0 * (double)(1u << l1) * B * l * nout);
     for (int wide = 0; wide < 2; wide++) {  // primes below 2^51, then the others
         a.listed = 0;
-        for (uint32_t I = i0; I < i0 + icount; I++)
+        for (uint32_t I = 0; I < nout; I++)
             if ((t.mod_host[out_primes_host[I]] >= kFpPrimeBound) == (wide != 0)) a.list[a.listed++] = I;
         if (!a.listed) continue;
         // outputs per workgroup: enough workgroups to fill the device, at least 4
@@ -604,13 +603,12 @@ void ks_lift_col(const DeviceTables &t, uint64_t *T, const uint64_t *coef, uint3
 void ks_row_inner(const DeviceTables &t, const KsRowInner &p, hipStream_t s)
 {
     const bool rot = p.perms != nullptr;
-    if (!p.count || (rot && p.count > (uint32_t)kMaxHoist) || (p.own_list && p.count > (uint32_t)kMaxHoist) ||
-        p.nout > (uint32_t)kMaxPrimes || p.i0 + p.icount > p.nout || t.logn < 14 || t.logn > 17)
+    if (!p.count || (rot && (p.count > (uint32_t)kMaxHoist || !p.sum)) ||
+        (p.own_list && p.count > (uint32_t)kMaxHoist) || p.nout > (uint32_t)kMaxPrimes || t.logn < 14 || t.logn > 17)
         throw std::invalid_argument("ks_row_inner: unsupported parameters");
     RowInnerArgs a;
     a.acc = p.acc;
     a.T = p.T;
-    a.t_stride = p.t_stride;
     a.own = p.own_list ? nullptr : p.own;
     bool seeded = true;
     for (uint32_t i = 0; i < (uint32_t)kMaxHoist; i++) {
@@ -623,27 +621,40 @@ void ks_row_inner(const DeviceTables &t, const KsRowInner &p, hipStream_t s)
         a.perm[i] = on && rot ? p.perms[i] : nullptr;
         seeded = seeded && (!on || a.aseed[i]);  // a key without seeds (uploaded): all are read in full
     }
+    // runs of inputs of one sum
+    a.B = rot ? 0 : p.count;
+    a.accumulate = 0;
+    for (uint32_t i = 0; i < (uint32_t)kMaxHoist; i++) {
+        a.sum[i] = 0;
+        a.first[i] = 0;
+    }
+    if (rot) {
+        for (uint32_t i = 0; i < p.count; i++) {
+            if (i && p.sum[i] == p.sum[i - 1]) continue;
+            a.first[a.B] = (uint8_t)i;
+            a.sum[a.B++] = p.sum[i];
+        }
+        a.accumulate = p.accumulate ? 1u : 0u;
+    }
+    a.first[rot ? a.B : 0] = (uint8_t)(rot ? p.count : 0);
     a.tw = t.fwd;
     a.twd = t.fwd_d;
     a.mod = t.mod;
     a.qd = t.qd;
-    a.B = p.count;
     a.l = p.l;
     a.alpha = p.alpha;
     a.digits = p.digits;
     a.nout = p.nout;
-    a.i0 = p.i0;
     a.key_limbs = p.key_limbs;
     a.logn = (uint32_t)t.logn;
     a.log_cw = 11u - (uint32_t)(t.logn / 2);  // ColTile: 2048 words a tile
-    a.accumulate = p.accumulate ? 1 : 0;
     for (int i = 0; i < kMaxPrimes; i++) a.outp[i] = i < (int)p.nout ? p.out_primes[i] : 0;
     const uint32_t n = 1u << t.logn;
     const int l2 = t.logn - t.logn / 2;
     ProfScope prof(rot ? "ks_row_inner_rot" : "ks_row_inner", s,
-                   (double)n * p.icount *
-                       ((8.0 + (seeded ? 8.0 : 16.0)) * p.count * p.digits + (rot ? 16.0 + 4.0 * p.count : 16.0 * p.count)));
-    const dim3 grid(n / (l2 == 9 ? 2048 : 1024), rot ? p.icount : p.icount * p.count);
+                   (double)n * p.nout *
+                       ((8.0 + (seeded ? 8.0 : 16.0)) * p.count * p.digits + 16.0 * a.B + (rot ? 4.0 * p.count : 0.0)));
+    const dim3 grid(n / (l2 == 9 ? 2048 : 1024), p.nout * a.B);
 #define NX_RI(L)                                                                             \
     if (l2 == L) {                                                                         \
         if (rot && seeded)                                                                 \

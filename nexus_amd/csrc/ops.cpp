@@ -365,75 +365,134 @@ bool ks_rows_fused(const Context &c) { return ks_row_inner_ok(c.tables, (uint32_
 // shorter launches leave more of the device idle at their ends.
 constexpr size_t kDigitWords = (size_t)1 << 28;
 
-void ks_inner(Context &c, uint64_t *acc, const uint64_t *targets, const uint64_t *const *target_list, size_t B,
-              size_t l, const uint64_t *const *keys, const uint64_t *const *aseeds, const uint32_t *const *perms,
-              bool accumulate)
+// Inputs a launch takes of B: as many as kDigitWords and the argument arrays
+// hold, in even chunks (no short last launch).
+static size_t ks_inner_chunk(const Context &c, size_t B, size_t l)
 {
-    const size_t n = c.n, nout = l + c.alpha, digits = c.digits(l);
-    uint8_t outp[kMaxPrimes];
-    ks_out_primes(c, l, outp);
-    DevBuf coef(&c, B * l * n);
-    const size_t per = nout * digits * n, most = kDigitWords;
-    size_t bc = std::max<size_t>(1, std::min({B, most / per, (size_t)kMaxHoist}));
-    bc = (B + (B + bc - 1) / bc - 1) / ((B + bc - 1) / bc);  // even chunks: no short last launch
-    // several special primes, large batches: the inverse's column pass in the conversion
-    const bool inverse = c.alpha > 1 && ks_modup_col_inverse(c.tables, (uint32_t)bc, (uint32_t)l, (uint32_t)c.alpha);
-    ks_coefficients(c, coef.get(), targets, target_list, B, l, inverse);
+    const size_t per = (l + c.alpha) * c.digits(l) * c.n;
+    const size_t most = std::max<size_t>(1, std::min(kDigitWords / per, (size_t)kMaxHoist));
+    const size_t chunks = (B + most - 1) / most;
+    return (B + chunks - 1) / chunks;
+}
+
+static KsRowInner ks_row_args(const Context &c, size_t l, const uint8_t *outp)
+{
     KsRowInner p;
     p.l = (uint32_t)l;
     p.alpha = (uint32_t)c.alpha;
-    p.digits = (uint32_t)digits;
-    p.nout = (uint32_t)nout;
+    p.digits = (uint32_t)c.digits(l);
+    p.nout = (uint32_t)(l + c.alpha);
     p.key_limbs = (uint32_t)c.key_limbs();
     p.out_primes = outp;
-    // chunks of inputs; one input alone is cut by output primes where a digit
-    // is cheap to read again (one prime)
-    size_t ic = nout;
-    if (c.alpha == 1 && bc == 1) ic = std::max<size_t>(1, std::min(nout, most / (digits * n)));
-    const size_t parts = (nout + ic - 1) / ic;
-    ic = (nout + parts - 1) / parts;
-    DevBuf T(&c, bc * ic * digits * n);
-    for (size_t b0 = 0; b0 < B; b0 += bc) {
-        const size_t cnt = std::min(bc, B - b0);
-        const uint64_t *x = coef.get() + b0 * l * n;
-        p.T = T.get();
-        p.count = (uint32_t)cnt;
-        p.own = targets ? targets + b0 * l * n : nullptr;
-        p.own_list = target_list ? target_list + b0 : nullptr;
-        p.keys = perms ? keys + b0 : keys;
-        p.aseeds = perms ? aseeds + b0 : aseeds;
-        p.perms = perms ? perms + b0 : nullptr;
-        p.acc = perms ? acc : acc + b0 * 2 * nout * n;
-        p.accumulate = perms && (accumulate || b0);
-        for (size_t i0 = 0; i0 < nout; i0 += ic) {
-            p.i0 = (uint32_t)i0;
-            p.icount = (uint32_t)std::min(ic, nout - i0);
-            p.t_stride = p.icount * digits * n;
-            if (c.alpha == 1)
-                ks_lift_col(c.tables, T.get(), x, (uint32_t)cnt, (uint32_t)l, p.i0, p.icount, outp, (uint32_t)nout,
-                            c.stream);
-            else
-                ks_modup_convert_col(c.tables, T.get(), x, c.d_modup_w, (uint32_t)cnt, (uint32_t)l,
-                                     (uint32_t)c.alpha, (uint32_t)c.key_limbs(), outp, (uint32_t)nout, c.stream, true,
-                                     inverse);
-            ks_row_inner(c.tables, p, c.stream);
-        }
-    }
+    return p;
+}
+
+// one chunk: digits of p.count inputs (coef as ks_coefficients left it) into T,
+// then the inner products
+static void ks_inner_run(Context &c, KsRowInner &p, uint64_t *T, const uint64_t *coef, bool inverse)
+{
+    if (c.alpha == 1)
+        ks_lift_col(c.tables, T, coef, p.count, p.l, p.out_primes, p.nout, c.stream);
+    else
+        ks_modup_convert_col(c.tables, T, coef, c.d_modup_w, p.count, p.l, p.alpha, p.key_limbs, p.out_primes, p.nout,
+                             c.stream, true, inverse);
+    p.T = T;
+    ks_row_inner(c.tables, p, c.stream);
+}
+
+// several special primes, large batches: the inverse's column pass in the conversion
+static bool ks_inner_inverse(const Context &c, size_t count, size_t l)
+{
+    return c.alpha > 1 && ks_modup_col_inverse(c.tables, (uint32_t)count, (uint32_t)l, (uint32_t)c.alpha);
 }
 
 void ks_inner_one_key(Context &c, uint64_t *acc, const uint64_t *targets, size_t B, size_t l, const DevBuf &key,
                       const uint64_t *aseed)
 {
-    if (ks_rows_fused(c)) {
-        const uint64_t *k = key.get();
-        ks_inner(c, acc, targets, nullptr, B, l, &k, &aseed, nullptr, false);
-        return;
-    }
+    const size_t n = c.n, nout = l + c.alpha, digits = c.digits(l);
     uint8_t outp[kMaxPrimes];
     ks_out_primes(c, l, outp);
-    DevBuf T = ks_modup(c, targets, B, l);
-    ks_inner_product(c.tables, acc, T.get(), key.get(), (uint32_t)B, (uint32_t)c.digits(l), (uint32_t)c.key_limbs(),
-                     outp, (uint32_t)(l + c.alpha), c.stream, aseed);
+    if (!ks_rows_fused(c)) {
+        DevBuf T = ks_modup(c, targets, B, l);
+        ks_inner_product(c.tables, acc, T.get(), key.get(), (uint32_t)B, (uint32_t)digits, (uint32_t)c.key_limbs(),
+                         outp, (uint32_t)nout, c.stream, aseed);
+        return;
+    }
+    const size_t bc = ks_inner_chunk(c, B, l);
+    const bool inverse = ks_inner_inverse(c, bc, l);
+    DevBuf coef(&c, B * l * n), T(&c, bc * nout * digits * n);
+    ks_coefficients(c, coef.get(), targets, nullptr, B, l, inverse);
+    const uint64_t *k = key.get();
+    KsRowInner p = ks_row_args(c, l, outp);
+    p.keys = &k;
+    p.aseeds = &aseed;
+    for (size_t b0 = 0; b0 < B; b0 += bc) {
+        p.count = (uint32_t)std::min(bc, B - b0);
+        p.own = targets + b0 * l * n;
+        p.acc = acc + b0 * 2 * nout * n;
+        ks_inner_run(c, p, T.get(), coef.get() + b0 * l * n, inverse);
+    }
+}
+
+// The inputs of all sums go through the conversions and one row launch together,
+// chunks cut wherever they fall: a sum that two chunks share is added to.  Each
+// sum by itself leaves the device idle where sums are short (20 limbs at N =
+// 2^16, eight special primes: 96 sums of one input 12.9 ms, together 10.0; 24 of
+// eight 11.2 and 10.0; nine limbs at 2^14 with one special prime: 7.2 and 2.2,
+// 5.9 and 3.2).
+void ks_inner_sums(Context &c, uint64_t *acc, const std::vector<KsRotated> &in, size_t l)
+{
+    if (in.empty()) return;
+    const size_t n = c.n, nout = l + c.alpha, digits = c.digits(l);
+    uint8_t outp[kMaxPrimes];
+    ks_out_primes(c, l, outp);
+    const bool fused = ks_rows_fused(c);
+    const size_t bc = fused ? ks_inner_chunk(c, in.size(), l) : std::min(in.size(), (size_t)kMaxHoist);
+    const bool inverse = fused && ks_inner_inverse(c, bc, l);
+    DevBuf coef, T;
+    if (fused) {
+        coef.reset(&c, bc * l * n);
+        T.reset(&c, bc * nout * digits * n);
+    }
+    for (size_t b0 = 0; b0 < in.size(); b0 += bc) {
+        const size_t cnt = std::min(bc, in.size() - b0);
+        std::vector<const uint64_t *> targets(cnt), keys(cnt), seeds(cnt);
+        std::vector<const uint32_t *> perms(cnt);
+        std::vector<uint32_t> sum(cnt);
+        for (size_t r = 0; r < cnt; r++) {
+            const KsRotated &x = in[b0 + r];
+            targets[r] = x.target;
+            keys[r] = x.key;
+            seeds[r] = x.aseed;
+            perms[r] = x.perm;
+            sum[r] = x.sum;
+        }
+        const bool accumulate = b0 && in[b0 - 1].sum == in[b0].sum;
+        if (fused) {
+            ks_coefficients(c, coef.get(), nullptr, targets.data(), cnt, l, inverse);
+            KsRowInner p = ks_row_args(c, l, outp);
+            p.count = (uint32_t)cnt;
+            p.acc = acc;
+            p.own_list = targets.data();
+            p.keys = keys.data();
+            p.aseeds = seeds.data();
+            p.perms = perms.data();
+            p.sum = sum.data();
+            p.accumulate = accumulate;
+            ks_inner_run(c, p, T.get(), coef.get(), inverse);
+            continue;
+        }
+        // one ModUp for the chunk, then each sum's inner products from its digits
+        DevBuf digit = ks_modup_list(c, targets.data(), cnt, l);
+        for (size_t r0 = 0, r1; r0 < cnt; r0 = r1) {
+            for (r1 = r0 + 1; r1 < cnt && sum[r1] == sum[r0];) r1++;
+            ks_inner_product_rot_sum(c.tables, acc + (size_t)sum[r0] * 2 * nout * n,
+                                     digit.get() + r0 * nout * digits * n, keys.data() + r0, perms.data() + r0,
+                                     (uint32_t)(r1 - r0), (uint32_t)digits, (uint32_t)c.key_limbs(), outp,
+                                     (uint32_t)nout, accumulate && r0 == 0, c.stream, nout * digits * n,
+                                     seeds.data() + r0);
+        }
+    }
 }
 
 void key_switch_batch(Context &c, uint64_t *cts, const uint64_t *targets, size_t B, size_t l, const DevBuf &key,
