@@ -260,7 +260,10 @@ bool ks_modup_col_inverse(const DeviceTables &t, uint32_t B, uint32_t l, uint32_
 // lazily reduced words above), written by ks_lift_col (one special prime) or
 // ks_modup_convert_col with raw set.  ks_row_inner runs the row pass and
 // multiplies by the keys.
-bool ks_row_inner_ok(const DeviceTables &t, uint32_t alpha);
+// Whether a key switch takes them: count inputs of one key, or sums of rotations,
+// a launch.
+bool ks_row_inner_ok(const DeviceTables &t, uint32_t alpha, const uint8_t *out_primes_host, uint32_t nout,
+                     uint32_t count);
 void ks_lift_col(const DeviceTables &t, uint64_t *T, const uint64_t *coef, uint32_t B, uint32_t l,
                  const uint8_t *out_primes_host, uint32_t nout, hipStream_t s);
 struct KsRowInner {

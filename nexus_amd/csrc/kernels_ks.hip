@@ -554,9 +554,27 @@ __global__ __launch_bounds__(kThreads) void k_row_inner(RowInnerArgs a)
 
 }  // namespace
 
-bool ks_row_inner_ok(const DeviceTables &t, uint32_t alpha)
+// Workgroups of k_row_inner for one output prime of one input or sum.
+static uint32_t row_inner_tiles(int logn) { return (1u << logn) / (logn == 17 ? 2048u : 1024u); }
+
+// Primes of 2^51 and above take the kernel's 64-bit form: a serial chain of digits
+// with two waves a SIMD (rows of 512: one) to hide it.  It needs the device full,
+// two workgroups a CU, to beat a stored ModUp, whose transforms and products
+// spread over every digit; at N = 2^17 it does not where most primes are wide.
+// Microseconds, stored ModUp / this one:
+//   160 blocks, N = 2^14, ten primes, two of 58 bits: one input 84 / 97, a sum of 16: 356 / 504
+//   320 blocks, 2^15, the same: 104 / 116, 619 / 748;  336, 2^14, 21 of 60 bits: 158 / 163, 1585 / 1715
+//   640 blocks, 2^16, ten of 60 bits: 163 / 158, 1360 / 1282;  six sums at 2^15: 3261 / 2827
+//   2^17: ten primes, two of 60 bits: 230 / 238, 2235 / 2071; 21 of 60 bits: 918 / 966, 24 sums of eight 135 / 147 ms
+// Below 2^51 it is ahead from the smallest call on (2^14, ten primes of 46 bits: 75 / 70, 333 / 315).
+bool ks_row_inner_ok(const DeviceTables &t, uint32_t alpha, const uint8_t *out_primes_host, uint32_t nout,
+                     uint32_t count)
 {
-    return t.logn >= 14 && t.logn <= 17 && t.max_bits <= 61 && (alpha == 1 || ks_modup_col_ok(t, alpha));
+    if (t.logn < 14 || t.logn > 17 || t.max_bits > 61 || !(alpha == 1 || ks_modup_col_ok(t, alpha))) return false;
+    uint32_t wide = 0;
+    for (uint32_t I = 0; I < nout; I++) wide += t.mod_host[out_primes_host[I]] >= kFpPrimeBound ? 1 : 0;
+    if (!wide) return true;
+    return row_inner_tiles(t.logn) * nout * count >= 512u && (t.logn < 17 || 2 * wide <= nout);
 }
 
 void ks_lift_col(const DeviceTables &t, uint64_t *T, const uint64_t *coef, uint32_t B, uint32_t l,
@@ -654,7 +672,7 @@ void ks_row_inner(const DeviceTables &t, const KsRowInner &p, hipStream_t s)
     ProfScope prof(rot ? "ks_row_inner_rot" : "ks_row_inner", s,
                    (double)n * p.nout *
                        ((8.0 + (seeded ? 8.0 : 16.0)) * p.count * p.digits + 16.0 * a.B + (rot ? 4.0 * p.count : 0.0)));
-    const dim3 grid(n / (l2 == 9 ? 2048 : 1024), p.nout * a.B);
+    const dim3 grid(row_inner_tiles(t.logn), p.nout * a.B);
 #define NX_RI(L)                                                                             \
     if (l2 == L) {                                                                         \
         if (rot && seeded)                                                                 \

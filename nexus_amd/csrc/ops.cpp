@@ -356,8 +356,6 @@ DevBuf ks_modup_list(Context &c, const uint64_t *const *targets, size_t B, size_
     return ks_modup_impl(c, nullptr, targets, B, l);
 }
 
-bool ks_rows_fused(const Context &c) { return ks_row_inner_ok(c.tables, (uint32_t)c.alpha); }
-
 // Words of digits in flight between the column pass and the inner product (2
 // GiB).  Smaller chunks that stay in the 256 MB last-level cache measured
 // slower (64 fused products at 20 limbs, N = 2^16: 7.12 ms at 256 MB, 6.80 at
@@ -412,13 +410,17 @@ void ks_inner_one_key(Context &c, uint64_t *acc, const uint64_t *targets, size_t
     const size_t n = c.n, nout = l + c.alpha, digits = c.digits(l);
     uint8_t outp[kMaxPrimes];
     ks_out_primes(c, l, outp);
-    if (!ks_rows_fused(c)) {
-        DevBuf T = ks_modup(c, targets, B, l);
-        ks_inner_product(c.tables, acc, T.get(), key.get(), (uint32_t)B, (uint32_t)digits, (uint32_t)c.key_limbs(),
-                         outp, (uint32_t)nout, c.stream, aseed);
+    const size_t bc = ks_inner_chunk(c, B, l);
+    if (!ks_row_inner_ok(c.tables, (uint32_t)c.alpha, outp, (uint32_t)nout, (uint32_t)bc)) {
+        const size_t most = std::max<size_t>(1, kDigitWords / (nout * digits * n));
+        for (size_t b0 = 0; b0 < B; b0 += most) {
+            const size_t cnt = std::min(most, B - b0);
+            DevBuf T = ks_modup(c, targets + b0 * l * n, cnt, l);
+            ks_inner_product(c.tables, acc + b0 * 2 * nout * n, T.get(), key.get(), (uint32_t)cnt, (uint32_t)digits,
+                             (uint32_t)c.key_limbs(), outp, (uint32_t)nout, c.stream, aseed);
+        }
         return;
     }
-    const size_t bc = ks_inner_chunk(c, B, l);
     const bool inverse = ks_inner_inverse(c, bc, l);
     DevBuf coef(&c, B * l * n), T(&c, bc * nout * digits * n);
     ks_coefficients(c, coef.get(), targets, nullptr, B, l, inverse);
@@ -446,8 +448,12 @@ void ks_inner_sums(Context &c, uint64_t *acc, const std::vector<KsRotated> &in, 
     const size_t n = c.n, nout = l + c.alpha, digits = c.digits(l);
     uint8_t outp[kMaxPrimes];
     ks_out_primes(c, l, outp);
-    const bool fused = ks_rows_fused(c);
-    const size_t bc = fused ? ks_inner_chunk(c, in.size(), l) : std::min(in.size(), (size_t)kMaxHoist);
+    size_t sums = 1;
+    for (size_t i = 1; i < in.size(); i++) sums += in[i].sum != in[i - 1].sum ? 1 : 0;
+    size_t bc = ks_inner_chunk(c, in.size(), l);
+    const bool fused = ks_row_inner_ok(c.tables, (uint32_t)c.alpha, outp, (uint32_t)nout,
+                                       (uint32_t)std::max<size_t>(1, sums * bc / in.size()));
+    if (!fused) bc = std::min(in.size(), (size_t)kMaxHoist);
     const bool inverse = fused && ks_inner_inverse(c, bc, l);
     DevBuf coef, T;
     if (fused) {

@@ -5,8 +5,9 @@ word for word against the oracle.
 The cases sit at the edges of the kernels: every pass split (7 + 7, 7 + 8,
 8 + 8, 8 + 9 stages), primes just below the bounds that choose the form of a
 sum of products (46 and 47 bits: unreduced digits or not; 50 and 51: the number
-of terms between two reductions; 58 and 60: 64-bit words), more digits than
-terms between two reductions, short last digits, levels below the top, one
+of terms between two reductions; 58 and 60, which calls as small as most of
+these take through a stored ModUp: test_gpu_ks_wide.py has both), more digits
+than terms between two reductions, short last digits, levels below the top, one
 output prime past a chunk, and keys uploaded with extreme words."""
 import sys
 
