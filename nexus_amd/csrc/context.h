@@ -409,7 +409,7 @@ struct PeriodicPlain {
     DevBuf table;
     // device term lists of block_mix, per index pattern (M, K, index)
     struct Terms {
-        DevBuf words;  // first[M + 1] (u32, padded), the runs (int32 quads), then block_mix_plan at word `plan`
+        DevBuf words;  // first[M + 1] (u32, padded), the runs (int32 quads), then block_mix_plan at word `plan` (0: none)
         uint32_t M = 0;
         size_t plan = 0;
     };

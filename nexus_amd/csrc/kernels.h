@@ -346,7 +346,8 @@ void block_mix(const DeviceTables &t, const MixPtrs &p, const uint64_t *table, c
                const uint32_t *first, const int32_t *plan, uint32_t K, uint32_t M, uint32_t limbs, uint32_t count,
                uint32_t blocks, hipStream_t s);
 // words: per group of four outputs the starts of its quad and of its single
-// segments, the end, then the segments
+// segments, the end, then the segments; empty (and null above) where the terms
+// are better taken one output at a time
 constexpr int kQuadWords = 8, kSingleWords = 8;
 std::vector<int32_t> block_mix_plan(const int32_t *index, uint32_t K, uint32_t M);
 

@@ -108,18 +108,17 @@ struct Acc3 {
 // terms (k0 + j, entry0 + j dentry) for j < len, so the inner loop computes its
 // LDS addresses instead of loading them.  FAST: every prime below 2^58
 // (products folded every 16 terms through Acc3); otherwise 128-bit sums folded
-// every 32 terms.
-template <bool FAST>
+// every 32 terms.  WIDE: limbs below 2^51 are k_block_mix_quads'.
+template <bool FAST, bool WIDE>
 __global__ __launch_bounds__(kBlock) void k_block_mix(MixPtrs ptrs, const uint64_t *__restrict__ table,
                                                       const int4 *__restrict__ runs,
                                                       const uint32_t *__restrict__ first, const ModConst *mod,
                                                       uint32_t K, uint32_t M, uint32_t limbs, uint32_t count,
-                                                      uint32_t blocks, uint32_t log_stride, uint32_t n, int skip_fp)
+                                                      uint32_t blocks, uint32_t log_stride, uint32_t n)
 {
     extern __shared__ uint64_t lds[];
     const uint32_t row = blockIdx.y;  // poly * limbs + limb
     const uint32_t limb = row % limbs;
-    if (skip_fp && mod[limb].q < kFpPrime) return;  // k_block_mix_quads
     const uint32_t pos0 = blockIdx.x * kTile;
     const uint32_t bpt = log_stride >= 6 ? 1u : (uint32_t)kTile >> log_stride;  // blocks per tile
     const uint32_t b0 = pos0 >> log_stride;
@@ -127,10 +126,11 @@ __global__ __launch_bounds__(kBlock) void k_block_mix(MixPtrs ptrs, const uint64
     uint64_t *ws = lds + K * kTile;   // [count][bpt]
     const uint64_t roff = (uint64_t)row * n + pos0;
     const ModConst m = mod[limb];
+    if (WIDE && m.q < kFpPrime) return;
     const uint32_t lane = threadIdx.x % kTile;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kTile);
     const uint32_t lb = log_stride >= 6 ? 0u : lane >> log_stride;
-    if (m.q < kFpPrime) {
+    if (!WIDE && m.q < kFpPrime) {
         // double precision: the tile and the weights as doubles, one exact
         // product per term, the sum reduced every second term (|sum| < 3 q)
         double *xd = reinterpret_cast<double *>(xs), *wd = reinterpret_cast<double *>(ws);
@@ -425,10 +425,20 @@ void periodic_expand(const DeviceTables &t, uint64_t *out, const uint64_t *table
 // One list of segments per group of four outputs: where all four have a term at
 // consecutive inputs with one common entry step, a quad segment (cut to a
 // multiple of four terms); everything else in runs of single outputs.
+//
+// Empty where k_block_mix is the faster one: a wave takes four outputs here, so
+// fewer than sixteen leave most of the eight waves idle, few inputs do not pay
+// for the segment lists, and a single term waits for its weight.  Microseconds,
+// k_block_mix / quads, ten limbs at N = 2^16 (inputs x outputs):
+//   banded rows: 127x4 252 / 497, 127x12 477 / 520, 16x16 124 / 121, 127x16 604 / 556, 8x24 114 / 124
+//   a quarter of the terms single: 16x24 200 / 223, 127x16 1325 / 1696, 64x32 941 / 823
+//   half of them: 64x64 1989 / 2372, 127x96 8977 / 9379
+//   runs of four inputs: 127x19 (three outputs without a fourth) 1768 / 2112, 127x33 3093 / 1439
 std::vector<int32_t> block_mix_plan(const int32_t *index, uint32_t K, uint32_t M)
 {
     const uint32_t groups = (M + 3) / 4;
     std::vector<int32_t> plan((size_t)2 * groups + 1);
+    size_t quads = 0, singles = 0;  // terms that four outputs take together, terms of one
     for (uint32_t g = 0; g < groups; g++) {
         const uint32_t rows = M - 4 * g < 4 ? M - 4 * g : 4;
         auto at = [&](uint32_t o, uint32_t k) { return index[(size_t)(4 * g + o) * K + k]; };
@@ -451,6 +461,7 @@ std::vector<int32_t> block_mix_plan(const int32_t *index, uint32_t K, uint32_t M
             }
             const int32_t quad[kQuadWords] = {(int32_t)k, (int32_t)len, at(0, k), at(1, k), at(2, k), at(3, k), step, 0};
             plan.insert(plan.end(), quad, quad + kQuadWords);
+            quads += len;
             for (uint32_t o = 0; o < 4; o++)
                 for (uint32_t j = 0; j < len; j++) taken[(size_t)o * K + k + j] = 1;
             k += len;
@@ -468,10 +479,12 @@ std::vector<int32_t> block_mix_plan(const int32_t *index, uint32_t K, uint32_t M
                 while (open(k + len) && at(o, k + len) == at(o, k) + (int32_t)len * step) len++;
                 const int32_t single[kSingleWords] = {(int32_t)k, (int32_t)len, at(o, k), step, (int32_t)o, 0, 0, 0};
                 plan.insert(plan.end(), single, single + kSingleWords);
+                singles += len;
                 k += len;
             }
     }
     plan[2 * groups] = (int32_t)plan.size();
+    if (K < 16 || M < 16 || 8 * singles > singles + 4 * quads) plan.clear();
     return plan;
 }
 
@@ -489,27 +502,27 @@ void block_mix(const DeviceTables &t, const MixPtrs &p, const uint64_t *table, c
     const uint32_t n = 1u << t.logn;
     const uint32_t log_stride = (uint32_t)t.logn - (uint32_t)__builtin_ctz(blocks);
     const size_t lds = block_mix_lds_bytes(K, count, blocks, t.logn);
-    // inputs read once, outputs written once (both polynomials of every limb)
-    ProfScope prof("block_mix", s, 16.0 * n * limbs * ((double)K + (double)M));
     const dim3 grid(n / kTile, 2 * limbs);
-    // a tile inside one block has uniform weights: the quad kernel for the
-    // limbs below 2^51, the general one for what is left
-    const bool quads = log_stride >= 6;
-    bool fp = false, wide = false;
-    for (uint32_t i = 0; i < limbs; i++) (t.mod_host[i] < kFpPrime ? fp : wide) = true;
-    if (quads && fp)
+    // a tile inside one block has uniform weights: the quad kernel (where there is
+    // a plan) for the limbs below 2^51, the general one for what is left
+    const bool quads = plan && log_stride >= 6;
+    uint32_t fp = 0;
+    for (uint32_t i = 0; i < limbs; i++) fp += t.mod_host[i] < kFpPrime ? 1 : 0;
+    // inputs read once, outputs written once (both polynomials of every limb)
+    const double limb_bytes = 16.0 * n * ((double)K + (double)M);
+    if (quads && fp) {
+        ProfScope prof("block_mix_quads", s, limb_bytes * fp);
         hipLaunchKernelGGL(k_block_mix_quads, grid, dim3(kMixThreads), (size_t)K * kTile * 8, s, p,
                            reinterpret_cast<const double *>(table), plan, t.mod, K, M, limbs, count, blocks, log_stride,
                            n);
-    if (quads && !wide) return;
-    if (t.max_bits <= 58)
-        hipLaunchKernelGGL(k_block_mix<true>, grid, dim3(kBlock), lds, s, p, table,
-                           reinterpret_cast<const int4 *>(terms), first, t.mod, K, M, limbs, count, blocks,
-                           log_stride, n, quads ? 1 : 0);
-    else
-        hipLaunchKernelGGL(k_block_mix<false>, grid, dim3(kBlock), lds, s, p, table,
-                           reinterpret_cast<const int4 *>(terms), first, t.mod, K, M, limbs, count, blocks,
-                           log_stride, n, quads ? 1 : 0);
+    }
+    if (quads && fp == limbs) return;
+    ProfScope prof("block_mix", s, limb_bytes * (quads ? limbs - fp : limbs));
+    const bool fast = t.max_bits <= 58, skip = quads || !fp;
+    auto *kernel = fast ? (skip ? k_block_mix<true, true> : k_block_mix<true, false>)
+                        : (skip ? k_block_mix<false, true> : k_block_mix<false, false>);
+    hipLaunchKernelGGL(kernel, grid, dim3(kBlock), lds, s, p, table, reinterpret_cast<const int4 *>(terms), first,
+                       t.mod, K, M, limbs, count, blocks, log_stride, n);
 }
 
 }  // namespace nx

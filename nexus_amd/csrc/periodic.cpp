@@ -203,8 +203,8 @@ void op_periodic_mix(const std::vector<const Ciphertext *> &in, PeriodicPlain &w
             h[M] = (int32_t)(runs.size() / 4);
             h.insert(h.end(), runs.begin(), runs.end());
             PeriodicPlain::Terms t;
-            t.plan = h.size();  // a multiple of four words
             const std::vector<int32_t> plan = block_mix_plan(index, (uint32_t)K, (uint32_t)M);
+            t.plan = plan.empty() ? 0 : h.size();  // a multiple of four words
             h.insert(h.end(), plan.begin(), plan.end());
             t.words.reset(&c, (h.size() + 1) / 2);
             // stream-ordered: the buffer may come from work still queued on the stream
@@ -231,7 +231,7 @@ void op_periodic_mix(const std::vector<const Ciphertext *> &in, PeriodicPlain &w
     }
     const uint32_t *first = reinterpret_cast<const uint32_t *>(terms->words.get());
     const int32_t *runs = reinterpret_cast<const int32_t *>(first + ((M + 1 + 3) & ~(size_t)3));
-    const int32_t *plan = reinterpret_cast<const int32_t *>(first) + terms->plan;
+    const int32_t *plan = terms->plan ? reinterpret_cast<const int32_t *>(first) + terms->plan : nullptr;
     block_mix(c.tables, p, w.table.get(), runs, first, plan, (uint32_t)K, (uint32_t)M, (uint32_t)l,
               (uint32_t)w.count, (uint32_t)w.blocks, c.stream);
     for (size_t m = 0; m < M; m++) *out[m] = std::move(res[m]);
