@@ -245,7 +245,7 @@ public:
     void linear_combination(const std::vector<const Ciphertext *> &cts, const std::vector<double> &values,
                             const std::vector<double> &scales, size_t chain_index, Ciphertext &dest) const;
     // dest[g] = sum_r pts[g K + r] * cts[r] (K = cts.size(), null: no term): the
-    // giant steps of one BSGS output at once, each ciphertext read once per 4 rows
+    // giant steps of one BSGS output at once, each ciphertext read once per up to 8 rows
     void multiply_plain_accumulate_multi(const std::vector<const Ciphertext *> &cts,
                                          const std::vector<const Plaintext *> &pts,
                                          std::vector<Ciphertext> &dest) const;

@@ -276,7 +276,7 @@ int nx_multiply_plain_accumulate(const nx_ciphertext *const *cts, const nx_plain
  * NULL: no term; every row needs one): all giant steps of one BSGS output at
  * once (no counterpart in the reference, which runs one multiply-accumulate per
  * giant step, cuda/src/bootstrapping/Bootstrapper.cu:1855-1919).  Each
- * ciphertext is read once for every 4 rows instead of once per row; each row
+ * ciphertext is read once for up to 8 rows instead of once per row; each row
  * equals nx_multiply_plain_accumulate over its terms word for word. */
 /* dest = sum_r cts[r] * encode_constant(values[r], scales[r]) at chain_index
  * (each input read at its first limbs, no copy): word for word mod_switch_to,

@@ -642,7 +642,7 @@ _sig("nx_multiply_plain_accumulate_multi", [ctypes.POINTER(vp), sz, ctypes.POINT
 
 
 def multiply_plain_accumulate_multi(cts, rows):
-    """[sum_r rows[g][r] * cts[r] for g] with each ciphertext read once per 4 rows
+    """[sum_r rows[g][r] * cts[r] for g] with each ciphertext read once per up to 8 rows
     (rows[g][r] may be None: no term)."""
     K, G = len(cts), len(rows)
     flat = []

@@ -1311,8 +1311,15 @@ void op_dot_plain_multi(const std::vector<const Ciphertext *> &cts, const std::v
     }
     std::vector<const uint64_t *> cp(K), pp;
     for (size_t r = 0; r < K; r++) cp[r] = cts[r]->data.get();
-    for (size_t g0 = 0; g0 < G; g0 += kMultiDotG) {
-        const size_t rows = std::min<size_t>(kMultiDotG, G - g0);
+    for (size_t g0 = 0, rows; g0 < G; g0 += rows) {
+        // a missing plaintext is a branch between a term's loads, and the more
+        // rows a thread takes the less hides it: seven or eight go as four and
+        // the rest.  21 limbs at N = 2^16, one plaintext of each eight rows
+        // missing, one launch / two: 4 inputs x 8 rows 143 / 122 us, 32 x 8 624 /
+        // 567; 4 x 6 101 / 101, 32 x 6 444 / 520; none missing 32 x 8 408 / 535
+        rows = std::min<size_t>(kMultiDotG, G - g0);
+        const auto end = pts.begin() + (g0 + rows) * K;
+        if (rows > 6 && std::find(pts.begin() + g0 * K, end, nullptr) != end) rows = 4;
         for (size_t r0 = 0; r0 < K; r0 += kMultiDotK) {
             const size_t cnt = std::min<size_t>(kMultiDotK, K - r0);
             pp.assign(rows * cnt, nullptr);
