@@ -466,7 +466,8 @@ def bench_bert_call(nx, reps):
     B["layer"].forward(cts, BERT_TOKENS)
     return {"ms_per_layer_call": ms, "tokens": BERT_TOKENS, "stages_ms": dict(B["layer"].stage_ms()),
             "autotune_ntt": B["autotune"]["ntt"],
-            "autotune_modup": B["autotune"].get("modup", []), "autotune_moddown": B["autotune"].get("moddown", []),
+            "autotune_modup": B["autotune"].get("modup", []), "autotune_digits": B["autotune"].get("digits", []),
+            "autotune_moddown": B["autotune"].get("moddown", []),
             "autotune_epilogue": B["autotune"].get("epilogue")}
 
 
@@ -474,8 +475,7 @@ def fused_mode(mode):
     """the autotuner's choice for a conversion fused into the NTT column pass"""
     if mode < 0:
         return "unfused"
-    return "conversion in the column pass, %s outputs per workgroup, %d-column tiles, %d threads" % (
-        mode & 255 or "default", 4 if mode & 256 else 8, 512 if mode & 512 else 256)
+    return "conversion in the column pass, %s outputs per workgroup" % (mode or "default")
 
 
 def bench_bert_sets(nx, reps, count=8):
@@ -799,6 +799,9 @@ def main():
                 "modup": ["batch %d at %d limbs: %s (%.1f vs %.1f us unfused)"
                           % (e["batch"], e["limbs"], fused_mode(e["mode"]), e["us"], e["unfused_us"])
                           for e in B["autotune"].get("modup", [])],
+                "digits": ["batch %d at %d limbs: %s (%.1f vs %.1f us by default)"
+                           % (e["batch"], e["limbs"], fused_mode(e["mode"]), e["us"], e["default_us"])
+                           for e in B["autotune"].get("digits", [])],
                 "moddown": ["batch %d at %d limbs: %s (%.1f vs %.1f us unfused)"
                             % (e["batch"], e["limbs"], fused_mode(e["mode"]), e["us"], e["unfused_us"])
                             for e in B["autotune"].get("moddown", [])],

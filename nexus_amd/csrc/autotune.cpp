@@ -1,11 +1,11 @@
 // Autotuner of launch shapes at a context's ring size: the tile widths and the
 // radix (8 or 16) of the two-pass NTT (per pass, direction and power-of-two
 // batch bucket), the thread layout of the fused multiply-accumulate (per limb
-// bucket), the base conversions fused into the NTT column pass or not (and
-// their outputs per workgroup, tile width and threads), and the arithmetic of
-// the ModDown epilogue.  Every
-// candidate's output is compared word for word with the default shape's on
-// the same data before it may be chosen; the choices are process-wide.
+// bucket), the base conversions fused into the NTT column pass or not and their
+// outputs per workgroup (stored ModUps, the digits of key switches, ModDowns),
+// and the arithmetic of the ModDown epilogue.  Every candidate's output is
+// compared word for word with the default shape's on the same data before it
+// may be chosen; the choices are process-wide.
 #include <algorithm>
 #include <cstdio>
 #include <cstring>
@@ -207,8 +207,8 @@ std::string autotune(Context &c, int reps)
     rep += "], \"modup\": [";
     first_entry = true;
     if (c.alpha > 1 && ks_modup_col_ok(c.tables, (uint32_t)c.alpha)) {
-        // hybrid ModUp at the top level: the conversion fused into the forward
-        // column pass (outputs per workgroup: default rule, 4, 8, 12, all of a
+        // hybrid ModUp at the top level, stored (hoisted rotations): the conversion
+        // fused into the forward column pass (outputs per workgroup: default rule, 4, 8, 12, all of a
         // digit) against separate conversion and column-pass launches
         const size_t l = c.L;
         for (uint32_t B : {1u, 2u, 4u, 8u, 16u, 32u}) {
@@ -248,6 +248,55 @@ std::string autotune(Context &c, int reps)
                           "%s{\"batch\": %u, \"limbs\": %zu, \"mode\": %d, \"us\": %.2f, \"unfused_us\": %.2f, "
                           "\"fused_us\": [%s]}",
                           first_entry ? "" : ", ", B, l, best_m, best * 1e3, t_off * 1e3, times.c_str() + 2);
+            rep += line;
+            first_entry = false;
+        }
+    }
+    rep += "], \"digits\": [";
+    first_entry = true;
+    if (c.alpha > 1 && ks_modup_col_ok(c.tables, (uint32_t)c.alpha)) {
+        // key switches at the top level, whose digits are not stored: the whole
+        // inner product as they run it (inverse, conversion, row pass) with the
+        // default rules, 4, 8, 12 or all outputs per workgroup of the conversion
+        const size_t l = c.L, nout = l + c.alpha, kl = c.key_limbs();
+        std::vector<uint64_t> h;
+        fill_random(c, h, c.digits(l) * 2 * kl, 400, kl);
+        DevBuf key(&c, h.size());
+        NX_HIP(hipMemcpyAsync(key.get(), h.data(), h.size() * 8, hipMemcpyHostToDevice, c.stream));
+        NX_HIP(hipStreamSynchronize(c.stream));
+        for (uint32_t B : {1u, 2u, 4u, 8u, 16u, 32u}) {
+            if (ks_inner_chunk(c, B, l) < B) break;  // larger batches run in the launches above
+            fill_random(c, h, B * l, 500 + B, l);
+            DevBuf tg(&c, B * l * n), acc(&c, (size_t)B * 2 * nout * n);
+            NX_HIP(hipMemcpyAsync(tg.get(), h.data(), h.size() * 8, hipMemcpyHostToDevice, c.stream));
+            NX_HIP(hipStreamSynchronize(c.stream));
+            auto run = [&] { ks_inner_one_key(c, acc.get(), tg.get(), B, l, key, nullptr); };
+            ks_digits_col_set(B, 0);
+            run();
+            const std::vector<uint64_t> ref = download(c, acc.get(), acc.words());
+            const double t_def = time_ms(run);
+            double best = t_def;
+            int best_m = 0;
+            std::string times;
+            char buf[64];
+            for (int m : {4, 8, 12, 64}) {
+                ks_digits_col_set(B, m);
+                run();
+                const bool same = download(c, acc.get(), acc.words()) == ref;
+                const double t = same ? time_ms(run) : 1e30;
+                std::snprintf(buf, sizeof buf, ", %.2f", same ? t * 1e3 : -1.0);
+                times += buf;
+                if (t < best * 0.98) {
+                    best = t;
+                    best_m = m;
+                }
+            }
+            ks_digits_col_set(B, best_m);
+            char line[300];
+            std::snprintf(line, sizeof line,
+                          "%s{\"batch\": %u, \"limbs\": %zu, \"mode\": %d, \"us\": %.2f, \"default_us\": %.2f, "
+                          "\"mode_us\": [%s]}",
+                          first_entry ? "" : ", ", B, l, best_m, best * 1e3, t_def * 1e3, times.c_str() + 2);
             rep += line;
             first_entry = false;
         }

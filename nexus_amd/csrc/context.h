@@ -351,6 +351,8 @@ void ks_out_primes(const Context &c, size_t l, uint8_t *outp);
 DevBuf ks_modup(Context &c, const uint64_t *targets, size_t B, size_t l);
 // ModUp of B <= kNttSrcMax targets given by pointer ([l][n] each)
 DevBuf ks_modup_list(Context &c, const uint64_t *const *targets, size_t B, size_t l);
+// inputs of B that one launch of the digits takes
+size_t ks_inner_chunk(const Context &c, size_t B, size_t l);
 // acc[B][2][l+alpha][n]: inner products of the digits of B targets ([B][l][n]
 // NTT form) with one key.  aseed as KSwitchKeys::seeds_of.
 void ks_inner_one_key(Context &c, uint64_t *acc, const uint64_t *targets, size_t B, size_t l, const DevBuf &key,

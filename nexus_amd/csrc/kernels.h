@@ -248,6 +248,8 @@ bool ks_modup_col_ok(const DeviceTables &t, uint32_t alpha);
 // outputs per workgroup (0: the default rule)
 void ks_modup_col_set(uint32_t B, int mode);
 int ks_modup_col_get(uint32_t B);
+// the same for raw digits (mode >= 0)
+void ks_digits_col_set(uint32_t B, int mode);
 void ks_modup_convert_col(const DeviceTables &t, uint64_t *T, const uint64_t *coef, const ulonglong2 *w,
                           uint32_t B, uint32_t l, uint32_t alpha, uint32_t key_limbs, const uint8_t *out_primes_host,
                           uint32_t nout, hipStream_t s, bool raw = false, bool inverse = false);

@@ -917,14 +917,20 @@ constexpr double kFlopsProduct = 8.0, kFlopsReduce = 4.0;
 inline double conv_flops(uint32_t A) { return A * (kFlopsProduct + 1.0) + (A / 2) * kFlopsReduce + kFlopsReduce; }
 inline double col_flops(int logs) { return logs * (kFlopsProduct + 2.0) / 2.0 + kFlopsReduce; }
 
-// Fused ModUp column pass per power-of-two bucket of the batch size B:
-// 0 = on (outputs per workgroup by the default rule), -1 = off (conversion and
-// column pass as separate launches), k > 0 = on with k outputs per workgroup.
+// Fused ModUp column pass of a stored ModUp, per power-of-two bucket of the batch
+// size B: 0 = on (outputs per workgroup by the default rule), -1 = off (conversion
+// and column pass as separate launches), k > 0 = on with k outputs per workgroup.
 // Process-wide; set by the autotuner.
 static std::atomic<int> g_modup_col[kTuneBuckets];
+// The same for the digits of key switches without a stored ModUp, which have no
+// separate form: 0 = the default rules (the inverse's column pass included where
+// ks_modup_col_inverse says so), k > 0 = k outputs per workgroup of the plain form.
+static std::atomic<int> g_digits_col[kTuneBuckets];
 constexpr int kColMaxA = 12;   // largest digit / special-prime count of the fused conversions
 
 void ks_modup_col_set(uint32_t B, int mode) { g_modup_col[tune_bucket(B)].store(mode); }
+
+void ks_digits_col_set(uint32_t B, int mode) { g_digits_col[tune_bucket(B)].store(mode); }
 
 int ks_modup_col_get(uint32_t B) { return g_modup_col[tune_bucket(B)].load(); }
 
@@ -936,14 +942,13 @@ bool ks_modup_col_ok(const DeviceTables &t, uint32_t alpha)
 
 // Outputs per workgroup: enough workgroups to fill the device, at least 4
 // outputs per read of the digit's inputs.
-static uint32_t modup_col_chunk(const DeviceTables &t, uint32_t B, uint32_t l, uint32_t alpha, uint32_t nout)
+static uint32_t modup_col_chunk(const DeviceTables &t, uint32_t B, uint32_t l, uint32_t alpha, uint32_t nout, int mode)
 {
     const uint32_t tiles = (1u << t.logn) / 2048u, digits = (l + alpha - 1) / alpha;
     const uint32_t count = nout - std::min(alpha, l);  // most outputs of a digit (a partial digit has more)
     const uint32_t want = (2048u + tiles * B * digits - 1) / (tiles * B * digits);
     uint32_t chunk = std::max((count + want - 1) / want, std::min(4u, count));
-    const int mode = g_modup_col[tune_bucket(B)].load();  // 0: this rule
-    if (mode > 0 && (mode & 255)) chunk = std::min((uint32_t)(mode & 255), count);
+    if (mode > 0) chunk = std::min((uint32_t)mode, count);  // 0: this rule
     return chunk;
 }
 
@@ -957,7 +962,7 @@ static uint32_t modup_col_chunk(const DeviceTables &t, uint32_t B, uint32_t l, u
 constexpr uint32_t kInverseBlocks = 1024;
 bool ks_modup_col_inverse(const DeviceTables &t, uint32_t B, uint32_t l, uint32_t alpha)
 {
-    return ks_modup_col_ok(t, alpha) && l >= 1 && g_modup_col[tune_bucket(B)].load() == 0 &&
+    return ks_modup_col_ok(t, alpha) && l >= 1 && g_digits_col[tune_bucket(B)].load() == 0 &&
            (1u << t.logn) / 2048u * B * ((l + alpha - 1) / alpha) >= kInverseBlocks;
 }
 
@@ -984,7 +989,8 @@ void ks_modup_convert_col(const DeviceTables &t, uint64_t *T, const uint64_t *co
     split_logn(t.logn, l1, l2);
     const uint32_t n = 1u << t.logn;
     const uint32_t tiles = n / 2048u;
-    const uint32_t chunk = inverse ? nout - 1 : modup_col_chunk(t, B, l, alpha, nout);
+    const int mode = (raw ? g_digits_col : g_modup_col)[tune_bucket(B)].load();
+    const uint32_t chunk = inverse ? nout - 1 : modup_col_chunk(t, B, l, alpha, nout, mode);
     a.invd = t.inv_d;
     a.ninvd = t.ninv_d;
     a.chunk = chunk;
@@ -1066,7 +1072,7 @@ static uint32_t moddown_col_chunk(const DeviceTables &t, uint32_t polys, uint32_
     const uint32_t want = (2048u + tiles * polys - 1) / (tiles * polys);
     uint32_t chunk = std::max((lo + want - 1) / want, std::min(4u, lo));
     const int mode = g_moddown_col[tune_bucket(polys)].load();
-    if (mode > 0 && (mode & 255)) chunk = std::min((uint32_t)(mode & 255), lo);
+    if (mode > 0) chunk = std::min((uint32_t)mode, lo);
     return chunk;
 }
 

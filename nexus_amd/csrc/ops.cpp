@@ -363,9 +363,9 @@ DevBuf ks_modup_list(Context &c, const uint64_t *const *targets, size_t B, size_
 // shorter launches leave more of the device idle at their ends.
 constexpr size_t kDigitWords = (size_t)1 << 28;
 
-// Inputs a launch takes of B: as many as kDigitWords and the argument arrays
-// hold, in even chunks (no short last launch).
-static size_t ks_inner_chunk(const Context &c, size_t B, size_t l)
+// As many as kDigitWords and the argument arrays hold, in even chunks (no short
+// last launch).
+size_t ks_inner_chunk(const Context &c, size_t B, size_t l)
 {
     const size_t per = (l + c.alpha) * c.digits(l) * c.n;
     const size_t most = std::max<size_t>(1, std::min(kDigitWords / per, (size_t)kMaxHoist));

@@ -61,10 +61,11 @@ def test_autotune_then_parity(logn, chain):
 
 
 def test_autotune_modup_then_parity():
-    """hybrid context with every prime below 2^51: the tuner times the ModUp and
-    ModDown conversions fused into the column pass against the separate
-    launches (each candidate checked word for word), and relinearisation stays
-    bit-exact under its choices"""
+    """hybrid context with every prime below 2^51: the tuner times the stored ModUp
+    and ModDown conversions fused into the column pass against the separate
+    launches and the key switch's digits per outputs of a workgroup (each
+    candidate checked word for word), and relinearisation stays bit-exact under
+    its choices"""
     if nx.device_count() < 1:
         pytest.skip("no GPU visible")
     from oracle import hybrid
@@ -75,11 +76,15 @@ def test_autotune_modup_then_parity():
     print(rep["modup"])
     assert [e["batch"] for e in rep["modup"]] == [1, 2, 4, 8, 16, 32]
     for e in rep["modup"]:
-        assert e["mode"] in (-1, 0, 4, 8, 12, 64, 256, 264, 268, 512, 520, 524)
+        assert e["mode"] in (-1, 0, 4, 8, 12, 64)
         assert all(t > 0 for t in e["fused_us"])  # every fused candidate equalled the unfused words
+    assert [e["batch"] for e in rep["digits"]] == [1, 2, 4, 8, 16, 32]
+    for e in rep["digits"]:
+        assert e["mode"] in (0, 4, 8, 12, 64)
+        assert e["default_us"] > 0 and all(t > 0 for t in e["mode_us"])
     assert [e["batch"] for e in rep["moddown"]] == [1, 2, 4, 8, 16]
     for e in rep["moddown"]:
-        assert e["mode"] in (-1, 0, 4, 8, 12, 64, 256, 264, 268, 512, 520, 524)
+        assert e["mode"] in (-1, 0, 4, 8, 12, 64)
         assert all(t > 0 for t in e["fused_us"])
     L = ctx.L
     sk = nx.SecretKey(ctx, seed=71)
