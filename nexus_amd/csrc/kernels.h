@@ -294,7 +294,7 @@ void ks_moddown_convert_col(const DeviceTables &t, uint64_t *z, const uint64_t *
                             const ulonglong2 *w, const double *convd, const uint8_t *in_primes_host, uint32_t A,
                             uint32_t polys, uint32_t lo, uint32_t L, hipStream_t s, bool inverse = false);
 // as ks_modup_col_inverse, for the limbs of acc
-bool ks_moddown_col_inverse(const DeviceTables &t, uint32_t polys);
+bool ks_moddown_col_inverse(const DeviceTables &t, uint32_t A, uint32_t polys);
 // per power-of-two bucket of the poly count: as ks_modup_col_set
 void ks_moddown_col_set(uint32_t polys, int mode);
 int ks_moddown_col_get(uint32_t polys);

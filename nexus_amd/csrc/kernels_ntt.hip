@@ -959,10 +959,17 @@ static uint32_t modup_col_chunk(const DeviceTables &t, uint32_t B, uint32_t l, u
 // 64 fused products at 20 limbs, N = 2^16: 6.37 ms with the column pass apart,
 // 5.99 with it here; with the line at 2048 workgroups and outputs cut up below
 // that, 6.14.  Six sums of sixteen rotations: 4.94, 4.80 and 4.91 ms.
-constexpr uint32_t kInverseBlocks = 1024;
+// Up to kInverseMaxA inputs: they are all live during the column passes, and from
+// ten on the conversions have one wave a SIMD to hide those.  33 fused products
+// (apart, here): ten special primes 3.45, 3.57 ms at N = 2^16 and 7.41, 7.72 at
+// 2^17; eight 3.35, 3.20 and 7.06, 6.83; 33 plain ones with nine at 2^16 3.60,
+// 3.50.  The ModDowns of eight and nine inputs spill (9 over columns of 2^8 40
+// words, of 2^7 105), which costs what the pass saves over columns of 2^7: 1.33
+// and 1.34 ms at 2^15.
+constexpr uint32_t kInverseBlocks = 1024, kInverseMaxA = 9;
 bool ks_modup_col_inverse(const DeviceTables &t, uint32_t B, uint32_t l, uint32_t alpha)
 {
-    return ks_modup_col_ok(t, alpha) && l >= 1 && g_digits_col[tune_bucket(B)].load() == 0 &&
+    return ks_modup_col_ok(t, alpha) && alpha <= kInverseMaxA && l >= 1 && g_digits_col[tune_bucket(B)].load() == 0 &&
            (1u << t.logn) / 2048u * B * ((l + alpha - 1) / alpha) >= kInverseBlocks;
 }
 
@@ -972,6 +979,7 @@ void ks_modup_convert_col(const DeviceTables &t, uint64_t *T, const uint64_t *co
 {
     if (!ks_modup_col_ok(t, alpha)) throw std::invalid_argument("ks_modup_convert_col: unsupported parameters");
     if (nout > (uint32_t)kMaxPrimes || l < 1 || nout <= alpha) throw std::invalid_argument("ks_modup_convert_col: bad sizes");
+    if (inverse && (!raw || alpha > kInverseMaxA)) throw std::invalid_argument("ks_modup_convert_col: no such form");
     ModUpColArgs a;
     a.T = T;
     a.coef = coef;
@@ -1004,7 +1012,7 @@ void ks_modup_convert_col(const DeviceTables &t, uint64_t *T, const uint64_t *co
 #define NX_MC(LOGS, A)                                                                      \
     if (l1 == LOGS && alpha == A) {                                                       \
         if (raw && inverse)                                                               \
-            hipLaunchKernelGGL((k_modup_col<LOGS, A, true, true>), grid, dim3(kThreads), 0, s, a);   \
+            hipLaunchKernelGGL((k_modup_col<LOGS, A, true, (A <= kInverseMaxA)>), grid, dim3(kThreads), 0, s, a); \
         else if (raw)                                                                     \
             hipLaunchKernelGGL((k_modup_col<LOGS, A, true, false>), grid, dim3(kThreads), 0, s, a);  \
         else                                                                              \
@@ -1076,9 +1084,9 @@ static uint32_t moddown_col_chunk(const DeviceTables &t, uint32_t polys, uint32_
     return chunk;
 }
 
-bool ks_moddown_col_inverse(const DeviceTables &t, uint32_t polys)
+bool ks_moddown_col_inverse(const DeviceTables &t, uint32_t A, uint32_t polys)
 {
-    return g_moddown_col[tune_bucket(polys)].load() == 0 && (1u << t.logn) / 2048u * polys >= kInverseBlocks;
+    return A <= kInverseMaxA && g_moddown_col[tune_bucket(polys)].load() == 0 && (1u << t.logn) / 2048u * polys >= kInverseBlocks;
 }
 
 void ks_moddown_convert_col(const DeviceTables &t, uint64_t *z, const uint64_t *acc, uint64_t acc_stride,
@@ -1087,6 +1095,7 @@ void ks_moddown_convert_col(const DeviceTables &t, uint64_t *z, const uint64_t *
 {
     if (!ks_moddown_col_ok(t, A) || !convd) throw std::invalid_argument("ks_moddown_convert_col: unsupported parameters");
     if (lo < 1 || lo + A > (uint32_t)kMaxPrimes) throw std::invalid_argument("ks_moddown_convert_col: bad sizes");
+    if (inverse && A > kInverseMaxA) throw std::invalid_argument("ks_moddown_convert_col: no such form");
     ModDownColArgs a;
     a.z = z;
     a.acc = acc;
@@ -1116,7 +1125,7 @@ void ks_moddown_convert_col(const DeviceTables &t, uint64_t *z, const uint64_t *
 #define NX_MD(LOGS, AA)                                                                     \
     if (l1 == LOGS && A == AA) {                                                          \
         if (inverse)                                                                      \
-            hipLaunchKernelGGL((k_moddown_col<LOGS, AA, true>), grid, dim3(kThreads), 0, s, a);  \
+            hipLaunchKernelGGL((k_moddown_col<LOGS, AA, (AA <= kInverseMaxA)>), grid, dim3(kThreads), 0, s, a); \
         else                                                                              \
             hipLaunchKernelGGL((k_moddown_col<LOGS, AA, false>), grid, dim3(kThreads), 0, s, a); \
         return;                                                                           \

@@ -517,7 +517,7 @@ DevBuf ks_moddown_prepare(Context &c, uint64_t *acc, size_t B, size_t l, FwdInpu
     const size_t nout = l + alpha;
     const bool col = alpha > 1 && c.d_moddown_conv_d && ks_moddown_col_ok(c.tables, (uint32_t)alpha) &&
                      ks_moddown_col_get((uint32_t)(2 * B)) >= 0;
-    const bool inverse = col && ks_moddown_col_inverse(c.tables, (uint32_t)(2 * B));
+    const bool inverse = col && ks_moddown_col_inverse(c.tables, (uint32_t)alpha, (uint32_t)(2 * B));
     // The special-prime limbs of acc are transformed in place: INTT of the
     // special limbs of every poly.
     {
@@ -926,7 +926,7 @@ void op_multiply_relin_rescale_fused_many(const std::vector<const Ciphertext *> 
         rns_add_limb_scaled(c.tables, acc.get(), nout * n, c01.get(), pw, (uint32_t)lo, c.mdr_pmod[l],
                             (uint32_t)(2 * cnt), c.stream);
         const bool col = ks_moddown_col_ok(c.tables, (uint32_t)A) && ks_moddown_col_get((uint32_t)(2 * cnt)) >= 0;
-        const bool inverse = col && ks_moddown_col_inverse(c.tables, (uint32_t)(2 * cnt));
+        const bool inverse = col && ks_moddown_col_inverse(c.tables, (uint32_t)A, (uint32_t)(2 * cnt));
         {
             NttBatch nb;
             nb.data = acc.get() + lo * n;

@@ -1,5 +1,5 @@
 """Where the inverse's column pass runs: large batches of a hybrid key switch fold
-it into their conversions, small ones launch it, and after autotuning the
+it into conversions of up to nine inputs, small ones launch it, and after autotuning the
 key switch's digits follow the choice measured on them.
 Fused products with a remainder chunk and the top word of every prime, against
 the same products one at a time.
@@ -44,7 +44,9 @@ def main():
     sys.path.insert(0, ROOT)
     import nexus_amd as nx
 
-    for logn, chain, alpha in ((16, [46] * 5 + [47] * 3, 3), (15, [51] + [46] * 9 + [51] * 8, 8)):
+    # the last: passes of a chunk of 32 and a remainder of 3, digits and ModDown of alpha + 1 inputs
+    for logn, chain, alpha, passes in ((16, [46] * 5 + [47] * 3, 3, 2), (15, [51] + [46] * 9 + [51] * 8, 8, 2),
+                                       (16, [46] * 9 + [47] * 9, 9, 3), (16, [46] * 10 + [47] * 10, 10, 4)):
         print("[case] inverse fold logn=%d alpha=%d" % (logn, alpha), flush=True)
         ctx = nx.Context(logn, chain, special_primes=alpha)
         sk = nx.SecretKey(ctx, seed=8)
@@ -59,7 +61,7 @@ def main():
         a = [cts[i % 4] for i in range(count)]
         b = [cts[(i + 1 + i // 4) % 4] for i in range(count)]
         many, cols = _inverse_columns(nx, ctx, lambda: nx.multiply_relin_rescale_many(a, b, rk, fused=True))
-        assert cols == 2, cols  # the remainder's digits and ModDown
+        assert cols == passes, cols
         ones = {}
         for i in range(count):
             key = (i % 4, (i + 1 + i // 4) % 4)
@@ -73,7 +75,7 @@ def main():
         digits = {e["batch"]: e["mode"] for e in rep["digits"]}[32]
         _, cols = _inverse_columns(nx, ctx, lambda: nx.multiply_relin_rescale_many(a[:32], b[:32], rk, fused=True))
         # the tuner's ModDowns end at 32 polys: these 64 keep the default rule
-        assert cols == (digits != 0), (cols, rep["digits"])
+        assert cols == (alpha > 9 or digits != 0) + (alpha > 8), (cols, rep["digits"])
         del ctx, sk, rk, cts, a, b, many, one
     print("ok", flush=True)
 
