@@ -1,8 +1,10 @@
 // Exact modular products in double precision for primes below 2^51 (device).
-// With |a| <= q (1 + eps) and 0 <= w < q (or a, w < 2^51, q < 2^51):
+// fp_mulmod(a, w) with integers |a w| <= 2^53 q:
 //   h = a w (rounded), e = fma(a, w, -h) = a w - h exactly,
-//   Q = rint(h / q) within 1.25 of a w / q,  r = fma(-Q, q, h) + e = a w - Q q,
-// every intermediate an integer below 2^53, so r is exact with |r| <= 1.25 q.
+//   Q = rint(h / q), off the quotient by at most 1/2 + 3 2^-53 |a w / q|,
+//   r = fma(-Q, q, h) + e = a w - Q q,
+// every intermediate an integer below 2^53, so r is exact: |r| <= 1.25 q for
+// |a|, |w| <= q, and |r| <= q/2 + 1.5 2^-53 q |a| for centred |w| <= q/2.
 // fp_reduce(z) = z - rint(z / q) q maps an integer |z| < 2^53 to a
 // representative of magnitude at most q/2 (1 + eps).  Files using these are
 // compiled without floating-point contraction.
@@ -13,6 +15,17 @@
 namespace nx {
 
 constexpr uint64_t kFpPrime = 1ull << 51;  // primes below this take the double-precision forms
+
+// p[i] of a table that no kernel writes, at an index that is the same for the
+// whole wave: a scalar load.  Through an ordinary pointer the compiler has to
+// assume that the kernel's own stores may reach the table, and takes a vector
+// load, which waits for them.
+template <class T>
+__device__ __forceinline__ T table_at(const T *p, uint64_t i)
+{
+    typedef const __attribute__((address_space(4))) T *Constant;
+    return ((Constant)(uintptr_t)p)[i];
+}
 
 // x < 2^52 as a double: two instructions (the compiler's conversion takes four)
 __device__ __forceinline__ double fp_from(uint64_t x)

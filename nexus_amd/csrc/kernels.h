@@ -241,8 +241,9 @@ void ks_modup_copy_own(const DeviceTables &t, uint64_t *T, const uint64_t *targe
 // ModUp conversion fused into the forward NTT's column pass: T[b][I][j] for
 // the output primes I outside digit j, column-transformed (the caller runs the
 // row pass with NttBatch::rows_only); the digit's own limbs are not written
-// (ks_modup_copy_own).  Needs ks_modup_col_ok: every prime below 2^51,
-// 2 <= alpha <= 8, 2^14 <= n <= 2^17, the double-precision factor table.
+// (ks_modup_copy_own).  raw: left as ks_row_inner reads them (below); inverse (raw
+// only): coef comes from the inverse's row pass alone (ks_modup_col_inverse).  Needs ks_modup_col_ok: every prime below 2^51,
+// 2 <= alpha <= 12, 2^14 <= n <= 2^17, the double-precision factor table.
 bool ks_modup_col_ok(const DeviceTables &t, uint32_t alpha);
 // per power-of-two bucket of B: -1 = unfused; otherwise fused, with `mode`
 // outputs per workgroup (0: the default rule)
@@ -288,7 +289,7 @@ void ks_row_inner(const DeviceTables &t, const KsRowInner &p, hipStream_t s);
 // Context::d_moddown_conv_d / d_mdr_conv_d) converted, centred, to the primes
 // q_0 .. q_(lo-1) and column-transformed into z[polys][lo][n]; the caller runs
 // the row pass (NttBatch::rows_only), with its epilogue.  Needs
-// ks_moddown_col_ok: every prime below 2^51, 2 <= A <= 9, 2^14 <= n <= 2^17.
+// ks_moddown_col_ok: every prime below 2^51, 2 <= A <= 13, 2^14 <= n <= 2^17.
 bool ks_moddown_col_ok(const DeviceTables &t, uint32_t A);
 void ks_moddown_convert_col(const DeviceTables &t, uint64_t *z, const uint64_t *acc, uint64_t acc_stride,
                             const ulonglong2 *w, const double *convd, const uint8_t *in_primes_host, uint32_t A,

@@ -66,7 +66,8 @@ __device__ __forceinline__ void col_stages_int(uint64_t *lds, const ulonglong2 *
 // Workgroup (column tile, b, digit j, chunk of the listed output primes): the
 // digit's coefficients are read once, and for every output prime of the chunk
 // but the digit's own they are reduced, column-transformed and stored.  INT:
-// the listed primes are 2^51 and above.
+// the listed primes are 2^51 and above.  Below, the bound of four waves a SIMD
+// costs six spilled words a lane.
 template <int LOGS, bool INT>
 __global__ __launch_bounds__(kThreads, INT ? 2 : 4) void k_lift_col(LiftColArgs a)
 {
@@ -108,11 +109,11 @@ __global__ __launch_bounds__(kThreads, INT ? 2 : 4) void k_lift_col(LiftColArgs 
             double v[8];
             if (small) {  // uniform
 #pragma unroll
-                for (int k = 0; k < 8; k++) v[k] = reduce_f(fp_from(x[k]), q, qinv);
+                for (int k = 0; k < 8; k++) v[k] = fp_reduce(fp_from(x[k]), q, qinv);
             } else {
                 const ModConst m = table_mod(a.mod, kp);
 #pragma unroll
-                for (int k = 0; k < 8; k++) v[k] = reduce_f(fp_from(barrett64(x[k], m)), q, qinv);
+                for (int k = 0; k < 8; k++) v[k] = fp_reduce(fp_from(barrett64(x[k], m)), q, qinv);
             }
             col_forward<LOGS, true>(v, reinterpret_cast<double *>(words) + buf * C::LDS, tw, q, qinv, (int)a.logn, N2,
                                     col0, out);
@@ -145,8 +146,10 @@ struct RowInnerArgs {
 // Rows of 2^LOGS words, whole rows per wave, W words a lane (4; 8 for rows of
 // 512): the row stages run in steps of log2 W in registers with an exchange
 // through the wave's own part of LDS between them, so no barrier is needed.
-// Four words a lane keep both accumulators, the row's twiddles and the key
-// words of a digit within 128 registers (four waves per SIMD).
+// Four words a lane hold both accumulators, the row's twiddles and the key words
+// of a digit: 136 to 138 registers for rows of 256 (three waves a SIMD), 150 to
+// 152 for rows of 128 (three); with rotations 166 to 168 (three) and 172 to 176
+// (two).  Rows of 512 take all 256 and one wave.
 // Step i (of K stages from stage s) joins 2^K positions D apart in blocks of
 // S >> s: group gg = o + LPR u of a lane is block gg / D, offset gg % D.  In
 // LDS position p sits at p + PAD (p / 16): blocks of four words 16 apart then
@@ -324,7 +327,7 @@ __global__ __launch_bounds__(kThreads) void k_row_inner(RowInnerArgs a)
     const uint32_t begin = ROT ? a.first[b] : b, end = ROT ? a.first[b + 1] : b + 1;
     const bool accumulate = ROT && a.accumulate && b == 0;
 
-    if (m.q < kFpPrimeBound) {
+    if (m.q < kFpPrime) {
         const double q = a.qd[kp].x, qinv = a.qd[kp].y;
         const double *tw = a.twd + (uint64_t)kp * n;
         // through: the digits come unreduced and stay so, |t| <= 2^50, in the sums
@@ -344,8 +347,8 @@ __global__ __launch_bounds__(kThreads) void k_row_inner(RowInnerArgs a)
             load_row<LOGS>(v1, out + poly1, o);
 #pragma unroll
             for (int k = 0; k < W; k++) {
-                s0[k].l = reduce_f(fp_from(v0[k]), q, qinv);
-                s1[k].l = reduce_f(fp_from(v1[k]), q, qinv);
+                s0[k].l = fp_reduce(fp_from(v0[k]), q, qinv);
+                s1[k].l = fp_reduce(fp_from(v1[k]), q, qinv);
             }
         }
         uint64_t mix[W];  // the counter's half of the generator, the same for every digit
@@ -397,7 +400,7 @@ __global__ __launch_bounds__(kThreads) void k_row_inner(RowInnerArgs a)
             load_digit(0);
             for (uint32_t j = 0; j < a.digits; j++) {
                 // the key words and the next digit are asked for ahead of the
-                // stages: four waves a SIMD do not hide the loads by themselves
+                // stages: two or three waves a SIMD do not hide the loads by themselves
                 double t[W];
 #pragma unroll
                 for (int k = 0; k < W; k++) t[k] = j == own_digit ? fp_from(x[k]) : __longlong_as_double((long long)x[k]);
@@ -408,7 +411,7 @@ __global__ __launch_bounds__(kThreads) void k_row_inner(RowInnerArgs a)
                 if (j + 1 < a.digits) load_digit(j + 1);
                 if (j == own_digit) {
 #pragma unroll
-                    for (int k = 0; k < W; k++) t[k] = reduce_f(t[k], q, qinv);
+                    for (int k = 0; k < W; k++) t[k] = fp_reduce(t[k], q, qinv);
                 } else {
                     if (lazy)
                         row_forward<LOGS, true>(t, lds, o, w, q, qinv);
@@ -424,7 +427,7 @@ __global__ __launch_bounds__(kThreads) void k_row_inner(RowInnerArgs a)
                     }
                     if (lazy && !through) {  // uniform
 #pragma unroll
-                        for (int k = 0; k < W; k++) t[k] = reduce_f(t[k], q, qinv);
+                        for (int k = 0; k < W; k++) t[k] = fp_reduce(t[k], q, qinv);
                     }
                 }
                 if (left == 0) {  // uniform
@@ -572,7 +575,7 @@ bool ks_row_inner_ok(const DeviceTables &t, uint32_t alpha, const uint8_t *out_p
 {
     if (t.logn < 14 || t.logn > 17 || t.max_bits > 61 || !(alpha == 1 || ks_modup_col_ok(t, alpha))) return false;
     uint32_t wide = 0;
-    for (uint32_t I = 0; I < nout; I++) wide += t.mod_host[out_primes_host[I]] >= kFpPrimeBound ? 1 : 0;
+    for (uint32_t I = 0; I < nout; I++) wide += t.mod_host[out_primes_host[I]] >= kFpPrime ? 1 : 0;
     if (!wide) return true;
     return row_inner_tiles(t.logn) * nout * count >= 512u && (t.logn < 17 || 2 * wide <= nout);
 }
@@ -599,7 +602,7 @@ void ks_lift_col(const DeviceTables &t, uint64_t *T, const uint64_t *coef, uint3
     for (int wide = 0; wide < 2; wide++) {  // primes below 2^51, then the others
         a.listed = 0;
         for (uint32_t I = 0; I < nout; I++)
-            if ((t.mod_host[out_primes_host[I]] >= kFpPrimeBound) == (wide != 0)) a.list[a.listed++] = I;
+            if ((t.mod_host[out_primes_host[I]] >= kFpPrime) == (wide != 0)) a.list[a.listed++] = I;
         if (!a.listed) continue;
         // outputs per workgroup: enough workgroups to fill the device, at least 4
         // outputs per read of the digit

@@ -254,14 +254,6 @@ __global__ __launch_bounds__(kBlock) void k_block_mix(MixPtrs ptrs, const uint64
 // k0, len, e, step, output in the group).
 constexpr int kMixThreads = 512;
 
-template <class T>
-__device__ __forceinline__ T mix_table(const T *p, int64_t i)
-{
-    // a table that no kernel writes, at a uniform index: a scalar load
-    typedef const __attribute__((address_space(4))) T *Constant;
-    return ((Constant)(uintptr_t)p)[i];
-}
-
 template <int STEP>
 __device__ __forceinline__ void quad_mac(FpSum *s, const double *x, const double *w, const int *e)
 {
@@ -269,7 +261,7 @@ __device__ __forceinline__ void quad_mac(FpSum *s, const double *x, const double
 #pragma unroll
     for (int o = 0; o < 4; o++)
 #pragma unroll
-        for (int j = 0; j < 4; j++) wv[o][j] = mix_table(w, e[o] + STEP * j);
+        for (int j = 0; j < 4; j++) wv[o][j] = table_at(w, e[o] + STEP * j);
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const double xv = x[j * kTile];
@@ -325,15 +317,15 @@ __global__ __launch_bounds__(kMixThreads) void k_block_mix_quads(MixPtrs ptrs, c
             }
             left = terms;
         };
-        const int32_t *d = plan + mix_table(plan, 2 * g), *end = plan + mix_table(plan, 2 * g + 2);
-        const int32_t *singles = plan + mix_table(plan, 2 * g + 1);
+        const int32_t *d = plan + table_at(plan, 2 * g), *end = plan + table_at(plan, 2 * g + 2);
+        const int32_t *singles = plan + table_at(plan, 2 * g + 1);
         for (; d < singles; d += kQuadWords) {
-            const int step = mix_table(d, 6);
+            const int step = table_at(d, 6);
             int e[4];
 #pragma unroll
-            for (int o = 0; o < 4; o++) e[o] = mix_table(d, 2 + o);
-            const double *x = xd + mix_table(d, 0) * kTile + lane;
-            for (int len = mix_table(d, 1); len > 0; len -= 4) {
+            for (int o = 0; o < 4; o++) e[o] = table_at(d, 2 + o);
+            const double *x = xd + table_at(d, 0) * kTile + lane;
+            for (int len = table_at(d, 1); len > 0; len -= 4) {
                 if (terms >= 4) {  // uniform
                     if (left < 4) fold();
                     left -= 4;
@@ -345,7 +337,7 @@ __global__ __launch_bounds__(kMixThreads) void k_block_mix_quads(MixPtrs ptrs, c
 #pragma unroll
                         for (int j = 0; j < 4; j++)
 #pragma unroll
-                            for (int o = 0; o < 4; o++) s[o].mac(mix_table(w, e[o] + step * j), x[j * kTile]);
+                            for (int o = 0; o < 4; o++) s[o].mac(table_at(w, e[o] + step * j), x[j * kTile]);
                     }
                 } else {
 #pragma unroll 1
@@ -353,7 +345,7 @@ __global__ __launch_bounds__(kMixThreads) void k_block_mix_quads(MixPtrs ptrs, c
                         if (left == 0) fold();
                         left--;
 #pragma unroll
-                        for (int o = 0; o < 4; o++) s[o].mac(mix_table(w, e[o] + step * j), x[j * kTile]);
+                        for (int o = 0; o < 4; o++) s[o].mac(table_at(w, e[o] + step * j), x[j * kTile]);
                     }
                 }
 #pragma unroll
@@ -362,15 +354,15 @@ __global__ __launch_bounds__(kMixThreads) void k_block_mix_quads(MixPtrs ptrs, c
             }
         }
         for (; d < end; d += kSingleWords) {
-            const int step = mix_table(d, 3), out = mix_table(d, 4);
+            const int step = table_at(d, 3), out = table_at(d, 4);
             // a loop per output, its sum known at compile time
             auto run = [&](FpSum &sum) {
-                int e = mix_table(d, 2);
-                const double *x = xd + mix_table(d, 0) * kTile + lane;
-                for (int len = mix_table(d, 1); len > 0; len--) {
+                int e = table_at(d, 2);
+                const double *x = xd + table_at(d, 0) * kTile + lane;
+                for (int len = table_at(d, 1); len > 0; len--) {
                     if (left == 0) fold();
                     left--;
-                    sum.mac(mix_table(w, e), x[0]);
+                    sum.mac(table_at(w, e), x[0]);
                     e += step;
                     x += kTile;
                 }

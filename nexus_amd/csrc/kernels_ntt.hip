@@ -13,21 +13,19 @@
 // limb is viewed as an N1 x N2 matrix (index = t * N2 + c).  The first log2(N1)
 // forward stages only pair elements of the same column c (gap >= N2), the last
 // log2(N2) stages only pair elements of the same row t; the inverse runs rows
-// first, then columns.  Each pass stages a tile of 16 columns (or 8 contiguous
-// rows) through LDS and runs radix-8/4/2 register butterflies between
-// barriers, 256 threads (four wave64) per workgroup.  Row twiddles for row r at
+// first, then columns.  Each pass stages a tile of 8 columns or 8 contiguous
+// rows (4 or 16 where the autotuner says so) through LDS and runs radix-8/4/2
+// register butterflies between barriers, 256 threads (four wave64) per workgroup.  Row twiddles for row r at
 // local stage s are the contiguous block fwd[2^s (N1 + r) ...].
 //
-// Arithmetic.  Limbs of primes q < 2^51 run in double precision, where the
-// FMA is full rate: with |a| <= q (1 + eps) and 0 <= w < q,
-//     h = a w (rounded), e = fma(a, w, -h) = a w - h exactly,
-//     Q = rint(h / q) (|Q - a w / q| <= 1.25), r = fma(-Q, q, h) + e = a w - Q q
-// is exact (every intermediate is an integer below 2^53) with |r| <= 1.25 q;
-// reduce(z) = fma(-rint(z / q), q, z) brings |z| < 2^52 to |z| <= q/2 (1 + eps).
-// Butterfly outputs are reduced, loads are reduced, and stores are mapped to
-// [0, q), so the output words equal the integer path's.  Larger primes use
-// 64-bit Shoup butterflies (ten 32-bit multiplies each) on [0, 4q).  This
-// file is compiled without floating-point contraction.
+// Arithmetic.  Limbs of primes q < 2^51 run in double precision, where the FMA
+// is full rate: exact products (fp_mulmod, six instructions) with centred
+// twiddles |w| <= q/2.  Loads are reduced to |v| <= q/2 (1 + eps); the sums of a
+// step of up to three stages are reduced at its end, or not at all in a pass
+// where they stay small enough (reduce_step, lazy_forward, lazy_inverse); stores
+// are mapped to [0, q), so the output words equal the integer path's.  Larger
+// primes use 64-bit Shoup butterflies (ten 32-bit multiplies each) on [0, 4q).
+// This file is compiled without floating-point contraction.
 #include <algorithm>
 #include <atomic>
 #include <cstdlib>
@@ -109,7 +107,7 @@ __device__ __forceinline__ void epi_store_f(const NttEpilogue &e, uint32_t p, ui
     const uint64_t off = (uint64_t)i * n + gidx;
     const uint32_t ct = p / e.polys_per, k = p - ct * e.polys_per;
     const uint64_t xv = e.xs[0] ? e.xs[ct][((uint64_t)k * e.x_limbs + i) * n + gidx] : e.x[p * e.x_stride + off];
-    double r = mulmod_f(fp_from(xv) - t, fp_from(e.inv[i].x), q, qinv);
+    double r = fp_mulmod(fp_from(xv) - t, fp_from(e.inv[i].x), q, qinv);
     uint64_t *o;
     if (e.out) {
         o = e.out + p * e.out_stride + off;
@@ -118,10 +116,10 @@ __device__ __forceinline__ void epi_store_f(const NttEpilogue &e, uint32_t p, ui
     } else {
         const uint64_t *a0 = e.a0s[0] ? e.a0s[ct] : e.a0;
         if (a0 && k == 0) r += fp_from(a0[(uint64_t)i * n + e.perm[ct][gidx]]);
-        if (e.d) r += mulmod_f(fp_from(e.d[p * e.d_stride + off]), fp_from(e.inv2[i].x), q, qinv);
+        if (e.d) r += fp_mulmod(fp_from(e.d[p * e.d_stride + off]), fp_from(e.inv2[i].x), q, qinv);
         o = e.outs[ct] + ((uint64_t)k * l + i) * n + gidx;
     }
-    r = reduce_f(r, q, qinv);
+    r = fp_reduce(r, q, qinv);
     *o = fp_to(r < 0 ? r + q : r);
 }
 
@@ -172,7 +170,7 @@ __device__ __forceinline__ void ntt_tile_f(const NttKArgs &a, uint64_t *lds_word
             double v[8];
 #pragma unroll
             for (int t = 0; t < 8; t++)
-                v[t] = reduce_f(fp_from(src[(uint64_t)(first + cc) * G::S + o + 32 * t]), q, qinv);
+                v[t] = fp_reduce(fp_from(src[(uint64_t)(first + cc) * G::S + o + 32 * t]), q, qinv);
             if (lazy)
                 fwd_group_f<3, true>(v, 0, 0, N1 + first + cc, tw, q, qinv);
             else
@@ -203,9 +201,9 @@ __device__ __forceinline__ void ntt_tile_f(const NttKArgs &a, uint64_t *lds_word
                 gidx = e;
             }
             if constexpr (LOAD == kPlain)
-                lds[e] = reduce_f(fp_from(src[gidx]), q, qinv);
+                lds[e] = fp_reduce(fp_from(src[gidx]), q, qinv);
             else
-                lds[e] = reduce_f(fp_from(load_word<LOAD>(src[gidx], a, a.mod[prime])), q, qinv);
+                lds[e] = fp_reduce(fp_from(load_word<LOAD>(src[gidx], a, a.mod[prime])), q, qinv);
         }
         __syncthreads();
         if (lazy)
@@ -227,9 +225,9 @@ __device__ __forceinline__ void ntt_tile_f(const NttKArgs &a, uint64_t *lds_word
         }
         double v = lds[e];
         if (scale_out)
-            v = reduce_f(mulmod_f(v, ni, q, qinv), q, qinv);
+            v = fp_reduce(fp_mulmod(v, ni, q, qinv), q, qinv);
         else if (lazy)
-            v = reduce_f(v, q, qinv);
+            v = fp_reduce(v, q, qinv);
         v = v < 0 ? v + q : v;
         if (epi) {
             if (a.epi_int)
@@ -271,7 +269,7 @@ __device__ __forceinline__ void ntt_pass(const NttKArgs &a)
     uint32_t tile = blockIdx.x;
     if (ROLE == kCol && (gridDim.x & 7) == 0) tile = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
     const uint32_t first = tile * G::C;  // first column / row of the tile
-    if (q < kFpPrimeBound) {
+    if (q < kFpPrime) {
         ntt_tile_f<LOGS, ROLE, FWD, CW, R16, NT, LOAD>(a, lds, data, src, prime, n, N2, N1, first, poly, limb);
         return;
     }
@@ -365,6 +363,26 @@ __global__ __launch_bounds__(NT) void k_ntt(NttKArgs a)
     ntt_pass<LOGS, ROLE, FWD, CW, R16, NT, LOAD>(a);
 }
 
+// The inverse's column pass of a tile, on the 8 words of a thread in the order the
+// conversions hold them; fully reduced to [0, q).  lds: 2048 doubles that no
+// other thread still reads.
+template <int LOGS>
+__device__ __forceinline__ void col_inverse(double *x, double *lds, const double *tw, double ninv, double q,
+                                            double qinv, uint32_t n, uint32_t col0)
+{
+    using C = ColTile<LOGS>;
+    const int tid = threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < 8; k++) lds[C::row_in(tid, k) * C::CW + tid % C::CW] = fp_reduce(x[k], q, qinv);
+    __syncthreads();
+    stages_f<LOGS, kCol, false, C::CW, false, kThreads, false>(lds, tw, q, qinv, n, 1u << LOGS, col0);
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const double v = fp_reduce(fp_mulmod(lds[C::row_in(tid, k) * C::CW + tid % C::CW], ninv, q, qinv), q, qinv);
+        x[k] = v < 0 ? v + q : v;
+    }
+}
+
 // ---- ModUp base conversion fused into the forward column pass
 //
 // Workgroup (tile, b, digit j, chunk): the digit's A input limbs are read once
@@ -377,26 +395,6 @@ __global__ __launch_bounds__(NT) void k_ntt(NttKArgs a)
 // products are the exact double-precision ones of the unfused conversion
 // (k_modup_conv_a), and the column stages those of the double-precision pass,
 // so the stored words equal the unfused conversion followed by the column pass.
-// The inverse's column pass of a tile, on the 8 words of a thread in the order the
-// conversions hold them; fully reduced to [0, q).  lds: 2048 doubles that no
-// other thread still reads.
-template <int LOGS>
-__device__ __forceinline__ void col_inverse(double *x, double *lds, const double *tw, double ninv, double q,
-                                            double qinv, uint32_t n, uint32_t col0)
-{
-    using C = ColTile<LOGS>;
-    const int tid = threadIdx.x;
-#pragma unroll
-    for (int k = 0; k < 8; k++) lds[C::row_in(tid, k) * C::CW + tid % C::CW] = reduce_f(x[k], q, qinv);
-    __syncthreads();
-    stages_f<LOGS, kCol, false, C::CW, false, kThreads, false>(lds, tw, q, qinv, n, 1u << LOGS, col0);
-#pragma unroll
-    for (int k = 0; k < 8; k++) {
-        const double v = reduce_f(mulmod_f(lds[C::row_in(tid, k) * C::CW + tid % C::CW], ninv, q, qinv), q, qinv);
-        x[k] = v < 0 ? v + q : v;
-    }
-}
-
 struct ModUpColArgs {
     const double *invd, *ninvd;  // the inverse's tables (INV)
     uint64_t *T;
@@ -444,7 +442,7 @@ __device__ __forceinline__ void modup_tile(const ModUpColArgs &a, double *lds, u
             col_inverse<LOGS>(y[i], lds + (i & 1) * C::LDS, a.invd + (uint64_t)p * n, a.ninvd[p], q, qinv, n, col0);
 #pragma unroll
         for (int k = 0; k < 8; k++) {
-            double v = reduce_f(mulmod_f(y[i][k], wi, q, qinv), q, qinv);
+            double v = fp_reduce(fp_mulmod(y[i][k], wi, q, qinv), q, qinv);
             v = v < 0 ? v + q : v;
             y[i][k] = on ? v : 0.0;
         }
@@ -455,7 +453,7 @@ __device__ __forceinline__ void modup_tile(const ModUpColArgs &a, double *lds, u
     double f[S], q, qinv;
     auto load_factors = [&](uint32_t kp) {
 #pragma unroll
-        for (int i = 0; i < S; i++) f[i] = table(factors, (uint64_t)i * a.key_limbs + kp);
+        for (int i = 0; i < S; i++) f[i] = table_at(factors, (uint64_t)i * a.key_limbs + kp);
         table_prime(a.qd, kp, q, qinv);
     };
     load_factors(prime(r0));
@@ -498,16 +496,6 @@ __global__ __launch_bounds__(kThreads, A <= 9 ? 2 : 1) void k_modup_col(ModUpCol
         modup_tile<LOGS, A, A, RAW, INV>(a, lds, b, j, s, r0, r1);
 }
 
-// ---- ModDown base conversion fused into the forward column pass
-//
-// Workgroup (tile, poly p, chunk): the A input limbs at limbs lo .. lo + A - 1
-// of poly p of acc (coefficient form) are read once over the tile; per
-// position v_k = [y_k w_k]_(p_k) (Shoup products, as k_moddown_conv_a) and the
-// centring quotient r = floor(sum_k v_k / p_k + 1/2) stay in registers; each
-// output prime q_i (i < lo) of the chunk gets sum_k v_k f_(k,i) - r (P mod q_i)
-// in exact double-precision products, transformed by the column stages of q_i
-// and stored into z[p][i].  The words equal the unfused conversion followed
-// by the column pass.  Every prime below 2^51.
 // ---- Rescale centring fused into the forward column pass
 //
 // Workgroup (tile, poly p, chunk): the INTT'd last limb of poly p (prime p_l,
@@ -515,7 +503,8 @@ __global__ __launch_bounds__(kThreads, A <= 9 ? 2 : 1) void k_modup_col(ModUpCol
 // gets (x + (p_l - 1)/2) mod p_l - (p_l - 1)/2 (SEAL's centred remainder,
 // an integer of magnitude below 2^51, exact in double precision) reduced mod
 // q_i, transformed by the column stages of q_i, stored into z[p][i].  The
-// words equal k_center_last followed by the column pass.  Every prime below 2^51.
+// words equal a transform's with that load (NttBatch::center).  Every prime below
+// 2^51.
 struct CenterColArgs {
     uint64_t *z;
     const uint64_t *last;
@@ -558,13 +547,23 @@ __global__ __launch_bounds__(kThreads) void k_center_col(CenterColArgs a)
         tw.load_uniform(a.twd + (uint64_t)i * n);
         double cv[8];
 #pragma unroll
-        for (int k = 0; k < 8; k++) cv[k] = reduce_f(v[k], q, qinv);
+        for (int k = 0; k < 8; k++) cv[k] = fp_reduce(v[k], q, qinv);
         next.load_lane(a.twd + (uint64_t)min(i + 1, i1 - 1) * n);
         col_forward<LOGS, false>(cv, lds + buf * C::LDS, tw, q, qinv, (int)a.logn, N2, col0,
                                  a.z + ((uint64_t)p * a.limbs + i) * n);
     }
 }
 
+// ---- ModDown base conversion fused into the forward column pass
+//
+// Workgroup (tile, poly p, chunk): the A input limbs at limbs lo .. lo + A - 1
+// of poly p of acc (coefficient form) are read once over the tile; per
+// position v_k = [y_k w_k]_(p_k) (as k_moddown_conv_a) and the
+// centring quotient r = floor(sum_k v_k / p_k + 1/2) stay in registers; each
+// output prime q_i (i < lo) of the chunk gets sum_k v_k f_(k,i) - r (P mod q_i)
+// in exact double-precision products, transformed by the column stages of q_i
+// and stored into z[p][i].  The words equal the unfused conversion followed
+// by the column pass.  Every prime below 2^51.
 struct ModDownColArgs {
     const double *invd, *ninvd;  // the inverse's tables (INV)
     uint64_t *z;
@@ -573,7 +572,6 @@ struct ModDownColArgs {
     const ulonglong2 *w;
     const double *convd;
     const double2 *qd;
-    const ModConst *mod;
     const double *twd;
     uint32_t lo, L, logn, chunk, chunks;
     uint32_t inp[kMaxPrimes];
@@ -610,7 +608,7 @@ __global__ __launch_bounds__(kThreads, A <= 9 ? 2 : 1) void k_moddown_col(ModDow
                               pinv, n, col0);
 #pragma unroll
         for (int k = 0; k < 8; k++) {
-            double x = reduce_f(mulmod_f(v[i][k], wi, pi, pinv), pi, pinv);
+            double x = fp_reduce(fp_mulmod(v[i][k], wi, pi, pinv), pi, pinv);
             x = x < 0 ? x + pi : x;
             // x / p_i correctly rounded: pinv is the correctly rounded 1 / p_i, so
             // one residual step on x pinv gives the quotient a division gives
@@ -625,7 +623,7 @@ __global__ __launch_bounds__(kThreads, A <= 9 ? 2 : 1) void k_moddown_col(ModDow
     double f[A + 1], q, qinv;
     auto load_factors = [&](uint32_t i) {
 #pragma unroll
-        for (int k = 0; k <= A; k++) f[k] = table(a.convd, (uint64_t)k * a.L + i);
+        for (int k = 0; k <= A; k++) f[k] = table_at(a.convd, (uint64_t)k * a.L + i);
         table_prime(a.qd, i, q, qinv);
     };
     load_factors(i0);
@@ -640,7 +638,7 @@ __global__ __launch_bounds__(kThreads, A <= 9 ? 2 : 1) void k_moddown_col(ModDow
         conv_tile<A>(cv, &v[0][0], f, qc, qic, pmax * qc <= 0x1p97);
         // - r (P mod q_i) as r times the centred q_i - P mod q_i
 #pragma unroll
-        for (int k = 0; k < 8; k++) cv[k] = reduce_f(cv[k] + mulmod_f(rr[k], f[A], qc, qic), qc, qic);
+        for (int k = 0; k < 8; k++) cv[k] = fp_reduce(cv[k] + fp_mulmod(rr[k], f[A], qc, qic), qc, qic);
         __builtin_amdgcn_sched_barrier(0);
         load_factors(min(i + 1, i1 - 1));
         __builtin_amdgcn_sched_barrier(0);
@@ -784,7 +782,7 @@ NttKArgs make_args(const DeviceTables &t, const NttBatch &b, bool fwd)
         const uint32_t m = b.prime_by_poly ? (b.poly_period ? b.poly_period : b.polys) : b.limbs;
         const uint32_t cnt = m < (uint32_t)kMaxPrimes ? m : (uint32_t)kMaxPrimes;
         uint32_t fp = 0;
-        for (uint32_t i = 0; i < cnt; i++) fp += t.mod_host[b.prime_of[i]] < kFpPrimeBound ? 1u : 0u;
+        for (uint32_t i = 0; i < cnt; i++) fp += t.mod_host[b.prime_of[i]] < kFpPrime ? 1u : 0u;
         a.tw_bytes = cnt ? (8.0 * fp + 16.0 * (cnt - fp)) / cnt : 16.0;
     }
     if (b.src_list) {
@@ -1103,7 +1101,6 @@ void ks_moddown_convert_col(const DeviceTables &t, uint64_t *z, const uint64_t *
     a.w = w;
     a.convd = convd;
     a.qd = t.qd;
-    a.mod = t.mod;
     a.twd = t.fwd_d;
     a.lo = lo;
     a.L = L;

@@ -142,24 +142,9 @@ __device__ __forceinline__ void inv_step(uint64_t *lds, int s, const ulonglong2 
     }
 }
 
-constexpr uint64_t kFpPrimeBound = kFpPrime;
-
-__device__ __forceinline__ double mulmod_f(double a, double w, double q, double qinv)
-{
-    const double h = a * w;
-    const double e = __builtin_fma(a, w, -h);
-    const double Q = __builtin_rint(h * qinv);
-    return __builtin_fma(-Q, q, h) + e;
-}
-
-__device__ __forceinline__ double reduce_f(double z, double q, double qinv)
-{
-    return __builtin_fma(-__builtin_rint(z * qinv), q, z);
-}
-
 // Sums of the double-precision butterflies.  Twiddles are centred, |w| <= q/2,
 // so the quotient of a product is off by at most 3 2^-53 |a| / 2 + 1/2 and
-// |mulmod_f(a, w)| <= q/2 + 1.5 2^-53 q |a|; it is exact while |a| < 2^53.
+// |fp_mulmod(a, w)| <= q/2 + 1.5 2^-53 q |a|; it is exact while |a| < 2^53.
 // Forward (v +- mulmod_f): from q/2 the bound grows to 1.19 q, 2.13 q and 3.43 q
 // < 2^53 over three stages for any q < 2^51, so a step of up to three stages
 // reduces once, at its end.  LAZY: q small enough for the whole pass
@@ -169,7 +154,7 @@ __device__ __forceinline__ void reduce_step(double *v, double q, double qinv)
 {
     if (!LAZY) {
 #pragma unroll
-        for (int t = 0; t < (1 << K); t++) v[t] = reduce_f(v[t], q, qinv);
+        for (int t = 0; t < (1 << K); t++) v[t] = fp_reduce(v[t], q, qinv);
     }
 }
 
@@ -190,7 +175,7 @@ __device__ __forceinline__ void fwd_group_f(double *v, int s, uint32_t blockid, 
             for (int u = 0; u < h; u++) {
                 const int t = j * 2 * h + u;
                 const double x = v[t];
-                const double y = mulmod_f(v[t + h], w, q, qinv);
+                const double y = fp_mulmod(v[t + h], w, q, qinv);
                 v[t] = x + y;
                 v[t + h] = x - y;
             }
@@ -282,7 +267,7 @@ __device__ __forceinline__ void inv_step_f(double *lds, int s, const double *tw,
                     const int t = j * (2 << d) + u;
                     const double x = v[t], y = v[t + (1 << d)];
                     v[t] = x + y;
-                    v[t + (1 << d)] = mulmod_f(x - y, w, q, qinv);
+                    v[t + (1 << d)] = fp_mulmod(x - y, w, q, qinv);
                 }
             }
             if (K > 3 && d == 1) reduce_step<K, LAZY>(v, q, qinv);
@@ -400,12 +385,12 @@ __device__ __forceinline__ double conv_sum(const double *y, int ystride, const d
 #pragma unroll
             for (int k = k0 + 4; k < k0 + 8 && k < A; k++) u.mac(y[k * ystride], f[k]);
             const double H = (s.h - 0x1.8p104) + (u.h - 0x1.8p104);
-            r = __builtin_fma(-__builtin_rint(H * qinv), q, H) + (reduce_f(s.l, q, qinv) + reduce_f(u.l, q, qinv));
+            r = __builtin_fma(-__builtin_rint(H * qinv), q, H) + (fp_reduce(s.l, q, qinv) + fp_reduce(u.l, q, qinv));
         }
         acc = k0 ? acc + r : r;
-        if (k0 + 8 < A) acc = reduce_f(acc, q, qinv);
+        if (k0 + 8 < A) acc = fp_reduce(acc, q, qinv);
     }
-    return reduce_f(acc, q, qinv);
+    return fp_reduce(acc, q, qinv);
 }
 
 // the 8 words of a thread, y[A][8]; four words at a time, so that the partial sums of only those are live at once
@@ -436,7 +421,7 @@ enum ColOut { kWords = 0, kReduced = 1, kUnreduced = 2 };
 template <bool LAZY, int OUT>
 __device__ __forceinline__ uint64_t col_out(double x, double q, double qinv)
 {
-    if (LAZY && OUT != kUnreduced) x = reduce_f(x, q, qinv);
+    if (LAZY && OUT != kUnreduced) x = fp_reduce(x, q, qinv);
     if (OUT != kWords) return (uint64_t)__double_as_longlong(x);
     return fp_to(x < 0 ? x + q : x);
 }
@@ -485,32 +470,21 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// p[i] of a table that no kernel writes, at an index that is the same for the
-// whole wave: a scalar load.  Through an ordinary pointer the compiler has to
-// assume that the kernel's own stores may reach the table, and takes a vector
-// load, which waits for them.
-template <class T>
-__device__ __forceinline__ T table(const T *p, uint64_t i)
-{
-    typedef const __attribute__((address_space(4))) T *Constant;
-    return ((Constant)(uintptr_t)p)[i];
-}
-
 __device__ __forceinline__ void table_prime(const double2 *qd, uint32_t i, double &q, double &qinv)
 {
     const double *p = reinterpret_cast<const double *>(qd);
-    q = table(p, 2 * i);
-    qinv = table(p, 2 * i + 1);
+    q = table_at(p, 2 * i);
+    qinv = table_at(p, 2 * i + 1);
 }
 
 __device__ __forceinline__ ModConst table_mod(const ModConst *mod, uint32_t i)
 {
     const uint64_t *p = reinterpret_cast<const uint64_t *>(mod + i);
     ModConst m;
-    m.q = table(p, 0);
-    m.ratio0 = table(p, 1);
-    m.ratio1 = table(p, 2);
-    m.two_q = table(p, 3);
+    m.q = table_at(p, 0);
+    m.ratio0 = table_at(p, 1);
+    m.ratio1 = table_at(p, 2);
+    m.two_q = table_at(p, 3);
     return m;
 }
 
@@ -527,7 +501,7 @@ __device__ __forceinline__ void group_f(double *v, const double *w, double q, do
 #pragma unroll
             for (int u = 0; u < h; u++) {
                 const int t = j * 2 * h + u;
-                const double x = v[t], y = mulmod_f(v[t + h], w[(1 << d) - 1 + j], q, qinv);
+                const double x = v[t], y = fp_mulmod(v[t + h], w[(1 << d) - 1 + j], q, qinv);
                 v[t] = x + y;
                 v[t + h] = x - y;
             }
@@ -542,7 +516,7 @@ __device__ __forceinline__ void uniform_group_tw(double *w, const double *tw, in
 #pragma unroll
     for (int d = 0; d < K; d++)
 #pragma unroll
-        for (int j = 0; j < (1 << d); j++) w[(1 << d) - 1 + j] = table(tw, ((uint32_t)1 << (s + d)) + (block << d) + j);
+        for (int j = 0; j < (1 << d); j++) w[(1 << d) - 1 + j] = table_at(tw, ((uint32_t)1 << (s + d)) + (block << d) + j);
 }
 
 template <int K>
