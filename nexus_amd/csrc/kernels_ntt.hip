@@ -906,14 +906,27 @@ void ntt_forward(const DeviceTables &t, const NttBatch &b, hipStream_t s)
 }
 
 // Algorithmic double-precision operations (an FMA counts two, rint one) of the
-// fused column kernels: an exact product (mul, fma, mul, rint, fma, add) is 8,
-// a reduction (mul, rint, fma) 4; a conversion to one output word over A
-// inputs is A products, A additions, a reduction every second term and a
-// final one; a column pass is half a butterfly (a product, an addition and a
-// subtraction) per word and stage plus the store's reduction.
+// fused column kernels: an exact product (mul, fma, mul, rint, fma, add) is 8, a
+// reduction (mul, rint, fma) 4.  A conversion to one output word is a term of
+// FpSum an input (two fma, a subtraction, an addition: 6), a quotient every eight
+// (conv_sum's narrow form: subtraction, mul, rint, fma, addition: 6), a sum and a
+// reduction between them and a reduction at the end.  A column pass is half a
+// butterfly (a product, an addition and a subtraction) per word and stage; stores
+// as words reduce once more, and the inverse's takes a reduction on load and the
+// reduced product with n^-1.
 constexpr double kFlopsProduct = 8.0, kFlopsReduce = 4.0;
-inline double conv_flops(uint32_t A) { return A * (kFlopsProduct + 1.0) + (A / 2) * kFlopsReduce + kFlopsReduce; }
-inline double col_flops(int logs) { return logs * (kFlopsProduct + 2.0) / 2.0 + kFlopsReduce; }
+inline double conv_flops(uint32_t A)
+{
+    const uint32_t sums = (A + 7) / 8;
+    return 6.0 * A + 6.0 * sums + (sums - 1) * (1.0 + kFlopsReduce) + kFlopsReduce;
+}
+inline double col_flops(int logs) { return logs * (kFlopsProduct + 2.0) / 2.0; }
+// one input word: its reduced product with a constant, and the inverse's column pass
+inline double input_flops(int logs, bool inverse)
+{
+    return kFlopsProduct + kFlopsReduce +
+           (inverse ? col_flops(logs) + kFlopsReduce + kFlopsProduct + kFlopsReduce : 0.0);
+}
 
 // Fused ModUp column pass of a stored ModUp, per power-of-two bucket of the batch
 // size B: 0 = on (outputs per workgroup by the default rule), -1 = off (conversion
@@ -1004,8 +1017,10 @@ void ks_modup_convert_col(const DeviceTables &t, uint64_t *T, const uint64_t *co
     uint32_t outs = 0;
     for (uint32_t j = 0; j < a.digits; j++) outs += nout - std::min(alpha, l - j * alpha);
     ProfScope prof("ks_modup_col", s,
-                   8.0 * n * ((double)B * l + (double)B * outs) + 8.0 * (double)(1u << l1) * B * outs,
-                   (double)n * B * ((double)l * kFlopsProduct + outs * (conv_flops(alpha) + col_flops(l1))));
+                   8.0 * n * ((double)B * l + (double)B * outs) +
+                       8.0 * (double)(1u << l1) * B * (outs + (inverse ? l : 0u)),
+                   (double)n * B * (l * input_flops(l1, inverse) +
+                                    outs * (conv_flops(alpha) + col_flops(l1) + (raw ? 0.0 : kFlopsReduce))));
     const dim3 grid(tiles, B * a.digits * a.chunks);
 #define NX_MC(LOGS, A)                                                                      \
     if (l1 == LOGS && alpha == A) {                                                       \
@@ -1051,7 +1066,7 @@ void rns_center_last_col(const DeviceTables &t, uint64_t *z, const uint64_t *las
     a.chunk = chunk;
     a.chunks = (limbs + chunk - 1) / chunk;
     ProfScope prof("rescale_col", s, 8.0 * n * polys * (1.0 + limbs) + 8.0 * (double)(1u << l1) * polys * limbs,
-                   (double)n * polys * limbs * (kFlopsReduce + col_flops(l1)));
+                   (double)n * polys * limbs * (2.0 * kFlopsReduce + col_flops(l1)));
     const dim3 grid(tiles, polys * a.chunks);
     if (l1 == 7)
         hipLaunchKernelGGL((k_center_col<7>), grid, dim3(kThreads), 0, s, a);
@@ -1116,8 +1131,13 @@ void ks_moddown_convert_col(const DeviceTables &t, uint64_t *z, const uint64_t *
     a.chunk = chunk;
     a.chunks = (lo + chunk - 1) / chunk;
     ProfScope prof("ks_moddown_col", s,
-                   8.0 * n * polys * ((double)A + lo) + 8.0 * (double)(1u << l1) * polys * lo,
-                   (double)n * polys * ((double)A * 2.0 + lo * (conv_flops(A + 1) + col_flops(l1))));
+                   8.0 * n * polys * ((double)A + lo) +
+                       8.0 * (double)(1u << l1) * polys * (lo + (inverse ? A : 0u)),
+                   // an input's share of the quotient: x / p_k (mul, two fma) and an addition; an output's
+                   // product with it, an addition and a reduction
+                   (double)n * polys * (A * (input_flops(l1, inverse) + 6.0) +
+                                        lo * (conv_flops(A) + kFlopsProduct + 1.0 + kFlopsReduce + col_flops(l1) +
+                                              kFlopsReduce)));
     const dim3 grid(tiles, polys * a.chunks);
 #define NX_MD(LOGS, AA)                                                                     \
     if (l1 == LOGS && A == AA) {                                                          \
