@@ -7,8 +7,10 @@
  * bytes.  Kernel classes include "ntt_fwd_col", "ntt_fwd_row",
  * "ntt_fwd_sub_mul" (a forward row pass that stores a ModDown or rescale
  * tail), "ntt_fwd_whole", "ntt_inv_row", "ntt_inv_col", "ntt_inv_whole",
- * "ks_inner", "ks_modup_conv", "ks_moddown_conv", "dot_plain", "lincomb",
- * "tensor", "mul_plain", "copy"; nx_profile_classes lists those seen.
+ * "ks_modup_col", "ks_lift_col", "ks_moddown_col" (conversions in a column
+ * pass), "ks_row_inner", "ks_row_inner_rot", "ks_inner_rot", "ks_inner",
+ * "dot_plain", "block_mix", "block_mix_quads", "lincomb", "tensor",
+ * "mul_plain", "copy"; nx_profile_classes lists those seen.
  */
 #ifndef NEXUS_PROF_H
 #define NEXUS_PROF_H

@@ -673,8 +673,10 @@ void ks_row_inner(const DeviceTables &t, const KsRowInner &p, hipStream_t s)
     const uint32_t n = 1u << t.logn;
     const int l2 = t.logn - t.logn / 2;
     ProfScope prof(rot ? "ks_row_inner_rot" : "ks_row_inner", s,
+                   // digits, the words of each key once, permutations, results
                    (double)n * p.nout *
-                       ((8.0 + (seeded ? 8.0 : 16.0)) * p.count * p.digits + 16.0 * a.B + (rot ? 4.0 * p.count : 0.0)));
+                       (8.0 * p.count * p.digits + (seeded ? 8.0 : 16.0) * (rot ? p.count : 1u) * p.digits +
+                        (rot ? 4.0 * p.count : 0.0) + 16.0 * (a.B + a.accumulate)));
     const dim3 grid(row_inner_tiles(t.logn), p.nout * a.B);
 #define NX_RI(L)                                                                             \
     if (l2 == L) {                                                                         \

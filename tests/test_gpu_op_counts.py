@@ -1,5 +1,6 @@
 """The double-precision operations that the profiler records for the fused
-conversions, against a count of what one output and one input word take.
+conversions, against a count of what one output and one input word take, and the
+bytes it records for the inner products, whose inputs share one key.
 
 The autotuner's choices are process-wide and may replace these launches, so the
 checks run in a process of their own (this file as a program)."""
@@ -43,10 +44,11 @@ def main():
         a = nx.encrypt(ctx, sk, nx.encode(ctx, [0.5], 2.0 ** 30), seed=3)
         t = nx.multiply(a, a)
         ctx.synchronize()
-        nx.profile_select("ks_modup_col,ks_moddown_col")
+        nx.profile_select("ks_modup_col,ks_moddown_col,ks_row_inner")
         nx.relinearize(t, rk)
         ctx.synchronize()
         up, down = (nx.profile_read_flops(c) for c in ("ks_modup_col", "ks_moddown_col"))
+        rows = nx.profile_read("ks_row_inner")
         nx.profile_select("")
         column = 7 * (PRODUCT + 2) / 2  # 2^7 rows: half a butterfly a word and stage
         # a partial digit is counted with a full one's terms
@@ -54,6 +56,16 @@ def main():
         assert up == ctx.n * (l * (PRODUCT + REDUCE) + outs * (_conversion(alpha) + column)), (alpha, up)
         out = _conversion(alpha) + PRODUCT + 1 + REDUCE + column + REDUCE
         assert down == 2 * ctx.n * (alpha * (PRODUCT + REDUCE + 6) + l * out), (alpha, down)
+        # one input: its key's uniform half comes from seeds
+        digits = -(-l // alpha)
+        word = 8 * ctx.n * (l + alpha)
+        assert rows[0] == 1 and rows[2] == word * (digits + digits + 2), (alpha, rows)
+        nx.profile_select("ks_row_inner")
+        nx.multiply_relin_rescale_many([a] * 3, [a] * 3, rk)
+        ctx.synchronize()
+        rows = nx.profile_read("ks_row_inner")
+        nx.profile_select("")
+        assert rows[0] == 1 and rows[2] == word * (3 * digits + 2 * digits + 3 * 2), (alpha, rows)
         del ctx, sk, rk, a, t
     print("ok", flush=True)
 
