@@ -1,7 +1,9 @@
 """Batches large enough that the conversions of a hybrid key switch run the
 inverse transform's column pass themselves, against the same operations one at a
 time (where they do not): the products' ModUp and ModDown, and a hoisted
-ModDown, with full and partial last digits and both column lengths."""
+ModDown, with full and partial last digits and both column lengths.  (Where the
+passes ran is read from the launches in test_gpu_inverse_fold.py: choices that
+the autotuner made in this process may have moved them here.)"""
 import sys
 
 import numpy as np
