@@ -108,8 +108,12 @@ struct Acc3 {
 // terms (k0 + j, entry0 + j dentry) for j < len, so the inner loop computes its
 // LDS addresses instead of loading them.  FAST: every prime below 2^58
 // (products folded every 16 terms through Acc3); otherwise 128-bit sums folded
-// every 32 terms.  WIDE: limbs below 2^51 are k_block_mix_quads'.
-template <bool FAST, bool WIDE>
+// every 32 terms.  LIMBS: with both bodies in one kernel long sums lose 3 to 5 %
+// (127 inputs to 127 outputs, scattered, ten limbs at N = 2^16: 16.5 ms, alone
+// 15.7), so chains of one arithmetic have instances of their own; kWide leaves
+// limbs below 2^51 to k_block_mix_quads.
+enum Limbs { kEvery = 0, kSmall = 1, kWide = 2 };  // any, all below 2^51, those above
+template <bool FAST, int LIMBS>
 __global__ __launch_bounds__(kBlock) void k_block_mix(MixPtrs ptrs, const uint64_t *__restrict__ table,
                                                       const int4 *__restrict__ runs,
                                                       const uint32_t *__restrict__ first, const ModConst *mod,
@@ -126,113 +130,113 @@ __global__ __launch_bounds__(kBlock) void k_block_mix(MixPtrs ptrs, const uint64
     uint64_t *ws = lds + K * kTile;   // [count][bpt]
     const uint64_t roff = (uint64_t)row * n + pos0;
     const ModConst m = mod[limb];
-    if (WIDE && m.q < kFpPrime) return;
+    if (LIMBS == kWide && m.q < kFpPrime) return;
     const uint32_t lane = threadIdx.x % kTile;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kTile);
     const uint32_t lb = log_stride >= 6 ? 0u : lane >> log_stride;
-    if (!WIDE && m.q < kFpPrime) {
-        // double precision: the tile and the weights as doubles, one exact
-        // product per term, the sum reduced every second term (|sum| < 3 q)
-        double *xd = reinterpret_cast<double *>(xs), *wd = reinterpret_cast<double *>(ws);
-        // wave w stages input rows w, w + 4, ...: the row (and its pointer) is
-        // uniform across the wave, eight loads in flight
+    if (LIMBS == kWide || (LIMBS == kEvery && m.q >= kFpPrime)) {
         {
-            const uint32_t w0 = wave;
-            uint32_t k = w0;
+            uint32_t k = wave;
             for (; k + 28 < K; k += 32) {
                 uint64_t v[8];
 #pragma unroll
                 for (int u = 0; u < 8; u++) v[u] = ptrs.in[k + 4 * u][roff + lane];
 #pragma unroll
-                for (int u = 0; u < 8; u++) xd[(k + 4 * u) * kTile + lane] = fp_from(v[u]);
+                for (int u = 0; u < 8; u++) xs[(k + 4 * u) * kTile + lane] = v[u];
             }
-            for (; k < K; k += 4) xd[k * kTile + lane] = fp_from(ptrs.in[k][roff + lane]);
+            for (; k < K; k += 4) xs[k * kTile + lane] = ptrs.in[k][roff + lane];
         }
         for (uint32_t e = threadIdx.x; e < count * bpt; e += kBlock) {
             const uint32_t p = e / bpt, b = e - p * bpt;
-            wd[e] = __longlong_as_double((long long)table[((uint64_t)limb * blocks + b0 + b) * count + p]);
+            ws[e] = table[((uint64_t)limb * blocks + b0 + b) * count + p];
         }
         __syncthreads();
-        const double q = (double)m.q, qinv = 1.0 / q;
         for (uint32_t o = wave; o < M; o += kBlock / kTile) {
-            // two independent sums (each reduced after every second term of its
-            // own) so consecutive products do not wait on one another
-            double a0 = 0.0, a1 = 0.0;
+            uint64_t r = 0;
+            Acc3 acc;
+            uint64_t lo = 0, hi = 0;
+            uint32_t cnt = 0;
             for (uint32_t ri = first[o]; ri < first[o + 1]; ri++) {
-                // a run: k = k0 + j, entry = p0 + j dp for j < len (indices computed, not loaded)
                 const int4 rn = runs[ri];
-                const double *xp = xd + rn.x * kTile + lane;
-                const int xstep = kTile, wstep = rn.w * (int)bpt;
-                const double *wp = wd + rn.y * (int)bpt + lb;
-                int j = 0;
-                for (; j + 4 <= rn.z; j += 4) {
-                    a0 += fp_mulmod(xp[0], wp[0], q, qinv);
-                    a1 += fp_mulmod(xp[xstep], wp[wstep], q, qinv);
-                    a0 += fp_mulmod(xp[2 * xstep], wp[2 * wstep], q, qinv);
-                    a1 += fp_mulmod(xp[3 * xstep], wp[3 * wstep], q, qinv);
-                    a0 = fp_reduce(a0, q, qinv);
-                    a1 = fp_reduce(a1, q, qinv);
-                    xp += 4 * xstep;
-                    wp += 4 * wstep;
-                }
-                for (; j < rn.z; j++) {
-                    a0 = fp_reduce(a0 + fp_mulmod(xp[0], wp[0], q, qinv), q, qinv);
-                    xp += xstep;
-                    wp += wstep;
+                for (int j = 0; j < rn.z; j++) {
+                    const uint64_t x = xs[(rn.x + j) * kTile + lane], w = ws[(rn.y + j * rn.w) * (int)bpt + lb];
+                    if (FAST) {
+                        acc.mac(x, w);
+                        if (++cnt == 16) {
+                            r = add_mod(r, acc.reduce(m), m.q);
+                            acc = Acc3();
+                            cnt = 0;
+                        }
+                    } else {
+                        const uint64_t plo = x * w, phi = mulhi64(x, w);
+                        lo += plo;
+                        hi += phi + (lo < plo);
+                        if (++cnt == 32) {
+                            r = add_mod(r, barrett128(hi, lo, m), m.q);
+                            lo = hi = 0;
+                            cnt = 0;
+                        }
+                    }
                 }
             }
-            double acc = fp_reduce(a0 + a1, q, qinv);
-            acc = acc < 0 ? acc + q : acc;
-            ptrs.out[o][roff + lane] = fp_to(acc);
+            r = FAST ? add_mod(r, acc.reduce(m), m.q) : add_mod(r, barrett128(hi, lo, m), m.q);
+            ptrs.out[o][roff + lane] = r;
         }
         return;
     }
+    // double precision: the tile and the weights as doubles, one exact
+    // product per term, the sum reduced every second term (|sum| < 3 q)
+    double *xd = reinterpret_cast<double *>(xs), *wd = reinterpret_cast<double *>(ws);
+    // wave w stages input rows w, w + 4, ...: the row (and its pointer) is
+    // uniform across the wave, eight loads in flight
     {
-        uint32_t k = wave;
+        const uint32_t w0 = wave;
+        uint32_t k = w0;
         for (; k + 28 < K; k += 32) {
             uint64_t v[8];
 #pragma unroll
             for (int u = 0; u < 8; u++) v[u] = ptrs.in[k + 4 * u][roff + lane];
 #pragma unroll
-            for (int u = 0; u < 8; u++) xs[(k + 4 * u) * kTile + lane] = v[u];
+            for (int u = 0; u < 8; u++) xd[(k + 4 * u) * kTile + lane] = fp_from(v[u]);
         }
-        for (; k < K; k += 4) xs[k * kTile + lane] = ptrs.in[k][roff + lane];
+        for (; k < K; k += 4) xd[k * kTile + lane] = fp_from(ptrs.in[k][roff + lane]);
     }
     for (uint32_t e = threadIdx.x; e < count * bpt; e += kBlock) {
         const uint32_t p = e / bpt, b = e - p * bpt;
-        ws[e] = table[((uint64_t)limb * blocks + b0 + b) * count + p];
+        wd[e] = __longlong_as_double((long long)table[((uint64_t)limb * blocks + b0 + b) * count + p]);
     }
     __syncthreads();
+    const double q = (double)m.q, qinv = 1.0 / q;
     for (uint32_t o = wave; o < M; o += kBlock / kTile) {
-        uint64_t r = 0;
-        Acc3 acc;
-        uint64_t lo = 0, hi = 0;
-        uint32_t cnt = 0;
+        // two independent sums (each reduced after every second term of its
+        // own) so consecutive products do not wait on one another
+        double a0 = 0.0, a1 = 0.0;
         for (uint32_t ri = first[o]; ri < first[o + 1]; ri++) {
+            // a run: k = k0 + j, entry = p0 + j dp for j < len (indices computed, not loaded)
             const int4 rn = runs[ri];
-            for (int j = 0; j < rn.z; j++) {
-                const uint64_t x = xs[(rn.x + j) * kTile + lane], w = ws[(rn.y + j * rn.w) * (int)bpt + lb];
-                if (FAST) {
-                    acc.mac(x, w);
-                    if (++cnt == 16) {
-                        r = add_mod(r, acc.reduce(m), m.q);
-                        acc = Acc3();
-                        cnt = 0;
-                    }
-                } else {
-                    const uint64_t plo = x * w, phi = mulhi64(x, w);
-                    lo += plo;
-                    hi += phi + (lo < plo);
-                    if (++cnt == 32) {
-                        r = add_mod(r, barrett128(hi, lo, m), m.q);
-                        lo = hi = 0;
-                        cnt = 0;
-                    }
-                }
+            const double *xp = xd + rn.x * kTile + lane;
+            const int xstep = kTile, wstep = rn.w * (int)bpt;
+            const double *wp = wd + rn.y * (int)bpt + lb;
+            int j = 0;
+            for (; j + 4 <= rn.z; j += 4) {
+                a0 += fp_mulmod(xp[0], wp[0], q, qinv);
+                a1 += fp_mulmod(xp[xstep], wp[wstep], q, qinv);
+                a0 += fp_mulmod(xp[2 * xstep], wp[2 * wstep], q, qinv);
+                a1 += fp_mulmod(xp[3 * xstep], wp[3 * wstep], q, qinv);
+                a0 = fp_reduce(a0, q, qinv);
+                a1 = fp_reduce(a1, q, qinv);
+                xp += 4 * xstep;
+                wp += 4 * wstep;
+            }
+            for (; j < rn.z; j++) {
+                a0 = fp_reduce(a0 + fp_mulmod(xp[0], wp[0], q, qinv), q, qinv);
+                xp += xstep;
+                wp += wstep;
             }
         }
-        r = FAST ? add_mod(r, acc.reduce(m), m.q) : add_mod(r, barrett128(hi, lo, m), m.q);
-        ptrs.out[o][roff + lane] = r;
+        double acc = fp_reduce(a0 + a1, q, qinv);
+        acc = acc < 0 ? acc + q : acc;
+        ptrs.out[o][roff + lane] = fp_to(acc);
     }
 }
 
@@ -511,8 +515,9 @@ void block_mix(const DeviceTables &t, const MixPtrs &p, const uint64_t *table, c
     if (quads && fp == limbs) return;
     ProfScope prof("block_mix", s, limb_bytes * (quads ? limbs - fp : limbs));
     const bool fast = t.max_bits <= 58, skip = quads || !fp;
-    auto *kernel = fast ? (skip ? k_block_mix<true, true> : k_block_mix<true, false>)
-                        : (skip ? k_block_mix<false, true> : k_block_mix<false, false>);
+    auto *kernel = fp == limbs ? k_block_mix<true, kSmall>
+                   : fast      ? (skip ? k_block_mix<true, kWide> : k_block_mix<true, kEvery>)
+                               : (skip ? k_block_mix<false, kWide> : k_block_mix<false, kEvery>);
     hipLaunchKernelGGL(kernel, grid, dim3(kBlock), lds, s, p, table, reinterpret_cast<const int4 *>(terms), first,
                        t.mod, K, M, limbs, count, blocks, log_stride, n);
 }
