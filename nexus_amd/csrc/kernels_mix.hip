@@ -108,10 +108,11 @@ struct Acc3 {
 // terms (k0 + j, entry0 + j dentry) for j < len, so the inner loop computes its
 // LDS addresses instead of loading them.  FAST: every prime below 2^58
 // (products folded every 16 terms through Acc3); otherwise 128-bit sums folded
-// every 32 terms.  LIMBS: with both bodies in one kernel long sums lose 3 to 5 %
-// (127 inputs to 127 outputs, scattered, ten limbs at N = 2^16: 16.5 ms, alone
-// 15.7), so chains of one arithmetic have instances of their own; kWide leaves
-// limbs below 2^51 to k_block_mix_quads.
+// every 32 terms.  LIMBS: with both bodies in one kernel long sums below 2^51
+// lose 2 % (double precision last, as here) to 5 % (first: 127 inputs to 127
+// outputs, scattered, ten limbs at N = 2^16 16.5 ms, alone 15.7), so chains of one
+// arithmetic have instances of their own; kWide leaves limbs below 2^51 to
+// k_block_mix_quads.
 enum Limbs { kEvery = 0, kSmall = 1, kWide = 2 };  // any, all below 2^51, those above
 template <bool FAST, int LIMBS>
 __global__ __launch_bounds__(kBlock) void k_block_mix(MixPtrs ptrs, const uint64_t *__restrict__ table,
